@@ -9,6 +9,14 @@
 namespace spirit_hip
 {
 
+// The mixed-radix plans of the three lengths (host memory; the plans' tables are device memory)
+// and their radices, from which the launches take their tile shapes.
+struct DdiMixHost
+{
+    MixPlan plan[3]; // a, b, c
+    int radix[3][MAX_MIX_STAGES];
+};
+
 struct DdiDev
 {
     int Na, Nb, Nc, nb; // lattice cells and basis atoms
@@ -32,6 +40,7 @@ struct DdiDev
     int c_kind;  // pass C kernel (DdiPassC), chosen by timing when the plan is built
     int c_tk;    // column tile of DDI_C_P2_LDS
     int rev;     // DDI_REV_* bits: passes that visit their blocks in reverse order
+    const DdiMixHost * mix; // host memory (read by the launchers only)
 };
 
 // Passes whose blocks run in reverse order, so that they first read what the pass before
@@ -46,7 +55,7 @@ enum DdiReverse
 
 enum DdiPassC
 {
-    DDI_C_GENERIC = 0, // mixed-radix LDS kernel (any length)
+    DDI_C_MIX     = 0, // mixed-radix tile kernel (any length)
     DDI_C_P2_LDS  = 1, // power of two, all 3*nb lines of c_tk columns held in LDS
     DDI_C_P2_REG  = 2, // power of two, one basis atom, real spectrum: components held in registers
     DDI_C_P4_REG  = 3, // as DDI_C_P2_REG with radix-4 transforms: 4 values per lane, more lanes per CU
@@ -73,6 +82,17 @@ int fft_lines_per_block( const FftLen & L );
 
 // Pass C kernels that can run this plan, as (c_kind, c_tk) pairs (at least one).
 std::vector<std::pair<int, int>> ddi_pass_c_candidates( const DdiDev & d );
+
+// The mixed-radix passes (ddi_mix_kernels.hip): whether a tile of the plan fits a block's LDS, and
+// their launches.  The convolution runs along c (pass C), or along b in place of the passes B, C
+// and B^-1 for lattices of one plane.
+bool mix_a_ok( const DdiDev & d );
+bool mix_b_ok( const DdiDev & d );
+bool mix_conv_ok( const DdiDev & d, bool along_b );
+void mix_launch_a_fwd( const DdiDev & d, const double * s, int nos, hipStream_t st );
+void mix_launch_a_inv( const DdiDev & d, double * h, int nos, hipStream_t st );
+void mix_launch_b( const DdiDev & d, bool inverse, hipStream_t st );
+void mix_launch_conv( const DdiDev & d, bool along_b, hipStream_t st );
 
 // nullptr if every pass of the plan fits the device's LDS, else the reason it does not.
 const char * ddi_plan_problem( const DdiDev & d );

@@ -11,10 +11,10 @@
 //   A^-1 Hermitian rows along a, keep a<Na, h = mu_i * res / M
 // X holds only the c < Nc planes (padded c planes never leave LDS); rows have the
 // stride Hs (Ha rounded up to 8 values = 128 bytes).  Power-of-two lengths run the
-// register-resident radix-8 kernels (fft_pow2.hpp); other lengths the generic
-// mixed-radix LDS kernels (fft_lds.hpp).  Pass A packs two real rows into one
-// complex transform.
-#include "ddi.hpp"
+// register-resident radix-8 kernels (fft_pow2.hpp); other lengths the mixed-radix
+// tile kernels (ddi_mix_kernels.hip).  Pass A packs two real rows into one complex
+// transform.
+#include "ddi_device.hpp"
 #include "fft_pow2.hpp"
 
 #include <algorithm>
@@ -27,100 +27,14 @@ namespace spirit_hip
 constexpr int FFT_THREADS = 256;
 constexpr int LDS_CPLX    = 4096; // 64 KiB of FP64 complex for the generic kernels
 
-// ---------------------------------------------------------------------------
-// kernel spectrum access and the symmetric 3x3 multiply (FFT.hpp:89-96 row order)
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ void dhat_load( const DdiDev & d, int kb, int ka, int kc, int b_inter, double2 * D )
-{
-    int kbs = kb, kcs = kc;
-    bool mb = false, mc = false;
-    if( d.sym_b && kb > d.Pb / 2 )
-    {
-        kbs = d.Pb - kb;
-        mb  = true;
-    }
-    if( d.sym_c && kc > d.Pc / 2 )
-    {
-        kcs = d.Pc - kc;
-        mc  = true;
-    }
-    const long long off = ( ( (long long)kbs * d.Ha + ka ) * d.KC + kcs ) * ( 6 * d.n_inter ) + 6 * b_inter;
-#pragma unroll
-    for( int q = 0; q < 6; ++q )
-    {
-        double2 v = d.dh_real ? make_double2( d.Dh_r[off + q], 0.0 ) : d.Dh[off + q];
-        int sg    = ( mb ? d.sig_b[q] : 1 ) * ( mc ? d.sig_c[q] : 1 );
-        if( sg < 0 )
-        {
-            v.x = -v.x;
-            v.y = -v.y;
-        }
-        D[q] = v;
-    }
-}
-
-// res_q = sum_p D_qp s_p, D symmetric (xx,xy,xz,yy,yz,zz)
-__device__ __forceinline__ void sym3_mul( const double2 * D, const double2 * s, double2 * r )
-{
-    const int rows[3][3] = { { 0, 1, 2 }, { 1, 3, 4 }, { 2, 4, 5 } };
-#pragma unroll
-    for( int q = 0; q < 3; ++q )
-    {
-        const double2 d1 = D[rows[q][0]], d2 = D[rows[q][1]], d3 = D[rows[q][2]];
-        r[q].x = d1.x * s[0].x + d2.x * s[1].x + d3.x * s[2].x - d1.y * s[0].y - d2.y * s[1].y - d3.y * s[2].y;
-        r[q].y = d1.x * s[0].y + d2.x * s[1].y + d3.x * s[2].y + d1.y * s[0].x + d2.y * s[1].x + d3.y * s[2].x;
-    }
-}
-
-// Hhat(b1) = sum_b2 Dhat(inter(b1,b2)) . Shat(b2) at one (kb, ka, kc); values in LDS at
-// lds[line(arr) * ls + pos], arr = 3*basis + component.
-template<typename IDX>
-__device__ __forceinline__ void conv_point( const DdiDev & d, int kb, int ka, int kc, double2 * lds, IDX idx )
-{
-    if( d.nb == 1 )
-    {
-        double2 D[6], s[3], r[3];
-        dhat_load( d, kb, ka, kc, 0, D );
-#pragma unroll
-        for( int q = 0; q < 3; ++q )
-            s[q] = lds[idx( q )];
-        sym3_mul( D, s, r );
-#pragma unroll
-        for( int q = 0; q < 3; ++q )
-            lds[idx( q )] = r[q];
-        return;
-    }
-    double2 S[MAX_BASIS][3];
-    for( int b2 = 0; b2 < d.nb; ++b2 )
-        for( int q = 0; q < 3; ++q )
-            S[b2][q] = lds[idx( 3 * b2 + q )];
-    for( int b1 = 0; b1 < d.nb; ++b1 )
-    {
-        double2 acc[3];
-        for( int b2 = 0; b2 < d.nb; ++b2 )
-        {
-            double2 D[6], r[3];
-            dhat_load( d, kb, ka, kc, d.inter[b1 + b2 * d.nb], D );
-            sym3_mul( D, S[b2], r );
-#pragma unroll
-            for( int q = 0; q < 3; ++q )
-                acc[q] = b2 == 0 ? r[q] : cadd( acc[q], r[q] );
-        }
-        for( int q = 0; q < 3; ++q )
-            lds[idx( 3 * b1 + q )] = acc[q];
-    }
-}
-
 // ===========================================================================
-// Generic mixed-radix kernels (any padded length with factors 2,3,5,7,11,13)
+// Kernel-spectrum set-up (any padded length with factors 2,3,5,7,11,13)
 // ===========================================================================
 
-// Pass A forward: real rows -> half spectra.  SRC 0: spins (times mu), SRC 1: plain real array.
-// line = b + Nb_in*(c + Nc_in*arr); output rows of stride hs, b extent b_ext, c extent c_ext.
-template<int SRC>
+// Pass A: real rows of n_arr arrays -> half spectra; output rows of stride hs.
 __global__ void __launch_bounds__( FFT_THREADS )
-    k_pass_a_fwd( DdiDev d, const double * __restrict__ src, int nos, int n_arr, int Na_in, int Nb_in, int Nc_in,
-                  int b_ext, int c_ext, int hs, double2 * __restrict__ out, int lines_per_block )
+    k_pass_a_fwd( DdiDev d, const double * __restrict__ src, int n_arr, int Na_in, int Nb_in, int Nc_in, int hs,
+                  double2 * __restrict__ out, int lines_per_block )
 {
     extern __shared__ double2 lds[];
     const int Pa            = d.La.n;
@@ -136,23 +50,7 @@ __global__ void __launch_bounds__( FFT_THREADS )
         int l          = e / Pa;
         int a          = e - l * Pa;
         long long line = line0 + l;
-        int b          = (int)( line % Nb_in );
-        long long rest = line / Nb_in;
-        int c          = (int)( rest % Nc_in );
-        int arr        = (int)( rest / Nc_in );
-        double v       = 0.0;
-        if( a < Na_in )
-        {
-            if( SRC == 0 )
-            {
-                int ib      = arr / 3;
-                int q       = arr - 3 * ib;
-                long long i = ib + (long long)d.nb * ( a + (long long)d.Na * ( b + (long long)d.Nb * c ) );
-                v           = src[(long long)q * nos + i] * d.mu[ib];
-            }
-            else
-                v = src[( ( (long long)arr * Nc_in + c ) * Nb_in + b ) * (long long)Na_in + a];
-        }
+        double v       = a < Na_in ? src[line * (long long)Na_in + a] : 0.0;
         lds[l * ls + a] = make_double2( v, 0.0 );
     }
     __syncthreads();
@@ -163,63 +61,13 @@ __global__ void __launch_bounds__( FFT_THREADS )
         int l          = e / Ha;
         int ka         = e - l * Ha;
         long long line = line0 + l;
-        int b          = (int)( line % Nb_in );
-        long long rest = line / Nb_in;
-        int c          = (int)( rest % Nc_in );
-        int arr        = (int)( rest / Nc_in );
-        out[( ( (long long)arr * c_ext + c ) * b_ext + b ) * hs + ka] = lds[l * ls + ka];
+        out[line * hs + ka] = lds[l * ls + ka];
     }
 }
 
-// Pass A inverse: half spectra -> real rows, h = mu * res / M (SoA, per spin)
+// Pass B: columns along b for (arr, c, ka-tile), in place; rows of stride hs.
 __global__ void __launch_bounds__( FFT_THREADS )
-    k_pass_a_inv( DdiDev d, const double2 * __restrict__ X, double * __restrict__ h, int nos, int lines_per_block )
-{
-    extern __shared__ double2 lds[];
-    const int Pa            = d.La.n;
-    const int Ha            = d.Ha;
-    const int ls            = Pa + 1;
-    const int n_arr         = 3 * d.nb;
-    const long long n_lines = (long long)n_arr * d.Nb * d.Nc;
-    const long long line0   = (long long)blockIdx.x * lines_per_block;
-    int nl                  = lines_per_block;
-    if( line0 + nl > n_lines )
-        nl = (int)( n_lines - line0 );
-
-    for( int e = threadIdx.x; e < nl * Pa; e += blockDim.x )
-    {
-        int l               = e / Pa;
-        int k               = e - l * Pa;
-        long long line      = line0 + l;
-        int b               = (int)( line % d.Nb );
-        long long rest      = line / d.Nb;
-        int c               = (int)( rest % d.Nc );
-        int arr             = (int)( rest / d.Nc );
-        const double2 * row = X + ( ( (long long)arr * d.Nc + c ) * d.Pb + b ) * d.Hs;
-        lds[l * ls + k]     = k < Ha ? row[k] : cconj( row[Pa - k] );
-    }
-    __syncthreads();
-    lds_fft<true>( lds, ls, nl, d.La );
-    for( int e = threadIdx.x; e < nl * d.Na; e += blockDim.x )
-    {
-        int l          = e / d.Na;
-        int a          = e - l * d.Na;
-        long long line = line0 + l;
-        int b          = (int)( line % d.Nb );
-        long long rest = line / d.Nb;
-        int c          = (int)( rest % d.Nc );
-        int arr        = (int)( rest / d.Nc );
-        int ib         = arr / 3;
-        int q          = arr - 3 * ib;
-        long long i    = ib + (long long)d.nb * ( a + (long long)d.Na * ( b + (long long)d.Nb * c ) );
-        h[(long long)q * nos + i] = d.mu[ib] * lds[l * ls + a].x / d.M;
-    }
-}
-
-// Pass B (forward or inverse): columns along b for (arr, c, ka-tile); rows of stride hs.
-template<bool INV>
-__global__ void __launch_bounds__( FFT_THREADS )
-    k_pass_b( DdiDev d, double2 * __restrict__ X, int n_arr, int c_ext, int b_in, int b_out, int hs, int tk )
+    k_pass_b( DdiDev d, double2 * __restrict__ X, int n_arr, int c_ext, int hs, int tk )
 {
     extern __shared__ double2 lds[];
     const int Pb      = d.Lb.n;
@@ -241,64 +89,15 @@ __global__ void __launch_bounds__( FFT_THREADS )
     {
         int l           = e % nk;
         int b           = e / nk;
-        lds[l * ls + b] = b < b_in ? slab[(long long)b * hs + ka0 + l] : make_double2( 0.0, 0.0 );
+        lds[l * ls + b] = slab[(long long)b * hs + ka0 + l];
     }
     __syncthreads();
-    lds_fft<INV>( lds, ls, nk, d.Lb );
-    for( int e = threadIdx.x; e < nk * b_out; e += blockDim.x )
+    lds_fft<false>( lds, ls, nk, d.Lb );
+    for( int e = threadIdx.x; e < nk * Pb; e += blockDim.x )
     {
         int l                             = e % nk;
         int b                             = e / nk;
         slab[(long long)b * hs + ka0 + l] = lds[l * ls + b];
-    }
-}
-
-// Pass C: columns along c for (kb, ka-tile), all 3*nb arrays: forward, multiply, inverse, keep c < Nc.
-__global__ void __launch_bounds__( FFT_THREADS ) k_pass_c_conv( DdiDev d, double2 * __restrict__ X, int tk )
-{
-    extern __shared__ double2 lds[];
-    const int Pc          = d.Lc.n;
-    const int Ha          = d.Ha;
-    const int Nc          = d.Nc;
-    const int ls          = Pc + 1;
-    const int n_arr       = 3 * d.nb;
-    const int n_tiles     = ( Ha + tk - 1 ) / tk;
-    const int tile        = (int)( blockIdx.x % n_tiles );
-    const int kb          = (int)( blockIdx.x / n_tiles );
-    const int ka0         = tile * tk;
-    int nk                = tk;
-    if( ka0 + nk > Ha )
-        nk = Ha - ka0;
-    const long long plane = (long long)d.Pb * d.Hs;
-
-    for( int e = threadIdx.x; e < n_arr * nk * Pc; e += blockDim.x )
-    {
-        int l     = e % nk;
-        int rest  = e / nk;
-        int c     = rest % Pc;
-        int arr   = rest / Pc;
-        double2 v = make_double2( 0.0, 0.0 );
-        if( c < Nc )
-            v = X[( (long long)arr * Nc + c ) * plane + (long long)kb * d.Hs + ka0 + l];
-        lds[( arr * nk + l ) * ls + c] = v;
-    }
-    __syncthreads();
-    lds_fft<false>( lds, ls, n_arr * nk, d.Lc );
-    for( int e = threadIdx.x; e < nk * Pc; e += blockDim.x )
-    {
-        int l  = e / Pc;
-        int kc = e - l * Pc;
-        conv_point( d, kb, ka0 + l, kc, lds, [&]( int arr ) { return ( arr * nk + l ) * ls + kc; } );
-    }
-    __syncthreads();
-    lds_fft<true>( lds, ls, n_arr * nk, d.Lc );
-    for( int e = threadIdx.x; e < n_arr * nk * Nc; e += blockDim.x )
-    {
-        int l    = e % nk;
-        int rest = e / nk;
-        int c    = rest % Nc;
-        int arr  = rest / Nc;
-        X[( (long long)arr * Nc + c ) * plane + (long long)kb * d.Hs + ka0 + l] = lds[( arr * nk + l ) * ls + c];
     }
 }
 
@@ -716,33 +515,6 @@ __global__ void __launch_bounds__( 512 ) k_p2_b( DdiDev d, double2 * __restrict_
             if( b < b_out )
                 col_ptr[(long long)b * d.Hs] = v[k];
         }
-    }
-}
-
-// Logical block lb of a pass C launch (n_tiles column tiles per kb plane, Pb planes) to its
-// (tile, kb).  With order_pairs: plane 0, then for 0 < p < Pb-p the tiles of the planes p and
-// Pb-p interleaved (tile j of p, tile j of Pb-p, ...), then plane Pb/2 if Pb is even, so the
-// second read of a stored spectrum tile (the two planes share it) follows the first by one
-// block and hits in L2.  A bijection on [0, n_tiles * Pb).
-__device__ __forceinline__ void pass_c_block( int lb, int n_tiles, int Pb, int order_pairs, int & tile, int & kb )
-{
-    tile = lb % n_tiles;
-    kb   = lb / n_tiles;
-    if( !order_pairs || lb < n_tiles )
-        return;
-    const int r     = lb - n_tiles;
-    const int pairs = ( Pb - 1 ) / 2; // planes p and Pb-p with 0 < p < Pb-p
-    if( r < 2 * n_tiles * pairs )
-    {
-        const int p = 1 + r / ( 2 * n_tiles );
-        const int w = r % ( 2 * n_tiles );
-        tile        = w >> 1;
-        kb          = ( w & 1 ) ? Pb - p : p;
-    }
-    else
-    {
-        tile = r - 2 * n_tiles * pairs;
-        kb   = Pb / 2;
     }
 }
 
@@ -1169,12 +941,6 @@ static int p2_c_tk( const DdiDev & d )
     return 0;
 }
 
-static int generic_c_tk( const DdiDev & d )
-{
-    int tk = fft_lines_per_block( d.Lc ) / ( 3 * d.nb );
-    return tk < 1 ? 1 : tk;
-}
-
 std::vector<std::pair<int, int>> ddi_pass_c_candidates( const DdiDev & d )
 {
     std::vector<std::pair<int, int>> c;
@@ -1190,18 +956,18 @@ std::vector<std::pair<int, int>> ddi_pass_c_candidates( const DdiDev & d )
             c.push_back( { DDI_C_P2_LDS, tk / 2 } );
     }
     if( c.empty() )
-        c.push_back( { DDI_C_GENERIC, 0 } );
+        c.push_back( { DDI_C_MIX, 0 } );
     return c;
 }
 
 const char * ddi_plan_problem( const DdiDev & d )
 {
     const size_t lim = (size_t)d.lds_max;
-    if( !p2_ab_ok( d, d.La ) && lds_bytes( fft_lines_per_block( d.La ), d.La.n ) > lim )
+    if( ( !p2_ab_ok( d, d.La ) && !mix_a_ok( d ) ) || lds_bytes( fft_lines_per_block( d.La ), d.La.n ) > lim )
         return "padded length along a exceeds the LDS of one block";
-    if( !p2_b_ok( d ) && lds_bytes( fft_lines_per_block( d.Lb ), d.Lb.n ) > lim )
+    if( ( !p2_b_ok( d ) && !mix_b_ok( d ) ) || lds_bytes( fft_lines_per_block( d.Lb ), d.Lb.n ) > lim )
         return "padded length along b exceeds the LDS of one block";
-    if( !p2_c1_ok( d ) && p2_c_tk( d ) == 0 && lds_bytes( 3 * d.nb * generic_c_tk( d ), d.Lc.n ) > lim )
+    if( !p2_c1_ok( d ) && p2_c_tk( d ) == 0 && !mix_conv_ok( d, false ) )
         return "padded length along c times 3*n_cell_atoms exceeds the LDS of one block";
     if( lds_bytes( 6 * std::max( 1, fft_lines_per_block( d.Lc ) / 6 ), d.Lc.n ) > lim )
         return "padded length along c exceeds the LDS of the kernel-spectrum set-up";
@@ -1287,7 +1053,6 @@ static void p2_launch_c( const DdiDev & d, int tk, hipStream_t st )
 void ddi_launch_field( const DdiDev & d, const double * spins, double * h, int nos, hipStream_t st, hipEvent_t evc0,
                        hipEvent_t evc1 )
 {
-    const int n_arr = 3 * d.nb;
     // pass A
     if( p2_ab_ok( d, d.La ) )
     {
@@ -1296,13 +1061,7 @@ void ddi_launch_field( const DdiDev & d, const double * spins, double * h, int n
 #undef CALL_A
     }
     else
-    {
-        const int lpb         = fft_lines_per_block( d.La );
-        const long long lines = (long long)n_arr * d.Nb * d.Nc;
-        const int blocks      = (int)( ( lines + lpb - 1 ) / lpb );
-        hipLaunchKernelGGL( k_pass_a_fwd<0>, dim3( blocks ), dim3( FFT_THREADS ), lds_bytes( lpb, d.La.n ), st, d,
-                            spins, nos, n_arr, d.Na, d.Nb, d.Nc, d.Pb, d.Nc, d.Hs, d.X, lpb );
-    }
+        mix_launch_a_fwd( d, spins, nos, st );
     // pass B
     if( p2_b_ok( d ) )
     {
@@ -1311,13 +1070,7 @@ void ddi_launch_field( const DdiDev & d, const double * spins, double * h, int n
 #undef CALL_B
     }
     else
-    {
-        const int tk     = fft_lines_per_block( d.Lb );
-        const int tiles  = ( d.Ha + tk - 1 ) / tk;
-        const int blocks = tiles * d.Nc * n_arr;
-        hipLaunchKernelGGL( k_pass_b<false>, dim3( blocks ), dim3( FFT_THREADS ), lds_bytes( tk, d.Lb.n ), st, d, d.X,
-                            n_arr, d.Nc, d.Nb, d.Pb, d.Hs, tk );
-    }
+        mix_launch_b( d, false, st );
     // pass C
     if( evc0 )
         (void)hipEventRecord( evc0, st );
@@ -1340,13 +1093,7 @@ void ddi_launch_field( const DdiDev & d, const double * spins, double * h, int n
 #undef CALL_C
     }
     else
-    {
-        const int tk     = generic_c_tk( d );
-        const int tiles  = ( d.Ha + tk - 1 ) / tk;
-        const int blocks = tiles * d.Pb;
-        hipLaunchKernelGGL( k_pass_c_conv, dim3( blocks ), dim3( FFT_THREADS ), lds_bytes( n_arr * tk, d.Lc.n ), st,
-                            d, d.X, tk );
-    }
+        mix_launch_conv( d, false, st );
     if( evc1 )
         (void)hipEventRecord( evc1, st );
     // pass B^-1
@@ -1357,13 +1104,7 @@ void ddi_launch_field( const DdiDev & d, const double * spins, double * h, int n
 #undef CALL_BI
     }
     else
-    {
-        const int tk     = fft_lines_per_block( d.Lb );
-        const int tiles  = ( d.Ha + tk - 1 ) / tk;
-        const int blocks = tiles * d.Nc * n_arr;
-        hipLaunchKernelGGL( k_pass_b<true>, dim3( blocks ), dim3( FFT_THREADS ), lds_bytes( tk, d.Lb.n ), st, d, d.X,
-                            n_arr, d.Nc, d.Pb, d.Nb, d.Hs, tk );
-    }
+        mix_launch_b( d, true, st );
     // pass A^-1
     if( p2_ab_ok( d, d.La ) )
     {
@@ -1372,13 +1113,7 @@ void ddi_launch_field( const DdiDev & d, const double * spins, double * h, int n
 #undef CALL_AI
     }
     else
-    {
-        const int lpb         = fft_lines_per_block( d.La );
-        const long long lines = (long long)n_arr * d.Nb * d.Nc;
-        const int blocks      = (int)( ( lines + lpb - 1 ) / lpb );
-        hipLaunchKernelGGL( k_pass_a_inv, dim3( blocks ), dim3( FFT_THREADS ), lds_bytes( lpb, d.La.n ), st, d, d.X,
-                            h, nos, lpb );
-    }
+        mix_launch_a_inv( d, h, nos, st );
 }
 
 void ddi_launch_kernel_spectrum( const DdiDev & d, const DipoleArgs & g, double * work, double2 * work2,
@@ -1392,15 +1127,15 @@ void ddi_launch_kernel_spectrum( const DdiDev & d, const DipoleArgs & g, double 
         const int lpb         = fft_lines_per_block( d.La );
         const long long lines = (long long)n_arr * Pb * Pc;
         const int blocks      = (int)( ( lines + lpb - 1 ) / lpb );
-        hipLaunchKernelGGL( k_pass_a_fwd<1>, dim3( blocks ), dim3( FFT_THREADS ), lds_bytes( lpb, Pa ), st, d, work,
-                            0, n_arr, Pa, Pb, Pc, Pb, Pc, d.Hs, work2, lpb );
+        hipLaunchKernelGGL( k_pass_a_fwd, dim3( blocks ), dim3( FFT_THREADS ), lds_bytes( lpb, Pa ), st, d, work,
+                            n_arr, Pa, Pb, Pc, d.Hs, work2, lpb );
     }
     {
         const int tk     = fft_lines_per_block( d.Lb );
         const int tiles  = ( d.Ha + tk - 1 ) / tk;
         const int blocks = tiles * Pc * n_arr;
-        hipLaunchKernelGGL( k_pass_b<false>, dim3( blocks ), dim3( FFT_THREADS ), lds_bytes( tk, Pb ), st, d, work2,
-                            n_arr, Pc, Pb, Pb, d.Hs, tk );
+        hipLaunchKernelGGL( k_pass_b, dim3( blocks ), dim3( FFT_THREADS ), lds_bytes( tk, Pb ), st, d, work2, n_arr,
+                            Pc, d.Hs, tk );
     }
     {
         int tk = fft_lines_per_block( d.Lc ) / 6;

@@ -1,0 +1,356 @@
+// The passes of the dipolar FFT convolution for lengths that are no power of two (and the
+// convolution pass wherever the power-of-two kernels do not apply), hand-written for gfx950 on
+// the mixed-radix tile transform of fft_mix.hpp.
+//
+// Every pass moves its part of the spectrum once (the padded half neither read nor written) and
+// is bound by that traffic: a block transforms a tile of lines held in LDS, its first stage reads
+// global memory straight into registers and its last one writes straight from them.  Two real
+// rows share one complex transform in passes A and A^-1.
+//
+// Measured on a 200x150x12 film (padded 400x300x24, 36 MB of spectrum, in the memory-side cache),
+// us a launch, against the one-row, one-stage-at-a-time LDS kernels these replaced: A 13 (47),
+// B 14 (40), C 31 (74), B^-1 14 (40), A^-1 13 (54); reading and writing their data once takes
+// 5, 10, 17, 10 and 5 at 5.4 TB/s.  What is left in A, B and their inverses is the chain load,
+// three stages with two barriers each, store, of too few waves to overlap; pass C issues vector
+// instructions half of its time.
+#include "ddi_device.hpp"
+#include "fft_mix.hpp"
+
+#include <algorithm>
+#include <cmath>
+
+namespace spirit_hip
+{
+
+// Pass A: row pairs (b0 = 2 bp, b0 + 1) of one component and plane, zero-padded.
+template<bool WIDE>
+__global__ void __launch_bounds__( 1024 )
+    k_mix_a_fwd( DdiDev d, MixPlan P, MixTile tile, const double * __restrict__ s, int nos )
+{
+    extern __shared__ double2 lds[];
+    const MixBlock T( tile, P, lds );
+    const int N         = P.n;
+    const int cw        = T.nl;
+    const int l         = T.lc; // this thread's line
+    const int npairs    = ( d.Nb + 1 ) / 2;
+    const int n_lines   = 3 * d.nb * npairs * d.Nc;
+    const int blk       = ( d.rev & DDI_REV_A_FWD ) ? gridDim.x - 1 - blockIdx.x : blockIdx.x;
+    const int line      = blk * cw + l;
+    const bool act      = line < n_lines;
+    const int rest      = line / npairs;
+    const int b0        = 2 * ( line - rest * npairs );
+    const int arr       = rest / d.Nc;
+    const int c         = rest - arr * d.Nc;
+    const bool has1     = act && b0 + 1 < d.Nb;
+    const int ib        = arr / 3;
+    const int q         = arr - 3 * ib;
+    const double mu     = act ? d.mu[ib] : 0.0;
+    const double * row0 = s + (long long)q * nos + ib + (long long)d.nb * d.Na * ( b0 + (long long)d.Nb * c );
+    const double * row1 = row0 + (long long)d.nb * d.Na;
+    mix_fft_to_lds<false, WIDE>( P, T, [&]( int, int a ) {
+        double2 v = make_double2( 0, 0 );
+        if( act && a < d.Na )
+        {
+            v.x = row0[(long long)d.nb * a] * mu;
+            if( has1 )
+                v.y = row1[(long long)d.nb * a] * mu;
+        }
+        return v;
+    } );
+    if( !act )
+        return;
+    // Z = X1 + i X2 of two real rows: X1 = (Z + conj Z[-k]) / 2, X2 = (Z - conj Z[-k]) / (2i)
+    double2 * out0 = d.X + ( ( (long long)arr * d.Nc + c ) * d.Pb + b0 ) * d.Hs;
+    double2 * out1 = out0 + d.Hs;
+    for( int k = T.j0; k < d.Ha; k += T.m )
+    {
+        const double2 z = T.at( k, l ), m = T.at( k == 0 ? 0 : N - k, l );
+        out0[k] = make_double2( 0.5 * ( z.x + m.x ), 0.5 * ( z.y - m.y ) );
+        if( has1 )
+            out1[k] = make_double2( 0.5 * ( z.y + m.y ), -0.5 * ( z.x - m.x ) );
+    }
+}
+
+// Pass A^-1: Z = X1 + i X2 from the stored halves of two Hermitian rows, h = mu res / M.
+template<bool WIDE>
+__global__ void __launch_bounds__( 1024 )
+    k_mix_a_inv( DdiDev d, MixPlan P, MixTile tile, double * __restrict__ h, int nos )
+{
+    extern __shared__ double2 lds[];
+    const MixBlock T( tile, P, lds );
+    const int N          = P.n;
+    const int cw         = T.nl;
+    const int l          = T.lc;
+    const int npairs     = ( d.Nb + 1 ) / 2;
+    const int n_lines    = 3 * d.nb * npairs * d.Nc;
+    const int blk        = ( d.rev & DDI_REV_A_INV ) ? gridDim.x - 1 - blockIdx.x : blockIdx.x;
+    const int line       = blk * cw + l;
+    const bool act       = line < n_lines;
+    const int rest       = line / npairs;
+    const int b0         = 2 * ( line - rest * npairs );
+    const int arr        = rest / d.Nc;
+    const int c          = rest - arr * d.Nc;
+    const bool has1      = act && b0 + 1 < d.Nb;
+    const int ib         = arr / 3;
+    const int q          = arr - 3 * ib;
+    const double mu      = act ? d.mu[ib] : 0.0;
+    const double2 * row0 = d.X + ( ( (long long)arr * d.Nc + c ) * d.Pb + b0 ) * d.Hs;
+    const double2 * row1 = row0 + d.Hs;
+    double * h0          = h + (long long)q * nos + ib + (long long)d.nb * d.Na * ( b0 + (long long)d.Nb * c );
+    double * h1          = h0 + (long long)d.nb * d.Na;
+    mix_fft<true, WIDE>(
+        P, T,
+        [&]( int, int k ) {
+            const bool half = k < d.Ha;
+            const int kk    = half ? k : N - k;
+            double2 x1 = make_double2( 0, 0 ), x2 = make_double2( 0, 0 );
+            if( act )
+                x1 = row0[kk];
+            if( has1 )
+                x2 = row1[kk];
+            if( !half )
+                x1.y = -x1.y, x2.y = -x2.y;
+            return make_double2( x1.x - x2.y, x1.y + x2.x );
+        },
+        [&]( int, int a, double2 v ) {
+            if( act && a < d.Na )
+            {
+                h0[(long long)d.nb * a] = mu * v.x / d.M;
+                if( has1 )
+                    h1[(long long)d.nb * a] = mu * v.y / d.M;
+            }
+        } );
+}
+
+// Pass B: columns along b of one (component, plane) slab, inputs b < b_in, outputs b < b_out.
+template<bool INV, bool WIDE>
+__global__ void __launch_bounds__( 1024 )
+    k_mix_b( DdiDev d, MixPlan P, MixTile tile, double2 * __restrict__ X, int n_tiles, int b_in, int b_out )
+{
+    extern __shared__ double2 lds[];
+    const MixBlock T( tile, P, lds );
+    const int cw   = T.nl;
+    const int l    = T.lc;
+    const int bid  = ( d.rev & ( INV ? DDI_REV_B_INV : DDI_REV_B_FWD ) ) ? gridDim.x - 1 - blockIdx.x : blockIdx.x;
+    const int slab = bid / n_tiles;
+    const int ka   = ( bid - slab * n_tiles ) * cw + l;
+    const bool col = ka < d.Ha;
+    double2 * p    = X + (long long)slab * P.n * d.Hs + ka;
+    mix_fft<INV, WIDE>(
+        P, T,
+        [&]( int, int b ) { return col && b < b_in ? p[(long long)b * d.Hs] : make_double2( 0, 0 ); },
+        [&]( int, int b, double2 v ) {
+            if( col && b < b_out )
+                p[(long long)b * d.Hs] = v;
+        } );
+}
+
+// The convolution along one axis: forward transform of all 3 nb arrays of cw columns (ka), the
+// product with the kernel spectrum, inverse transform, the first n_in points kept.
+// ALONG_B = false: pass C, the axis is c, one kb plane a block (planes kb and Pb-kb interleaved
+// with order_pairs).  ALONG_B = true: a lattice of one plane has nothing to transform along c, so
+// passes B, C and B^-1 are this one kernel along b.  ONE: one basis atom (the product over pairs of
+// basis atoms indexes a private array, which costs scratch memory).
+template<bool ALONG_B, bool WIDE, bool ONE>
+__global__ void __launch_bounds__( 1024 )
+    k_mix_conv( DdiDev d, MixPlan P, MixTile mt, double2 * __restrict__ X, int cw, MixDiv by_cw, MixDiv by_n,
+                int n_tiles, int order_pairs )
+{
+    extern __shared__ double2 lds[];
+    const MixBlock T( mt, P, lds );
+    // XCD-contiguous block order: neighbouring column tiles share cache lines of a row
+    const int nblk = gridDim.x;
+    const int full = ( nblk / 8 ) * 8;
+    int lb         = blockIdx.x;
+    if( lb < full )
+        lb = ( lb % 8 ) * ( full / 8 ) + lb / 8;
+    int tile = lb, kb = 0;
+    if( !ALONG_B )
+        pass_c_block( lb, n_tiles, d.Pb, order_pairs, tile, kb );
+    const int ka0         = tile * cw;
+    const int nk          = min( cw, d.Ha - ka0 );
+    const long long plane = (long long)d.Pb * d.Hs;
+    const int n_in        = ALONG_B ? d.Nb : d.Nc;
+    double2 * base        = ALONG_B ? X + ka0 : X + (long long)kb * d.Hs + ka0;
+    const long long es    = ALONG_B ? d.Hs : plane;                   // one point further along the axis
+    const long long as    = ALONG_B ? plane : plane * (long long)d.Nc; // one array further
+    mix_fft_to_lds<false, WIDE>( P, T, [&]( int l, int p ) {
+        const int arr = mix_div( l, by_cw ), col = l - arr * cw;
+        return col < nk && p < n_in ? base[arr * as + p * es + col] : make_double2( 0, 0 );
+    } );
+    // one spectrum point a thread: along c the points of a column are contiguous in the stored
+    // kernel spectrum, along b those of a row
+    for( int e = threadIdx.x; e < cw * P.n; e += blockDim.x )
+    {
+        const int hi = mix_div( e, ALONG_B ? by_cw : by_n );
+        const int lo = e - hi * ( ALONG_B ? cw : P.n );
+        const int col = ALONG_B ? lo : hi, p = ALONG_B ? hi : lo;
+        if( col < nk )
+            conv_point<ONE>( d, ALONG_B ? p : kb, ka0 + col, ALONG_B ? 0 : p, lds,
+                        [&]( int arr ) { return p * T.lsr + arr * cw + col; } );
+    }
+    __syncthreads();
+    mix_fft_from_lds<true, WIDE>( P, T, [&]( int l, int p, double2 v ) {
+        const int arr = mix_div( l, by_cw ), col = l - arr * cw;
+        if( col < nk && p < n_in )
+            base[arr * as + p * es + col] = v;
+    } );
+}
+
+// ---------------------------------------------------------------------------
+// host side
+// ---------------------------------------------------------------------------
+// LDS of a tile of nl lines (row stride lsr) and the twiddles behind it
+static size_t mix_lds( const MixPlan & P, int lsr )
+{
+    return sizeof( double2 ) * ( (size_t)P.n * (size_t)lsr + (size_t)P.n_tw );
+}
+
+// The tile of nl lines and the threads a line gets: at least what the in-place stages' registers
+// need (mix_per), and of the counts up to a quarter of the line the one with the fewest idle lanes
+// over the stages and wavefronts, weighed against the waves a CU then holds (sixteen at the
+// kernels' registers).  All lines at once, or the largest divisor of nl whose threads fit a block.
+static MixTile mix_tile( const DdiDev & d, int axis, int nl, int lsr )
+{
+    const MixPlan & P = d.mix->plan[axis];
+    const int * rad   = d.mix->radix[axis];
+    const int blocks  = std::max( 1, (int)( (size_t)d.lds_max / mix_lds( P, lsr ) ) );
+    int lo            = 1;
+    for( int s = 0; s < P.ns; ++s )
+        lo = std::max( lo, ( P.n / rad[s] + mix_per( rad[s] ) - 1 ) / mix_per( rad[s] ) );
+    MixTile best{ nl, lsr, 1, lo };
+    double best_score = -1;
+    for( int m = lo; m <= std::max( lo, ( P.n + 3 ) / 4 ); ++m )
+    {
+        int nc = nl;
+        while( nc > 1 && ( nc * m > 1024 || nl % nc != 0 ) )
+            --nc;
+        double rounds = 0;
+        for( int s = 0; s < P.ns; ++s )
+            rounds += ( P.n / rad[s] + m - 1 ) / m * rad[s];
+        const int waves    = ( nc * m + 63 ) / 64;
+        const double use   = (double)P.n * P.ns / ( rounds * m ) * ( nc * m ) / ( 64.0 * waves );
+        const double score = use * std::sqrt( std::min( 1.0, blocks * waves / 16.0 ) );
+        if( nc * m <= 1024 && score > best_score + 1e-9 )
+            best_score = score, best.nc = nc, best.m = m;
+    }
+    return best;
+}
+
+static bool mix_wide( const DdiDev & d, int axis )
+{
+    return d.mix->radix[axis][0] > 10; // the largest radix is the first
+}
+
+// Lines of a tile (a power of two).  A row piece of a column tile is 16 cw bytes, so tiles of the
+// column passes are 16 wide where two blocks then fit a CU's LDS, else 8, and narrower only where
+// LDS forces it or fewer than 192 blocks would leave CUs idle (not below 4, 64 bytes): 14 us a
+// pass against 18 and 22 at 16, 8, 4 columns of 300 points, 13 against 16 and 22 at 8, 4, 2 of
+// 1000.  Row pairs (pass A) are contiguous whatever cw is: 4, fewer where that fills the chip.
+static int mix_lines( const DdiDev & d, const MixPlan & P, int arrays, long long n_cols, int want, int least )
+{
+    auto lds = [&]( int cw ) { return mix_lds( P, arrays * cw ); };
+    int cw   = want;
+    while( cw > 1
+           && ( lds( cw ) > (size_t)d.lds_max / ( cw > 8 ? 2 : 1 )
+                || ( cw > least && ( n_cols + cw - 1 ) / cw < 192 ) ) )
+        cw /= 2;
+    return cw;
+}
+
+static int mix_a_lines( const DdiDev & d )
+{
+    return mix_lines( d, d.mix->plan[0], 1, 3LL * d.nb * ( ( d.Nb + 1 ) / 2 ) * d.Nc, 4, 1 );
+}
+
+static int mix_b_cols( const DdiDev & d )
+{
+    return mix_lines( d, d.mix->plan[1], 1, (long long)d.Ha * d.Nc * 3 * d.nb, 16, 4 );
+}
+
+bool mix_a_ok( const DdiDev & d )
+{
+    return mix_lds( d.mix->plan[0], mix_a_lines( d ) ) <= (size_t)d.lds_max;
+}
+
+bool mix_b_ok( const DdiDev & d )
+{
+    return mix_lds( d.mix->plan[1], mix_b_cols( d ) ) <= (size_t)d.lds_max;
+}
+
+// Columns and LDS row stride of the convolution pass.  Along b a block holds all arrays of its
+// columns and there are only Ha / cw blocks, so its tiles narrow down to one column.
+static int mix_conv_cols( const DdiDev & d, bool along_b, int & lsr )
+{
+    const MixPlan & P = d.mix->plan[along_b ? 1 : 2];
+    const int cw      = along_b ? mix_lines( d, P, 3 * d.nb, d.Ha, 16, 1 )
+                                : mix_lines( d, P, 3 * d.nb, (long long)d.Ha * d.Pb, 16, 4 );
+    // an odd row stride spreads the spectrum product's column accesses over the banks
+    lsr = ( 3 * d.nb * cw ) | 1;
+    if( mix_lds( P, lsr ) > (size_t)d.lds_max )
+        lsr = 3 * d.nb * cw;
+    return cw;
+}
+
+bool mix_conv_ok( const DdiDev & d, bool along_b )
+{
+    int lsr;
+    (void)mix_conv_cols( d, along_b, lsr );
+    return mix_lds( d.mix->plan[along_b ? 1 : 2], lsr ) <= (size_t)d.lds_max;
+}
+
+void mix_launch_a_fwd( const DdiDev & d, const double * s, int nos, hipStream_t st )
+{
+    const int cw          = mix_a_lines( d );
+    const MixTile T       = mix_tile( d, 0, cw, cw );
+    const long long lines = 3LL * d.nb * ( ( d.Nb + 1 ) / 2 ) * d.Nc;
+    const auto k          = mix_wide( d, 0 ) ? k_mix_a_fwd<true> : k_mix_a_fwd<false>;
+    hipLaunchKernelGGL( k, dim3( (unsigned)( ( lines + cw - 1 ) / cw ) ), dim3( T.nc * T.m ),
+                        mix_lds( d.mix->plan[0], cw ), st, d, d.mix->plan[0], T, s, nos );
+}
+
+void mix_launch_a_inv( const DdiDev & d, double * h, int nos, hipStream_t st )
+{
+    const int cw          = mix_a_lines( d );
+    const MixTile T       = mix_tile( d, 0, cw, cw );
+    const long long lines = 3LL * d.nb * ( ( d.Nb + 1 ) / 2 ) * d.Nc;
+    const auto k          = mix_wide( d, 0 ) ? k_mix_a_inv<true> : k_mix_a_inv<false>;
+    hipLaunchKernelGGL( k, dim3( (unsigned)( ( lines + cw - 1 ) / cw ) ), dim3( T.nc * T.m ),
+                        mix_lds( d.mix->plan[0], cw ), st, d, d.mix->plan[0], T, h, nos );
+}
+
+void mix_launch_b( const DdiDev & d, bool inverse, hipStream_t st )
+{
+    const int cw    = mix_b_cols( d );
+    const MixTile T = mix_tile( d, 1, cw, cw );
+    const int tiles = ( d.Ha + cw - 1 ) / cw;
+    const dim3 g( (unsigned)( (long long)tiles * d.Nc * 3 * d.nb ) ), b( T.nc * T.m );
+    const size_t lds = mix_lds( d.mix->plan[1], cw );
+    const bool w     = mix_wide( d, 1 );
+    const auto k     = inverse ? ( w ? k_mix_b<true, true> : k_mix_b<true, false> )
+                               : ( w ? k_mix_b<false, true> : k_mix_b<false, false> );
+    hipLaunchKernelGGL( k, g, b, lds, st, d, d.mix->plan[1], T, d.X, tiles, inverse ? d.Pb : d.Nb,
+                        inverse ? d.Nb : d.Pb );
+}
+
+void mix_launch_conv( const DdiDev & d, bool along_b, hipStream_t st )
+{
+    int lsr           = 0;
+    const int axis    = along_b ? 1 : 2;
+    const int cw      = mix_conv_cols( d, along_b, lsr );
+    const MixPlan & P = d.mix->plan[axis];
+    const int tiles   = ( d.Ha + cw - 1 ) / cw;
+    const MixTile T   = mix_tile( d, axis, 3 * d.nb * cw, lsr );
+    const MixDiv by_cw{ 1.0f / (float)cw }, by_n{ 1.0f / (float)P.n };
+    const bool w = mix_wide( d, axis ), one = d.nb == 1;
+    const auto k = along_b ? ( w     ? k_mix_conv<true, true, false>
+                               : one ? k_mix_conv<true, false, true>
+                                     : k_mix_conv<true, false, false> )
+                           : ( w     ? k_mix_conv<false, true, false>
+                               : one ? k_mix_conv<false, false, true>
+                                     : k_mix_conv<false, false, false> );
+    hipLaunchKernelGGL( k, dim3( (unsigned)( (long long)tiles * ( along_b ? 1 : d.Pb ) ) ), dim3( T.nc * T.m ),
+                        mix_lds( P, lsr ), st, d, P, T, d.X, cw, by_cw, by_n, tiles, !along_b && d.sym_b ? 1 : 0 );
+}
+
+} // namespace spirit_hip

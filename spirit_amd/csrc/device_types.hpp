@@ -139,6 +139,40 @@ struct ImageDev
     int n_blocks;       // blocks of this image
 };
 
+// Division by d for small numerators (mix_div): the rounded reciprocal.
+struct MixDiv
+{
+    float inv;
+};
+
+// Mixed-radix plan of one length (fft_mix.hpp): stages of radix R after Ns = product of the
+// earlier radices, nbf = n / R butterflies a line, stage twiddles w_n^(r jm n/(Ns R)) at
+// tw[tw + (r - 1) Ns + jm].
+struct MixStage
+{
+    int R, Ns, nbf, tw;
+    MixDiv by_ns;
+};
+struct MixPlan
+{
+    int n, ns, n_tw;
+    const MixStage * st; // ns stages, device memory
+    const double2 * tw;  // n_tw stage twiddles, device memory
+};
+constexpr int MAX_MIX_STAGES = 5; // enough for every length to 4096 with prime factors to 13
+
+// most butterflies of radix R a thread holds in an in-place stage
+constexpr int mix_per( int R )
+{
+    return R >= 8 ? 1 : ( 10 + R - 1 ) / R;
+}
+
+// A tile of lines (MixBlock): nl lines in groups of nc, LDS row stride lsr, m threads a line.
+struct MixTile
+{
+    int nl, lsr, nc, m;
+};
+
 // One FFT length: Stockham stage radices and the n-th roots of unity exp(-2 pi i e / n).
 // For powers of two >= 8, tw2 holds the twiddles of the register-resident radix-8
 // plan in stage order: stage s (>= 1, radix R, Ns = 8^s) at offset 8^s - 8,

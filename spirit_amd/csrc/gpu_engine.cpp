@@ -3,6 +3,7 @@
 
 #include <algorithm>
 #include <chrono>
+#include <functional>
 #include <map>
 #include <mutex>
 #include <cmath>
@@ -85,6 +86,7 @@ void FftLenHost::build( int n )
     HIPCHECK( hipMemcpy( W.as<void>(), w.data(), sizeof( double2 ) * n, hipMemcpyHostToDevice ) );
     dev.W   = W.as<double2>();
     dev.tw2 = nullptr;
+    build_mix( w );
 
     // Power-of-two plan: radix-8 stages then one radix-2/4 stage.  Stage s >= 1 has
     // Ns = 8^s and stores, at offset 8^s - 8, w_n^(r*jm*n/(Ns*R)) at jm*(R-1) + r-1.
@@ -113,6 +115,86 @@ void FftLenHost::build( int n )
         HIPCHECK( hipMemcpy( TW2.as<void>(), t.data(), sizeof( double2 ) * t.size(), hipMemcpyHostToDevice ) );
         dev.tw2 = TW2.as<double2>();
     }
+}
+
+// The radices of the mixed-radix plan of n (at most 10, or 13 with a factor 11 or 13): as few stages
+// as possible, then the smallest largest radix (registers), then the smallest sum; the largest
+// first, where half of a zero-padded line's inputs need no load.
+static std::vector<int> mix_radices( int n )
+{
+    std::vector<int> best, now;
+    auto better = [&]( const std::vector<int> & a ) {
+        if( best.empty() )
+            return true;
+        if( a.size() != best.size() )
+            return a.size() < best.size();
+        if( a[0] != best[0] )
+            return a[0] < best[0];
+        int sa = 0, sb = 0;
+        for( size_t k = 0; k < a.size(); ++k )
+            sa += a[k], sb += best[k];
+        return sa < sb;
+    };
+    // radices in descending order
+    std::function<void( int, int )> search = [&]( int m, int top ) {
+        if( m == 1 )
+        {
+            if( better( now ) )
+                best = now;
+            return;
+        }
+        if( now.size() == MAX_MIX_STAGES )
+            return;
+        for( int r = std::min( top, m ); r >= 2; --r )
+            if( m % r == 0 )
+            {
+                now.push_back( r );
+                search( m / r, r );
+                now.pop_back();
+            }
+    };
+    if( n == 1 )
+        return { 1 };
+    search( n, n % 11 == 0 || n % 13 == 0 ? 13 : 10 );
+    if( best.empty() )
+        throw std::runtime_error( "DDI FFT: no mixed-radix plan for length " + std::to_string( n ) );
+    return best;
+}
+
+void FftLenHost::build_mix( const std::vector<double2> & w )
+{
+    const int n                = dev.n;
+    const std::vector<int> rad = mix_radices( n );
+    std::vector<MixStage> st;
+    std::vector<double2> t;
+    int Ns = 1;
+    for( int R : rad )
+    {
+        MixStage S{};
+        S.R     = R;
+        S.Ns    = Ns;
+        S.nbf   = n / R;
+        S.tw    = (int)t.size();
+        S.by_ns = MixDiv{ 1.0f / (float)Ns };
+        if( Ns > 1 )
+            for( int r = 1; r < R; ++r )
+                for( int jm = 0; jm < Ns; ++jm )
+                    t.push_back( w[( (long long)r * jm * ( n / ( Ns * R ) ) ) % n] );
+        mix_radix[st.size()] = R;
+        st.push_back( S );
+        Ns *= R;
+    }
+    mix.n_tw = (int)t.size();
+    if( t.empty() )
+        t.push_back( make_double2( 1.0, 0.0 ) );
+    mix_st.resize( sizeof( MixStage ) * st.size() );
+    mix_tw.resize( sizeof( double2 ) * t.size() );
+    HIPCHECK( hipMemcpy( mix_st.as<void>(), st.data(), sizeof( MixStage ) * st.size(), hipMemcpyHostToDevice ) );
+    HIPCHECK( hipMemcpy( mix_tw.as<void>(), t.data(), sizeof( double2 ) * t.size(), hipMemcpyHostToDevice ) );
+    mix.n  = n;
+    mix.ns = (int)st.size();
+    mix.st = mix_st.as<MixStage>();
+    mix.tw = mix_tw.as<double2>();
 }
 
 std::array<int, 3> ddi_padded_dims( const Geometry & g, const Hamiltonian & h )
@@ -250,6 +332,13 @@ void DdiPlan::build( const Geometry & g, const Hamiltonian & h, hipStream_t st )
     d.La  = La.dev;
     d.Lb  = Lb.dev;
     d.Lc  = Lc.dev;
+    const FftLenHost * len[3] = { &La, &Lb, &Lc };
+    for( int k = 0; k < 3; ++k )
+    {
+        mix.plan[k] = len[k]->mix;
+        std::copy( len[k]->mix_radix, len[k]->mix_radix + MAX_MIX_STAGES, mix.radix[k] );
+    }
+    d.mix = &mix;
     // inter_sublattice_lookup, Hamiltonian_Heisenberg.cpp:1415-1428 and 1545-1554
     int b_inter = -1;
     for( int b1 = 0; b1 < g.nb; ++b1 )
@@ -273,7 +362,7 @@ void DdiPlan::build( const Geometry & g, const Hamiltonian & h, hipStream_t st )
     X.resize( sizeof( double2 ) * nX );
     d.X = X.as<double2>();
     // component signs of D under b -> -b and c -> -c for an orthogonal lattice
-    // (xx, xy, xz, yy, yz, zz); used only where the spectrum shows them.
+    // (xx, xy, xz, yy, yz, zz; conv_point states them too); used only where the spectrum shows them.
     const int sb[6] = { +1, -1, +1, +1, -1, +1 };
     const int sc[6] = { +1, +1, -1, +1, -1, +1 };
     for( int q = 0; q < 6; ++q )
@@ -357,7 +446,7 @@ void DdiPlan::choose_pass_c( hipStream_t st )
     if( const char * force = std::getenv( "SPIRIT_HIP_DDI_PASS_C" ) )
     {
         const std::string f( force );
-        const int want = f == "generic" ? DDI_C_GENERIC
+        const int want = f == "generic" ? DDI_C_MIX
                          : f == "lds"   ? DDI_C_P2_LDS
                          : f == "reg"   ? DDI_C_P2_REG
                          : f == "reg4"  ? DDI_C_P4_REG
@@ -366,8 +455,8 @@ void DdiPlan::choose_pass_c( hipStream_t st )
         for( auto & c : cand )
             if( c.first == want )
                 keep.push_back( c );
-        if( keep.empty() && want == DDI_C_GENERIC )
-            keep.push_back( { DDI_C_GENERIC, 0 } );
+        if( keep.empty() && want == DDI_C_MIX && mix_conv_ok( d, false ) )
+            keep.push_back( { DDI_C_MIX, 0 } );
         if( keep.empty() )
             log_message( 2, "SPIRIT_HIP_DDI_PASS_C=" + f + " cannot run this DDI plan; timing every candidate" );
         else

@@ -61,8 +61,13 @@ private:
 struct FftLenHost
 {
     FftLen dev{};
-    DeviceBuffer W, TW2;
+    MixPlan mix{};
+    int mix_radix[MAX_MIX_STAGES] = {};
+    DeviceBuffer W, TW2, mix_st, mix_tw;
     void build( int n );
+
+private:
+    void build_mix( const std::vector<double2> & w );
 };
 
 // One zero-padded FFT convolution plan (one image geometry).
@@ -107,6 +112,7 @@ private:
     DdiRsDev rs{};
     DeviceBuffer b_pos, b_pairs;
     DdiDev d{};
+    DdiMixHost mix{};
     DhatSymmetry sym{};
     double c_ms = 0;
     FftLenHost La, Lb, Lc;
