@@ -944,6 +944,13 @@ static int p2_c_tk( const DdiDev & d )
 std::vector<std::pair<int, int>> ddi_pass_c_candidates( const DdiDev & d )
 {
     std::vector<std::pair<int, int>> c;
+    // a lattice of one plane: two round trips of the spectrum less than B, C and B^-1 in turn
+    // (500x500x1, padded 1000x1000: 24 us against 15 + 28 + 17), wherever a tile fits
+    if( d.Pc == 1 && mix_conv_ok( d, true ) )
+    {
+        c.push_back( { DDI_C_MIX_B, 0 } );
+        return c;
+    }
     if( p2_c1_ok( d ) )
         c.push_back( { DDI_C_P2_REG, 0 } );
     if( p4_c1_ok( d ) )
@@ -1062,14 +1069,15 @@ void ddi_launch_field( const DdiDev & d, const double * spins, double * h, int n
     }
     else
         mix_launch_a_fwd( d, spins, nos, st );
+    const bool one_plane = d.c_kind == DDI_C_MIX_B;
     // pass B
-    if( p2_b_ok( d ) )
+    if( !one_plane && p2_b_ok( d ) )
     {
 #define CALL_B( n ) p2_launch_b<n, false>( d, st )
         P2_DISPATCH( d.Pb, CALL_B );
 #undef CALL_B
     }
-    else
+    else if( !one_plane )
         mix_launch_b( d, false, st );
     // pass C
     if( evc0 )
@@ -1093,17 +1101,17 @@ void ddi_launch_field( const DdiDev & d, const double * spins, double * h, int n
 #undef CALL_C
     }
     else
-        mix_launch_conv( d, false, st );
+        mix_launch_conv( d, one_plane, st );
     if( evc1 )
         (void)hipEventRecord( evc1, st );
     // pass B^-1
-    if( p2_b_ok( d ) )
+    if( !one_plane && p2_b_ok( d ) )
     {
 #define CALL_BI( n ) p2_launch_b<n, true>( d, st )
         P2_DISPATCH( d.Pb, CALL_BI );
 #undef CALL_BI
     }
-    else
+    else if( !one_plane )
         mix_launch_b( d, true, st );
     // pass A^-1
     if( p2_ab_ok( d, d.La ) )
