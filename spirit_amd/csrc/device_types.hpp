@@ -14,6 +14,7 @@ namespace spirit_hip
 constexpr int MAX_BASIS      = 8;
 constexpr int MAX_PAIRS      = 64;
 constexpr int MAX_FFT_STAGES = 16;
+constexpr int MAX_REACH      = 3; // cells away that the pair loops' offset table covers (SiteOffsets)
 constexpr int GATHER_PAIRS   = 6; // pair tables up to this size are gathered into registers per spin
 
 // Physical constants, core/include/utility/Constants.hpp:18-40
@@ -76,7 +77,7 @@ struct HamDev
     int has_ddi;
     int has_site_K;
     int dmi_same;            // DMI pair k has exchange pair k's (i, j, translation) for every k < n_dmi
-    int halo[3];             // largest |translation| of an exchange pair along a, b, c
+    int reach[3];            // largest |translation| of an exchange or DMI pair along a, b, c
     int row_tile_log2;       // stage kernels sweep tiles of 2^row_tile_log2 rows along b through the c planes
     FastDiv div_nb, div_Na, div_Nb; // index -> (basis atom, a, b, c) without hardware division
     double B;                // external_field_magnitude * mu_B (Hamiltonian_Heisenberg.cpp:35)
@@ -100,6 +101,13 @@ struct HamDev
     PairDev exch_g[GATHER_PAIRS];
     PairDev dmi_g[GATHER_PAIRS];
 };
+
+// The exchange pairs of an image fit one gathered group and its DMI pairs are among them
+// (local_gradient<FEW>).
+inline bool few_pairs( const HamDev & H )
+{
+    return H.n_exch <= GATHER_PAIRS && H.dmi_same;
+}
 
 // Spin-transfer torque of the dynamics' virtual force (Method_LLG.cpp:182-212).
 enum SttMode

@@ -81,6 +81,7 @@ struct GnebArgs
 {
     const ImageDev * imgs;
     int noi, nos, bpi, n_blocks; // images, spins per image, blocks per image, blocks
+    int few_pairs;               // every image's pair tables are few_pairs
     const double * x;            // configuration of this force evaluation
     const double * xc;           // the chain's current spins (path shortening, translation)
     const double * h;            // DDI field of x (nullable)

@@ -57,11 +57,14 @@ GNEBRunner::GNEBRunner( const std::vector<ImageSpec> & images, const GNEBParamet
     HIPCHECK( hipMemsetAsync( b_stop.as<void>(), 0, sizeof( int ), st ) );
     HIPCHECK( hipMemsetAsync( b_iter.as<void>(), 0, sizeof( long long ), st ) );
 
-    A.imgs     = field->dev_images();
-    A.noi      = noi;
-    A.nos      = nos;
-    A.bpi      = bpi;
-    A.n_blocks = noi * bpi;
+    A.imgs      = field->dev_images();
+    A.noi       = noi;
+    A.nos       = nos;
+    A.bpi       = bpi;
+    A.n_blocks  = noi * bpi;
+    A.few_pairs = 1;
+    for( int k = 0; k < noi; ++k )
+        A.few_pairs = A.few_pairs && few_pairs( field->image_host( k ).ham );
     A.xc       = field->dev_spins();
     A.eff      = b_eff.as<double>();
     A.Fg       = b_Fg.as<double>();

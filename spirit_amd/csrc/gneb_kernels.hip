@@ -248,7 +248,8 @@ __device__ __forceinline__ void pass_tail( const GnebArgs & A );
 // One per-spin pass over every image of the chain; with PHASE >= 0 the last block to finish
 // runs that chain phase on the pass's partial sums (pass_tail), so a pass and the chain step
 // that consumes it are one launch.
-template<int PASS, int PHASE>
+// FEW: local_gradient's (the gradient pass).
+template<int PASS, int PHASE, bool FEW = false>
 __global__ void __launch_bounds__( GNEB_THREADS ) k_gneb_pass( GnebArgs A )
 {
     if( *A.stop )
@@ -272,7 +273,7 @@ __global__ void __launch_bounds__( GNEB_THREADS ) k_gneb_pass( GnebArgs A )
         {
             const ImageDev & I = A.imgs[img];
             double g[3], e;
-            local_gradient( I.ham, A.x + base, nos, i, ( A.h && I.ham.has_ddi ) ? A.h + base : nullptr, g, e );
+            local_gradient<FEW>( I.ham, A.x + base, nos, i, ( A.h && I.ham.has_ddi ) ? A.h + base : nullptr, g, e );
             v[0] = e;
             double ef[3] = { -1 * g[0], -1 * g[1], -1 * g[2] };
             store3( A.eff + base, nos, i, ef );
@@ -1033,11 +1034,11 @@ __global__ void __launch_bounds__( GNEB_THREADS ) k_gneb_stage( GnebSolverArgs S
 // ---------------------------------------------------------------------------
 // host launchers
 // ---------------------------------------------------------------------------
-template<int PASS, int PHASE>
+template<int PASS, int PHASE, bool FEW = false>
 static void launch_pass( const GnebArgs & A, dim3 grid, hipStream_t st )
 {
     const size_t lds = ( PHASE >= 0 && A.noi <= GNEB_CH_LDS ) ? sizeof( double ) * A.noi * GNEB_NCH : 0;
-    hipLaunchKernelGGL( ( k_gneb_pass<PASS, PHASE> ), grid, dim3( GNEB_THREADS ), lds, st, A );
+    hipLaunchKernelGGL( ( k_gneb_pass<PASS, PHASE, FEW> ), grid, dim3( GNEB_THREADS ), lds, st, A );
 }
 
 void gneb_launch_pass( int pass, const GnebArgs & A, hipStream_t st )
@@ -1045,7 +1046,12 @@ void gneb_launch_pass( int pass, const GnebArgs & A, hipStream_t st )
     const dim3 all( A.n_blocks ), first( A.bpi );
     switch( pass )
     {
-        case GPASS_GRAD: launch_pass<GPASS_GRAD, GPH_DIST>( A, all, st ); break;
+        case GPASS_GRAD:
+            if( A.few_pairs )
+                launch_pass<GPASS_GRAD, GPH_DIST, true>( A, all, st );
+            else
+                launch_pass<GPASS_GRAD, GPH_DIST, false>( A, all, st );
+            break;
         case GPASS_TANGENT: launch_pass<GPASS_TANGENT, GPH_TANGENT>( A, all, st ); break;
         case GPASS_TRANSLATE: launch_pass<GPASS_TRANSLATE, GPH_TRANSLATE>( A, first, st ); break;
         case GPASS_SHRINK1: launch_pass<GPASS_SHRINK1, GPH_SHRINK1>( A, all, st ); break;

@@ -685,11 +685,11 @@ int fill_ham_dev( const Geometry & g, const Hamiltonian & h, HamDev & H, PairDev
     }
     H.n_exch = (int)h.exch_pairs.size();
     H.n_dmi  = (int)h.dmi_pairs.size();
-    for( int k = 0; k < H.n_exch; ++k )
+    for( size_t k = 0; k < np; ++k )
     {
-        H.halo[0] = std::max( H.halo[0], std::abs( pv[k].da ) );
-        H.halo[1] = std::max( H.halo[1], std::abs( pv[k].db ) );
-        H.halo[2] = std::max( H.halo[2], std::abs( pv[k].dc ) );
+        H.reach[0] = std::max( H.reach[0], std::abs( pv[k].da ) );
+        H.reach[1] = std::max( H.reach[1], std::abs( pv[k].db ) );
+        H.reach[2] = std::max( H.reach[2], std::abs( pv[k].dc ) );
     }
     // stage-kernel row tile: 16 rows by default (256x256x128 Depondt+DDI: 0.308 / 0.300 /
     // 0.287 / 0.286 ms per stage at 4 / 8 / 16 / 32 rows); SPIRIT_HIP_STAGE_ROW_TILE (a power
@@ -1387,16 +1387,20 @@ static StepArgs base_args_of( DeviceBuffer & imgs, DeviceBuffer & blk, DeviceBuf
     return A;
 }
 
-static StepArgs with_stt( StepArgs A, int stt_gradient )
+// the choices between instantiations of a kernel that all images of a launch share
+static StepArgs with_variants( StepArgs A, int stt_gradient, const std::vector<ImageDev> & imgs )
 {
     A.stt_gradient = stt_gradient;
+    A.few_pairs    = 1;
+    for( const auto & I : imgs )
+        A.few_pairs = A.few_pairs && few_pairs( I.ham );
     return A;
 }
 
 #define STEP_ARGS()                                                                                                    \
-    with_stt( base_args_of( b_imgs, b_blk, b_s, b_sp, b_sp2, b_aux, b_aux2, b_h, b_eff, b_efft, b_pE, b_pT, b_stop,   \
-                            b_img_stop, b_xi ),                                                                        \
-              stt_gradient_any )
+    with_variants( base_args_of( b_imgs, b_blk, b_s, b_sp, b_sp2, b_aux, b_aux2, b_h, b_eff, b_efft, b_pE, b_pT,      \
+                                 b_stop, b_img_stop, b_xi ),                                                           \
+                   stt_gradient_any, imgs_host )
 
 // The stage kernels' row tile (rows along b swept through the c planes) by timing: the first
 // solver stage at tiles of 8, 16 and 32 rows (64 measured 5-8% slower than 32), where every

@@ -233,29 +233,120 @@ __device__ __forceinline__ int pair_neighbour( const HamDev & H, int a, int b, i
     return p.j + H.nb * ( ja + Na * ( jb + Nb * jc ) );
 }
 
-// neighbours a spin gathers into registers before using them (larger tables loop)
+// The same neighbour (-1: beyond an open boundary) from the pair's fixed index offset: away from the
+// boundaries the neighbour is i + delta, and along an axis with a translation one comparison of the
+// site's coordinate with a uniform number says whether to wrap.  Three vector instructions per axis
+// the pair leaves, against about thirty for the coordinates' general wrap.
+__device__ __forceinline__ int pair_neighbour_delta( const HamDev & H, int i, int a, int b, int c, const PairDev & p )
+{
+    const int N[3] = { H.Na, H.Nb, H.Nc }, x[3] = { a, b, c }, d[3] = { p.da, p.db, p.dc };
+    int j = i + p.delta, unit = H.nb;
+    bool out = false;
+#pragma unroll
+    for( int u = 0; u < 3; ++u )
+    {
+        const int wrap = unit * N[u];
+        if( abs( d[u] ) > N[u] )
+            return -1;
+        if( d[u] > 0 )
+        {
+            const bool w = x[u] >= N[u] - d[u];
+            j -= w ? wrap : 0;
+            out = out || ( w && !H.bc[u] );
+        }
+        else if( d[u] < 0 )
+        {
+            const bool w = x[u] < -d[u];
+            j += w ? wrap : 0;
+            out = out || ( w && !H.bc[u] );
+        }
+        unit = wrap;
+    }
+    return out ? -1 : j;
+}
+
+// neighbours a spin gathers into registers before using them (larger tables in groups)
 constexpr int LG_MAX_NB = GATHER_PAIRS;
 
-// The exchange neighbours of spin i (tables of up to LG_MAX_NB pairs), all loads issued
-// before any is used.  A pair that does not start at this basis atom or leaves an open
-// boundary reads the spin itself and yields exactly zero (its loaded values are replaced).
+// The exchange neighbours of spin i (a table of few_pairs), all loads issued before any is used.
+// A pair that does not start at this basis atom or leaves an open boundary reads the spin itself
+// and yields exactly zero (its loaded values are replaced).
 __device__ __forceinline__ void gather_exchange_neighbours( const HamDev & H, const double * __restrict__ x, int nos,
                                                             int i, int ib, int a, int b, int c,
                                                             double ( &se )[LG_MAX_NB][3] )
 {
-    // away from every boundary a neighbour is the site's index plus a fixed offset
-    const bool interior = a >= H.halo[0] && a < H.Na - H.halo[0] && b >= H.halo[1] && b < H.Nb - H.halo[1]
-                          && c >= H.halo[2] && c < H.Nc - H.halo[2];
 #pragma unroll
     for( int k = 0; k < LG_MAX_NB; ++k )
         if( k < H.n_exch )
         {
             const PairDev & p = H.exch_g[k];
-            const int j = p.i != ib ? -1 : interior ? i + p.delta : pair_neighbour( H, a, b, c, p );
+            const int j       = p.i != ib ? -1 : pair_neighbour_delta( H, i, a, b, c, p );
             load3( x, nos, j >= 0 ? j : i, se[k] );
             if( j < 0 )
                 se[k][0] = se[k][1] = se[k][2] = 0.0;
         }
+}
+
+// Index offsets of the sites up to MAX_REACH cells away along each axis, one column of LDS per
+// thread: a pair of a long table then costs three LDS reads and two additions instead of its
+// coordinates' comparisons and branches (1200 vector and 1100 scalar instructions a spin with 26
+// pairs otherwise).  Offsets beyond an open boundary make the sum of three negative for any site.
+constexpr int NO_SITE = -( 1 << 29 );
+struct SiteOffsets
+{
+    int ( *tab )[256];
+    __device__ __forceinline__ SiteOffsets( const HamDev & H, int a, int b, int c )
+    {
+        __shared__ int lds[3 * ( 2 * MAX_REACH + 1 )][256];
+        tab = lds;
+        const int N[3] = { H.Na, H.Nb, H.Nc }, x[3] = { a, b, c };
+        int unit = H.nb;
+#pragma unroll
+        for( int u = 0; u < 3; ++u )
+        {
+            for( int d = -H.reach[u]; d <= H.reach[u]; ++d )
+            {
+                const int t  = x[u] + d;
+                const int up = t < 0 ? N[u] : t >= N[u] ? -N[u] : 0;
+                const bool no = abs( d ) > N[u] || ( up != 0 && !H.bc[u] );
+                tab[u * ( 2 * MAX_REACH + 1 ) + MAX_REACH + d][threadIdx.x] = no ? NO_SITE : ( d + up ) * unit;
+            }
+            unit *= N[u];
+        }
+    }
+    // index of the pair's other site, negative where there is none
+    __device__ __forceinline__ int neighbour( const PairDev & p, int i, int ib ) const
+    {
+        constexpr int W = 2 * MAX_REACH + 1;
+        const int j     = i - ib + p.j + tab[MAX_REACH + p.da][threadIdx.x] + tab[W + MAX_REACH + p.db][threadIdx.x]
+                      + tab[2 * W + MAX_REACH + p.dc][threadIdx.x];
+        return p.i == ib ? j : -1;
+    }
+};
+
+// f( k, spin, weight ) for the n pairs at p of spin i, weight 0 (and the spin itself) for a pair
+// without a neighbour; the loads of a group of LG_MAX_NB pairs are issued before any is used
+template<typename F>
+__device__ __forceinline__ void for_pairs( const HamDev & H, const SiteOffsets & off, const PairDev * __restrict__ p,
+                                           int n, const double * __restrict__ x, int nos, int i, int ib, F f )
+{
+    for( int k0 = 0; k0 < n; k0 += LG_MAX_NB )
+    {
+        double se[LG_MAX_NB][3];
+        bool is[LG_MAX_NB];
+#pragma unroll
+        for( int k = 0; k < LG_MAX_NB; ++k )
+        {
+            // the last group reads its last pair again rather than branch around each load
+            const PairDev & q = p[k0 + k < n ? k0 + k : n - 1];
+            const int j       = off.neighbour( q, i, ib );
+            is[k]             = j >= 0 && k0 + k < n;
+            load3( x, nos, j >= 0 ? j : i, se[k] );
+        }
+#pragma unroll
+        for( int k = 0; k < LG_MAX_NB; ++k )
+            f( k0 + k < n ? k0 + k : n - 1, se[k], is[k] ? 1.0 : 0.0 );
+    }
 }
 
 // The quadruplet part of spin i's gradient, gathered: Gradient_Quadruplet
@@ -336,6 +427,9 @@ __device__ __forceinline__ void quadruplet_gradient( const HamDev & H, const dou
 
 // Gradient_and_Energy for one spin: g (all terms) and its energy share e
 // (1/2 g.s over aniso+exchange+DMI+DDI, plus the cubic and Zeeman energies).
+// FEW: every image's exchange table fits one group and holds its DMI pairs (few_pairs), the usual
+// nearest-neighbour model; its kernels need no group loops, which cost ten registers.
+template<bool FEW = false>
 __device__ __forceinline__ void local_gradient( const HamDev & H, const double * __restrict__ x, int nos, int i,
                                                 const double * __restrict__ hddi, double * g, double & e )
 {
@@ -353,9 +447,8 @@ __device__ __forceinline__ void local_gradient( const HamDev & H, const double *
     double hd[3]    = { 0, 0, 0 };
     if( hddi )
         load3( hddi, nos, i, hd );
-    const bool gather = H.n_exch <= LG_MAX_NB;
-    double se[LG_MAX_NB][3];
-    if( gather )
+    double se[FEW ? LG_MAX_NB : 1][3];
+    if constexpr( FEW )
         gather_exchange_neighbours( H, x, nos, i, ib, a, b, c, se );
     g[0] = g[1] = g[2] = 0;
     // anisotropy, :785-800
@@ -376,8 +469,9 @@ __device__ __forceinline__ void local_gradient( const HamDev & H, const double *
         for( int q = 0; q < 3; ++q )
             g[q] -= 2.0 * Ki * H.site_n[q] * d;
     }
-    // exchange, :822-842 (gather over the redundant table)
-    if( gather )
+    // exchange, :822-842, and DMI, :844-864 (gather over the redundant tables; the DMI pairs use the
+    // exchange pairs' neighbours where the tables coincide)
+    if constexpr( FEW )
     {
 #pragma unroll
         for( int k = 0; k < LG_MAX_NB; ++k )
@@ -388,24 +482,6 @@ __device__ __forceinline__ void local_gradient( const HamDev & H, const double *
                 for( int q = 0; q < 3; ++q )
                     g[q] -= J * se[k][q];
             }
-    }
-    else
-        for( int k = 0; k < H.n_exch; ++k )
-        {
-            const PairDev & p = H.exch[k];
-            if( p.i != ib )
-                continue;
-            int j = pair_neighbour( H, a, b, c, p );
-            if( j >= 0 )
-            {
-                g[0] -= p.J * x[j];
-                g[1] -= p.J * x[nos + j];
-                g[2] -= p.J * x[2 * nos + j];
-            }
-        }
-    // DMI, :844-864 (on the exchange pairs' neighbours when the tables coincide)
-    if( gather && H.dmi_same )
-    {
 #pragma unroll
         for( int k = 0; k < LG_MAX_NB; ++k )
             if( k < H.n_dmi )
@@ -418,23 +494,44 @@ __device__ __forceinline__ void local_gradient( const HamDev & H, const double *
                     g[q] -= p.D * cr[q];
             }
     }
-    else
-        for( int k = 0; k < H.n_dmi; ++k )
-        {
-            const PairDev & p = H.dmi[k];
-            if( p.i != ib )
-                continue;
-            int j = pair_neighbour( H, a, b, c, p );
-            if( j >= 0 )
-            {
-                const double sj[3] = { x[j], x[nos + j], x[2 * nos + j] };
-                double cr[3];
-                cross3( sj, p.n, cr );
+    else if( H.reach[0] <= MAX_REACH && H.reach[1] <= MAX_REACH && H.reach[2] <= MAX_REACH && H.nos < -NO_SITE )
+    {
+        const SiteOffsets off( H, a, b, c );
+        const PairDev * __restrict__ ex = H.exch;
+        const PairDev * __restrict__ dm = H.dmi;
+        for_pairs( H, off, ex, H.n_exch, x, nos, i, ib, [&]( int k, const double * sj, double w ) {
+            const double J = w * ex[k].J;
 #pragma unroll
-                for( int q = 0; q < 3; ++q )
-                    g[q] -= p.D * cr[q];
-            }
+            for( int q = 0; q < 3; ++q )
+                g[q] -= J * sj[q];
+        } );
+        for_pairs( H, off, dm, H.n_dmi, x, nos, i, ib, [&]( int k, const double * sj, double w ) {
+            const double D = w * dm[k].D;
+            double cr[3];
+            cross3( sj, dm[k].n, cr );
+#pragma unroll
+            for( int q = 0; q < 3; ++q )
+                g[q] -= D * cr[q];
+        } );
+    }
+    else
+    {
+        // pairs further away than the offset table reaches (or indices beyond its marker)
+        for( int k = 0; k < H.n_exch + H.n_dmi; ++k )
+        {
+            const bool ex     = k < H.n_exch;
+            const PairDev & p = ex ? H.exch[k] : H.dmi[k - H.n_exch];
+            const int j       = p.i != ib ? -1 : pair_neighbour_delta( H, i, a, b, c, p );
+            if( j < 0 )
+                continue;
+            double sj[3], cr[3];
+            load3( x, nos, j, sj );
+            cross3( sj, p.n, cr );
+#pragma unroll
+            for( int q = 0; q < 3; ++q )
+                g[q] -= ex ? p.J * sj[q] : p.D * cr[q];
         }
+    }
     // DDI field (precomputed by the FFT passes), :995-1013
     if( hddi )
     {

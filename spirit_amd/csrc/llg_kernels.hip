@@ -24,8 +24,9 @@ namespace spirit_hip
 // the stage kernel
 // ---------------------------------------------------------------------------
 // STT_G: some image takes the spin-transfer torque from the spin's derivative along the
-// current (a separate instantiation: its six neighbour loads cost registers the others need)
-template<int SOLVER, int STAGE, bool STT_G>
+// current (a separate instantiation: its six neighbour loads cost registers the others need);
+// FEW: local_gradient's
+template<int SOLVER, int STAGE, bool STT_G, bool FEW>
 __global__ void __launch_bounds__( LLG_THREADS ) k_llg_stage( StepArgs A )
 {
     if( *A.stop )
@@ -62,7 +63,7 @@ __global__ void __launch_bounds__( LLG_THREADS ) k_llg_stage( StepArgs A )
         if( FV1_IN )
             load3( A.aux + base, nos, i, fv1 );
         double g[3], e;
-        local_gradient( H, x, nos, i, ( A.h && H.has_ddi ) ? A.h + base : nullptr, g, e );
+        local_gradient<FEW>( H, x, nos, i, ( A.h && H.has_ddi ) ? A.h + base : nullptr, g, e );
         e_i            = e;
         const double mu = H.mu[basis_of( H, i )];
         double si[3];
@@ -334,6 +335,7 @@ void llg_launch_observe( const StepArgs & A, int solver, int n_blocks, hipStream
 }
 
 // Gradient (SoA) and energy partials of a configuration, for getters and parity tests.
+template<bool FEW>
 __global__ void __launch_bounds__( LLG_THREADS ) k_gradient( StepArgs A, const double * __restrict__ x0,
                                                             double * __restrict__ grad )
 {
@@ -347,7 +349,7 @@ __global__ void __launch_bounds__( LLG_THREADS ) k_gradient( StepArgs A, const d
     if( i < nos )
     {
         double g[3], e;
-        local_gradient( H, x0 + base, nos, i, ( A.h && H.has_ddi ) ? A.h + base : nullptr, g, e );
+        local_gradient<FEW>( H, x0 + base, nos, i, ( A.h && H.has_ddi ) ? A.h + base : nullptr, g, e );
         e_i = e;
         store3( grad + base, nos, i, g );
     }
@@ -453,10 +455,10 @@ __global__ void __launch_bounds__( FIN_THREADS )
 template<int SOLVER, int STAGE>
 static void launch_stage( const StepArgs & A, int n_blocks, hipStream_t st )
 {
-    if( A.stt_gradient )
-        hipLaunchKernelGGL( ( k_llg_stage<SOLVER, STAGE, true> ), dim3( n_blocks ), dim3( LLG_THREADS ), 0, st, A );
-    else
-        hipLaunchKernelGGL( ( k_llg_stage<SOLVER, STAGE, false> ), dim3( n_blocks ), dim3( LLG_THREADS ), 0, st, A );
+    const auto k = A.stt_gradient ? k_llg_stage<SOLVER, STAGE, true, false>
+                   : A.few_pairs  ? k_llg_stage<SOLVER, STAGE, false, true>
+                                  : k_llg_stage<SOLVER, STAGE, false, false>;
+    hipLaunchKernelGGL( k, dim3( n_blocks ), dim3( LLG_THREADS ), 0, st, A );
 }
 
 __global__ void k_step_advance( uint64_t * step, int by )
@@ -508,7 +510,8 @@ void llg_launch_stage( int solver, int stage, const StepArgs & A, int n_blocks, 
 
 void llg_launch_gradient( const StepArgs & A, const double * x, double * grad, int n_blocks, hipStream_t st )
 {
-    hipLaunchKernelGGL( k_gradient, dim3( n_blocks ), dim3( LLG_THREADS ), 0, st, A, x, grad );
+    const auto k = A.few_pairs ? k_gradient<true> : k_gradient<false>;
+    hipLaunchKernelGGL( k, dim3( n_blocks ), dim3( LLG_THREADS ), 0, st, A, x, grad );
 }
 
 void llg_launch_finalize( const StepArgs & A, int n_images, double * obs, int * img_stop, int * n_stopped,

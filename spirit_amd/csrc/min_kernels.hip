@@ -184,7 +184,7 @@ __device__ __forceinline__ void atlas_rotate( const double * sp, double a3, cons
 // force evaluation: energy partials, force, solver gradient, velocity (VP) or the newest
 // L-BFGS pair and its dot products.  Chains take their forces from M.F_ext.
 // ---------------------------------------------------------------------------
-template<int SOLVER>
+template<int SOLVER, bool FEW>
 __global__ void __launch_bounds__( LLG_THREADS ) k_min_force( StepArgs A, MinArgs M, int nos )
 {
     if( min_stopped( A, M ) )
@@ -203,7 +203,7 @@ __global__ void __launch_bounds__( LLG_THREADS ) k_min_force( StepArgs A, MinArg
         {
             const HamDev & H = A.imgs->ham;
             double g[3], e;
-            local_gradient( H, A.s, nos, i, ( A.h && H.has_ddi ) ? A.h : nullptr, g, e );
+            local_gradient<FEW>( H, A.s, nos, i, ( A.h && H.has_ddi ) ? A.h : nullptr, g, e );
             x[3] = e;
             F[0] = -1 * g[0], F[1] = -1 * g[1], F[2] = -1 * g[2];
             store3( M.f, nos, i, F );
@@ -722,7 +722,8 @@ template<int SOLVER>
 static void vp_iteration( const StepArgs & A, const MinArgs & M, int nos, hipStream_t st )
 {
     const dim3 g( M.n_blocks ), b( LLG_THREADS );
-    hipLaunchKernelGGL( k_min_force<SOLVER>, g, b, 0, st, A, M, nos );
+    const auto force = A.few_pairs ? k_min_force<SOLVER, true> : k_min_force<SOLVER, false>;
+    hipLaunchKernelGGL( force, g, b, 0, st, A, M, nos );
     launch_scalar( A, M, PH_VP, 0, nos, st );
     hipLaunchKernelGGL( k_min_update<SOLVER>, g, b, 0, st, A, M, nos );
 }
@@ -732,7 +733,8 @@ static void lbfgs_iteration( const StepArgs & A, const MinArgs & M, int nos, hip
 {
     constexpr int D = SOLVER == SOLVER_LBFGS_ATLAS ? 2 : 3;
     const dim3 g( M.n_blocks ), b( LLG_THREADS );
-    hipLaunchKernelGGL( k_min_force<SOLVER>, g, b, 0, st, A, M, nos );
+    const auto force = A.few_pairs ? k_min_force<SOLVER, true> : k_min_force<SOLVER, false>;
+    hipLaunchKernelGGL( force, g, b, 0, st, A, M, nos );
     launch_scalar( A, M, PH_RHO, 0, nos, st );
     for( int k = MIN_MEMORY - 2; k >= 0; --k )
     {

@@ -234,10 +234,11 @@ try
     hipLaunchKernelGGL( k_na_aos_to_soa, dim3( n_blocks ), dim3( LLG_THREADS ), 0, st, spins, d_x, nos );
 
     StepArgs A{};
-    A.imgs    = d_img;
-    A.blk_img = d_blk_img;
-    A.part_E  = d_part_E;
-    A.part_T  = d_part_T;
+    A.imgs      = d_img;
+    A.blk_img   = d_blk_img;
+    A.part_E    = d_part_E;
+    A.part_T    = d_part_T;
+    A.few_pairs = few_pairs( I.ham ) ? 1 : 0;
     llg_launch_gradient( A, d_x, d_g, n_blocks, st );
     hipLaunchKernelGGL( k_na_soa_to_aos, dim3( n_blocks ), dim3( LLG_THREADS ), 0, st, d_g, gradient, nos );
     hipLaunchKernelGGL( k_na_sum_partials, dim3( 1 ), dim3( 64 ), 0, st, d_part_E, n_blocks, energy );
