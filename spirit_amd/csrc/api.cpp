@@ -799,6 +799,7 @@ static std::shared_ptr<MethodMC> mc_setup( State * state, const std::shared_ptr<
 // n Metropolis iterations (Method_MC::Iteration, Method_MC.cpp:40-183) on the device
 static void mc_sweeps( MethodMC & m, long n )
 {
+    m.A.few_pairs = few_pairs( m.runner->image_host( 0 ).ham ) ? 1 : 0; // the Hamiltonian may have changed
     for( long k = 0; k < n; ++k )
         mc_launch_iteration( m.A, m.step.as<uint64_t>(), m.runner->stream );
     HIPCHECK( hipGetLastError() );
@@ -815,7 +816,7 @@ static void mc_download( MethodMC & m )
     HIPCHECK( hipMemcpy( &cone_end, m.cone.as<void>(), sizeof( double ), hipMemcpyDeviceToHost ) );
     if( P.metropolis_step_cone && P.metropolis_cone_adaptive )
         P.metropolis_cone_angle = cone_end * 180.0 / Pi;
-    m.image->E = update_image_energy( *m.image, true );
+    m.image->E = update_image_energy( *m.image, *m.runner, 0, true );
 }
 
 // Method_MC::Finalize (Method_MC.cpp:203-206) of a single-shot run

@@ -40,6 +40,7 @@ void notify_image_changed( State * state, int idx_image, bool spins_changed, boo
 bool stop_file_present();
 // energy, effective field (store_field) and energy contributions of an image's host spins,
 // evaluated on the GPU; per_spin (nullable) receives the six per-spin terms [6][nos]
+double update_image_energy( Image & image, LLGRunner & r, int img, bool store_field );
 double update_image_energy( Image & image, bool store_field, std::vector<double> * per_spin = nullptr );
 std::vector<std::pair<std::string, int>> energy_contribution_list( const Image & image );
 void llg_save_configuration( const Image & img, int idx_image, const std::string & starttime, long iteration,

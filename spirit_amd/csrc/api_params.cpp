@@ -531,6 +531,18 @@ std::vector<std::pair<std::string, int>> spirit_hip::energy_contribution_list( c
     return c;
 }
 
+// the image's energy, contributions and (with store_field) effective field from a runner that holds
+// its current spins
+double spirit_hip::update_image_energy( Image & image, LLGRunner & r, int img, bool store_field )
+{
+    double sums[N_ENERGY_TERMS_HOST];
+    const double E = r.energy_and_sums( img, store_field ? image.eff_field.data() : nullptr, sums );
+    image.E_array.clear();
+    for( auto & c : energy_contribution_list( image ) )
+        image.E_array.push_back( { c.first, sums[c.second] } );
+    return E;
+}
+
 // The energy of the image's host spins, with the effective field -dE/ds and the energy
 // contributions (Spin_System::UpdateEnergy / UpdateEffectiveField, core/src/data/Spin_System.cpp:138-161,
 // Hamiltonian_Heisenberg::Energy_Contributions), evaluated on the GPU.
@@ -538,24 +550,12 @@ double spirit_hip::update_image_energy( Image & image, bool store_field, std::ve
 {
     ImageSpec sp{ image.geometry, image.hamiltonian, *image.llg, image.spins.data() };
     LLGRunner r( { sp }, SOLVER_DEPONDT );
-    std::vector<double> g( 3 * (size_t)image.nos() );
-    double E = r.gradient( 0, g.data() );
-    if( store_field )
-        for( size_t k = 0; k < g.size(); ++k )
-            image.eff_field[k] = -1 * g[k];
-    const size_t nos = (size_t)image.nos();
-    std::vector<double> terms( N_ENERGY_TERMS_HOST * nos );
-    r.energy_terms( 0, terms.data() );
-    image.E_array.clear();
-    for( auto & c : energy_contribution_list( image ) )
-    {
-        double sum = 0;
-        for( size_t i = 0; i < nos; ++i )
-            sum += terms[(size_t)c.second * nos + i];
-        image.E_array.push_back( { c.first, sum } );
-    }
+    const double E = update_image_energy( image, r, 0, store_field );
     if( per_spin )
-        *per_spin = std::move( terms );
+    {
+        per_spin->resize( N_ENERGY_TERMS_HOST * (size_t)image.nos() );
+        r.energy_terms( 0, per_spin->data() );
+    }
     return E;
 }
 

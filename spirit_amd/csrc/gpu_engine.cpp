@@ -1734,6 +1734,48 @@ void LLGRunner::energy_terms( int img, double * out )
                          hipMemcpyDeviceToHost ) );
 }
 
+double LLGRunner::energy_and_sums( int img, double * field_aos, double * sums )
+{
+    StepArgs A = STEP_ARGS();
+    if( any_ddi )
+        ddi_field( A.s );
+    // the observation stores -gradient in b_eff and every block's energy
+    llg_launch_observe( A, SOLVER_DEPONDT, n_blocks, stream );
+    eff_raw = true;
+    DeviceBuffer part( sizeof( double ) * N_ENERGY_TERMS_HOST * (size_t)n_blocks );
+    llg_launch_energy_sums( A, A.s, part.as<double>(), n_blocks, stream );
+    const ImageDev & I = imgs_host[img];
+    const size_t nb    = (size_t)I.n_blocks;
+    std::vector<double> pE( nb ), pt( N_ENERGY_TERMS_HOST * (size_t)n_blocks );
+    HIPCHECK( hipGetLastError() );
+    HIPCHECK( hipMemcpyAsync( pE.data(), b_pE.as<double>() + I.block_begin, sizeof( double ) * nb,
+                              hipMemcpyDeviceToHost, stream ) );
+    HIPCHECK( hipMemcpyAsync( pt.data(), part.as<void>(), sizeof( double ) * pt.size(), hipMemcpyDeviceToHost,
+                              stream ) );
+    if( field_aos )
+    {
+        if( b_stage.size() < sizeof( double ) * 3 * (size_t)n_total )
+            b_stage.resize( sizeof( double ) * 3 * (size_t)n_total );
+        device_soa_to_aos( b_eff.as<double>() + 3 * I.off, b_stage.as<double>() + 3 * I.off,
+                           specs[img].geometry->nos, stream );
+        HIPCHECK( hipGetLastError() );
+        std::vector<double *> dst( specs.size(), nullptr );
+        dst[img] = field_aos;
+        stage_to_host( dst );
+    }
+    HIPCHECK( hipStreamSynchronize( stream ) );
+    for( int t = 0; t < N_ENERGY_TERMS_HOST; ++t )
+    {
+        sums[t] = 0;
+        for( size_t b = 0; b < nb; ++b )
+            sums[t] += pt[(size_t)t * n_blocks + I.block_begin + b];
+    }
+    double E = 0;
+    for( double v : pE )
+        E += v;
+    return E;
+}
+
 double LLGRunner::gradient( int img, double * grad_aos )
 {
     StepArgs A = STEP_ARGS();

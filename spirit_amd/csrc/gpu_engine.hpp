@@ -200,6 +200,9 @@ public:
     // per-spin energy contributions of image img's current spins, out[t * nos + i] for the
     // N_ENERGY_TERMS_HOST terms Zeeman, anisotropy, cubic anisotropy, exchange, DMI, DDI, quadruplets
     void energy_terms( int img, double * out );
+    // energy of image img's current spins, its contributions sums[0 .. N_ENERGY_TERMS_HOST) in that order
+    // and, where field_aos is given, the field -gradient (AoS); with the runner's own buffers
+    double energy_and_sums( int img, double * field_aos, double * sums );
     // injected N(0,1) noise for the next `n_steps` steps, AoS per spin over all images
     void set_injected_noise( const double * noise, long n_steps );
 

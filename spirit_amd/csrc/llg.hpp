@@ -49,6 +49,8 @@ void llg_launch_gradient( const StepArgs & A, const double * x, double * grad, i
 // anisotropy, exchange, DMI, DDI, quadruplets ([term][spin] per image)
 constexpr int N_ENERGY_TERMS_HOST = 7;
 void llg_launch_energy_terms( const StepArgs & A, const double * x, double * out, int n_blocks, hipStream_t st );
+// the contributions summed over each block, part[term * n_blocks + block]
+void llg_launch_energy_sums( const StepArgs & A, const double * x, double * part, int n_blocks, hipStream_t st );
 void llg_launch_observe( const StepArgs & A, int solver, int n_blocks, hipStream_t st );
 // out = F - (F.s) s per spin (one image's SoA fields)
 void llg_launch_project_field( const double * F, const double * s, double * out, int nos, hipStream_t st );

@@ -378,6 +378,45 @@ __global__ void __launch_bounds__( LLG_THREADS ) k_energy_terms( StepArgs A, con
 
 static_assert( N_ENERGY_TERMS == N_ENERGY_TERMS_HOST, "energy term count" );
 
+// The contributions summed over each block's spins, part[term * gridDim.x + block]: callers that want
+// the sums read 56 bytes a block instead of 56 a spin.
+__global__ void __launch_bounds__( LLG_THREADS ) k_energy_sums( StepArgs A, const double * __restrict__ x0,
+                                                               double * __restrict__ part )
+{
+    __shared__ double sh[N_ENERGY_TERMS][LLG_THREADS / 64];
+    const int blk           = xcd_contiguous_block();
+    const ImageDev * __restrict__ I = A.imgs + A.blk_img[blk];
+    const HamDev & H        = I->ham;
+    const int nos           = H.nos;
+    const long long base    = 3 * I->off;
+    const int i             = ( blk - I->block_begin ) * LLG_THREADS + threadIdx.x;
+    double E[N_ENERGY_TERMS] = {};
+    if( i < nos )
+        local_energy_terms( H, x0 + base, nos, i, ( A.h && H.has_ddi ) ? A.h + base : nullptr, E );
+#pragma unroll
+    for( int t = 0; t < N_ENERGY_TERMS; ++t )
+    {
+#pragma unroll
+        for( int off = 32; off > 0; off >>= 1 )
+            E[t] += __shfl_down( E[t], off, 64 );
+        if( threadIdx.x % 64 == 0 )
+            sh[t][threadIdx.x / 64] = E[t];
+    }
+    __syncthreads();
+    if( threadIdx.x < N_ENERGY_TERMS )
+    {
+        double e = sh[threadIdx.x][0];
+        for( int w = 1; w < LLG_THREADS / 64; ++w )
+            e += sh[threadIdx.x][w];
+        part[(long long)threadIdx.x * gridDim.x + blk] = e;
+    }
+}
+
+void llg_launch_energy_sums( const StepArgs & A, const double * x, double * part, int n_blocks, hipStream_t st )
+{
+    hipLaunchKernelGGL( k_energy_sums, dim3( n_blocks ), dim3( LLG_THREADS ), 0, st, A, x, part );
+}
+
 void llg_launch_energy_terms( const StepArgs & A, const double * x, double * out, int n_blocks, hipStream_t st )
 {
     hipLaunchKernelGGL( k_energy_terms, dim3( n_blocks ), dim3( LLG_THREADS ), 0, st, A, x, out );

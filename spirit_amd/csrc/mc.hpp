@@ -28,6 +28,7 @@ struct McArgs
     int groups;            // ceil(Na / K): groups of K cells per row
     int n_blocks_rows;     // blocks of the per-colour sweep (<= n_blocks)
     const uint64_t * step; // Monte Carlo step index (random-number counter)
+    int few_pairs;         // the image's pair tables are few_pairs
 };
 
 // One Metropolis iteration: the cone feedback from the previous iteration's rejections, then
