@@ -151,6 +151,42 @@ __device__ __forceinline__ double u53( uint32_t a, uint32_t b )
 {
     return ( (double)( a >> 5 ) * 67108864.0 + (double)( b >> 6 ) ) * ( 1.0 / 9007199254740992.0 );
 }
+// log u of a uniform u in (0, 1], u a multiple of 2^-53: no infinities, denormals or negative
+// arguments to sort out.  With u = m 2^k, m in [sqrt(1/2), sqrt(2)), f = m - 1 and s = f / (2 + f),
+// log m = 2 artanh s = f - s (f - 2 (s^2/3 + s^4/5 + ...)); s^2 <= 0.0295, the first omitted term is
+// below 2.4e-17 of f.  s itself counts only by a sixth of f, so a reciprocal with two Newton steps is
+// enough for it.  At most 1.1 units in the last place off (2 10^7 values over all binades).
+__device__ __forceinline__ double log_uniform( double u )
+{
+    int k;
+    double m       = frexp( u, &k );
+    const bool low = m < 0.70710678118654752;
+    m              = low ? m + m : m;
+    k              = low ? k - 1 : k;
+    const double f = m - 1.0, d = 2.0 + f;
+    double r       = __builtin_amdgcn_rcp( d );
+    r              = fma( fma( -d, r, 1.0 ), r, r );
+    r              = fma( fma( -d, r, 1.0 ), r, r );
+    const double s = f * r, z = s * s;
+    double p       = 1.0 / 19.0;
+    p              = fma( p, z, 1.0 / 17.0 );
+    p              = fma( p, z, 1.0 / 15.0 );
+    p              = fma( p, z, 1.0 / 13.0 );
+    p              = fma( p, z, 1.0 / 11.0 );
+    p              = fma( p, z, 1.0 / 9.0 );
+    p              = fma( p, z, 1.0 / 7.0 );
+    p              = fma( p, z, 1.0 / 5.0 );
+    p              = fma( p, z, 1.0 / 3.0 );
+    // ln 2 as its nearest double and the rest; t holds k ln 2 + f, w what its roundings left
+    const double kd = (double)k;
+    const double t  = fma( kd, 0.69314718055994531, f );
+    const double w  = fma( kd, 0.69314718055994531, f - t );
+    return t + ( w - fma( s, f - 2.0 * ( p * z ), -kd * 2.3190468138462996e-17 ) );
+}
+// A draw is bound by its arithmetic (two Philox blocks, two logarithms, roots and sines): with
+// log_uniform and the sine of a multiple of pi, whose argument needs no rounded product, the first
+// Depondt stage of 8.2 10^5 thermal spins takes 34.1 us instead of 38.6, and a normal's error falls
+// from 5.6e-16 to 1.8e-16 (root mean square over 2 10^7 draws).
 __device__ __forceinline__ void normal3( uint64_t seed, uint64_t step, uint64_t site, double * z )
 {
     uint32_t k0 = (uint32_t)seed, k1 = (uint32_t)( seed >> 32 );
@@ -162,13 +198,13 @@ __device__ __forceinline__ void normal3( uint64_t seed, uint64_t step, uint64_t 
     double u2 = u53( c0[2], c0[3] );
     double u3 = 1.0 - u53( c1[0], c1[1] );
     double u4 = u53( c1[2], c1[3] );
-    double r1 = sqrt( -2.0 * log( u1 ) );
-    double r2 = sqrt( -2.0 * log( u3 ) );
+    double r1 = sqrt( -2.0 * log_uniform( u1 ) );
+    double r2 = sqrt( -2.0 * log_uniform( u3 ) );
     double sn, cs;
-    sincos( 2.0 * Pi * u2, &sn, &cs ); // one argument reduction for both
+    sincospi( 2.0 * u2, &sn, &cs ); // an exact argument reduction for both
     z[0] = r1 * cs;
     z[1] = r1 * sn;
-    z[2]      = r2 * cos( 2.0 * Pi * u4 );
+    z[2] = r2 * cospi( 2.0 * u4 );
 }
 
 // floor(n / f.d) for 0 <= n < 2^31 (FastDiv)
