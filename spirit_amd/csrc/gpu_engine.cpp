@@ -930,6 +930,12 @@ LLGRunner::LLGRunner( const std::vector<ImageSpec> & images, int solver_ ) : spe
     b_obs.resize( sizeof( double ) * 2 * specs.size() );
     HIPCHECK( hipMemset( b_obs.as<void>(), 0, sizeof( double ) * 2 * specs.size() ) );
     HIPCHECK( hipMemset( b_eff.as<void>(), 0, f3 ) );
+    b_count.resize( sizeof( int ) * FOLD_COUNT_STRIDE * specs.size() );
+    HIPCHECK( hipMemset( b_count.as<void>(), 0, b_count.size() ) );
+    const FoldDev fold_dev = { b_count.as<int>(), b_obs.as<double>(), b_img_stop.as<int>(), b_nstop.as<int>(),
+                               b_stopstep.as<long long>() };
+    b_fold.resize( sizeof( FoldDev ) );
+    HIPCHECK( hipMemcpy( b_fold.as<void>(), &fold_dev, sizeof( FoldDev ), hipMemcpyHostToDevice ) );
     obs_host.assign( 2 * specs.size(), 0.0 );
     b_blk.resize( sizeof( int ) * blk_img_host.size() );
     HIPCHECK( hipMemcpy( b_blk.as<void>(), blk_img_host.data(), sizeof( int ) * blk_img_host.size(),
@@ -1394,6 +1400,7 @@ static StepArgs with_variants( StepArgs A, int stt_gradient, const std::vector<I
     A.few_pairs    = 1;
     for( const auto & I : imgs )
         A.few_pairs = A.few_pairs && few_pairs( I.ham );
+    A.n_images = (int)imgs.size();
     return A;
 }
 
@@ -1472,6 +1479,16 @@ void LLGRunner::tune_stage_tiles()
     upload_images();
 }
 
+bool LLGRunner::folds() const
+{
+    if( min_is_solver( solver ) || stt_gradient_any )
+        return false;
+    for( auto & I : imgs_host )
+        if( I.n_blocks > FOLD_BLOCKS || !few_pairs( I.ham ) )
+            return false;
+    return true;
+}
+
 void LLGRunner::launch_step( const StepArgs & A )
 {
     if( min_is_solver( solver ) )
@@ -1515,8 +1532,11 @@ void LLGRunner::step( bool obs, bool count, bool check, double conv )
         A.noise = b_noise.as<double>() + (size_t)noise_pos * 3 * (size_t)n_total;
         ++noise_pos;
     }
+    const bool fold     = obs && folds();
+    A.fold              = fold ? b_fold.as<FoldDev>() : nullptr;
+    A.check_convergence = check ? 1 : 0;
     launch_step( A );
-    if( obs )
+    if( obs && !fold )
         llg_launch_finalize( A, (int)specs.size(), b_obs.as<double>(), b_img_stop.as<int>(), b_nstop.as<int>(),
                              b_stopstep.as<long long>(), (long long)A.step, conv, check ? 1 : 0, stream );
     if( dev_step )
@@ -1549,8 +1569,11 @@ bool LLGRunner::capture_step_graph( int len, int period, bool check, double conv
         const bool obs = period > 0 && ( k + 1 ) % period == 0;
         A.obs          = obs ? 1 : 0;
         A.step         = (uint64_t)k;
+        const bool fold     = obs && folds();
+        A.fold              = fold ? b_fold.as<FoldDev>() : nullptr;
+        A.check_convergence = check ? 1 : 0;
         launch_step( A );
-        if( obs )
+        if( obs && !fold )
             llg_launch_finalize( A, (int)specs.size(), b_obs.as<double>(), b_img_stop.as<int>(), b_nstop.as<int>(),
                                  b_stopstep.as<long long>(), (long long)k, conv, check ? 1 : 0, stream );
     }

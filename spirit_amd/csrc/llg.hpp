@@ -8,6 +8,17 @@ namespace spirit_hip
 
 constexpr int LLG_THREADS = 256;
 
+// Where an observed step's results go when its last stage reduces the partials (device memory: read only
+// by the blocks that end an image, its pointers would cost every block registers as arguments).
+struct FoldDev
+{
+    int * count; // per image (FOLD_COUNT_STRIDE apart): blocks that have stored their partials
+    double * obs;
+    int * img_stop;
+    int * n_stopped;
+    long long * stop_step;
+};
+
 // Arguments of one stage launch.  Fields are batched SoA buffers; image k's
 // three components start at 3*imgs[k].off.
 struct StepArgs
@@ -35,6 +46,9 @@ struct StepArgs
     uint64_t step;         // global step index (thermal-noise counter); with step_dev, the offset from *step_dev
     const uint64_t * step_dev; // base step index in device memory (graph replays); nullptr: step is absolute
     int obs;               // compute observables (energy, torque, effective field)
+    int n_images;
+    int check_convergence; // with fold: images whose torque is below their limit stop
+    const FoldDev * fold;  // observed steps: the last stage also reduces each image's partials (nullable)
     int few_pairs;         // every image's pair tables are few_pairs
     int stt_gradient;      // some image's STT uses the spin derivative along the current (STT_GRADIENT)
 };
@@ -54,6 +68,10 @@ void llg_launch_energy_sums( const StepArgs & A, const double * x, double * part
 void llg_launch_observe( const StepArgs & A, int solver, int n_blocks, hipStream_t st );
 // out = F - (F.s) s per spin (one image's SoA fields)
 void llg_launch_project_field( const double * F, const double * s, double * out, int nos, hipStream_t st );
+// An image's partials are reduced by its last block of the last stage up to FOLD_BLOCKS blocks an image
+// (fold_finalize has both sides' times), by a kernel of their own (llg_launch_finalize) above.
+constexpr int FOLD_BLOCKS       = 128;
+constexpr int FOLD_COUNT_STRIDE = 32; // ints: a cache line of its own per counter
 // Per-image energy / max torque into obs[2*img], [2*img+1]; with check_convergence an image whose
 // torque is below force_convergence stops (img_stop, stop_step[img]); the run-wide stop flag is set
 // when n_stopped reaches n_images.

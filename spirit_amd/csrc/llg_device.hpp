@@ -841,16 +841,22 @@ __device__ __forceinline__ int stage_block_order( const HamDev & H, int q )
     return ( ( bt << TL ) + bi + H.Nb * c ) * per_row + j;
 }
 
-// block-wide reduction of (sum e, max t) into partials[blk]
-__device__ __forceinline__ void block_reduce_store( double e, double t, double * part_E, double * part_T, int blk )
+// sum e and max t over the wave, in its lane 0
+__device__ __forceinline__ void wave_reduce( double & e, double & t )
 {
-    __shared__ double sE[LLG_THREADS / 64], sT[LLG_THREADS / 64];
 #pragma unroll
     for( int off = 32; off > 0; off >>= 1 )
     {
         e += __shfl_down( e, off, 64 );
         t = fmax( t, __shfl_down( t, off, 64 ) );
     }
+}
+
+// block-wide reduction of (sum e, max t) into partials[blk]
+__device__ __forceinline__ void block_reduce_store( double e, double t, double * part_E, double * part_T, int blk )
+{
+    __shared__ double sE[LLG_THREADS / 64], sT[LLG_THREADS / 64];
+    wave_reduce( e, t );
     const int w = threadIdx.x / 64, lane = threadIdx.x % 64;
     if( lane == 0 )
     {

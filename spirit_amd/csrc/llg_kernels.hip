@@ -20,6 +20,87 @@
 
 namespace spirit_hip
 {
+// An image's energy and torque, and with check_convergence whether it stops (Method_Solver.hpp:232-239),
+// with the index of the step at which it did.  Once every image has stopped, the run-wide flag stops
+// all further stages.
+__device__ __forceinline__ void image_result( const ImageDev & I, int img, int n_images, double E, double T2,
+                                              double * obs, int * stop, int * img_stop, int * n_stopped,
+                                              long long * stop_step, uint64_t step, int check_convergence )
+{
+    const double torque = sqrt( T2 );
+    obs[2 * img]        = E;
+    obs[2 * img + 1]    = torque;
+    if( check_convergence && torque < I.llg.force_convergence )
+    {
+        img_stop[img]  = 1;
+        stop_step[img] = (long long)step;
+        if( atomicAdd( n_stopped, 1 ) + 1 == n_images )
+            *stop = 1;
+    }
+}
+
+// The end of an observed step: the block's sums go to the image's partials, and the first wave of the
+// image's last block to arrive reduces them in k_finalize's order, so that both give the same bits.
+// Partials are stored and read at device scope and a block counts itself only when its stores are
+// performed (pass_tail of the chain kernels has why no cache is written back or invalidated for it);
+// the counter is rearmed by the block that completed it.  A launch of its own for the reduction costs
+// 4.4 us of a 16.3 us step of 64 x 64 spins; here the step takes 14.9 us, of 181 x 181 spins (128 blocks)
+// 16.1 instead of 16.7.  The arrivals take 8 ns each, one after the other: 256 blocks 18.3 instead of
+// 17.4 us, 1024 blocks 31.8 instead of 23.5, hence FOLD_BLOCKS.
+__device__ __forceinline__ void fold_finalize( const StepArgs & A, const ImageDev & I, int img, int blk, double e,
+                                               double t )
+{
+    __shared__ double sE[LLG_THREADS / 64], sT[LLG_THREADS / 64];
+    wave_reduce( e, t );
+    if( threadIdx.x % 64 == 0 )
+    {
+        sE[threadIdx.x / 64] = e;
+        sT[threadIdx.x / 64] = t;
+    }
+    __syncthreads();
+    if( threadIdx.x >= 64 )
+        return;
+    int * count = A.fold->count + FOLD_COUNT_STRIDE * img;
+    int arrived = 0;
+    if( threadIdx.x == 0 )
+    {
+        for( int k = 1; k < LLG_THREADS / 64; ++k )
+        {
+            e += sE[k];
+            t = fmax( t, sT[k] );
+        }
+        __hip_atomic_store( A.part_E + blk, e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
+        __hip_atomic_store( A.part_T + blk, t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
+        __builtin_amdgcn_fence( __ATOMIC_RELEASE, "workgroup" );
+        __builtin_amdgcn_s_waitcnt( 0 ); // the stores are performed
+        arrived = __hip_atomic_fetch_add( count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
+    }
+    if( __builtin_amdgcn_readfirstlane( arrived ) != I.n_blocks - 1 )
+        return;
+    static_assert( FOLD_BLOCKS == 128, "two partials a lane" );
+    double pe[2], pt[2];
+#pragma unroll
+    for( int u = 0; u < 2; ++u )
+    {
+        const int k     = threadIdx.x + 64 * u;
+        const bool in   = k < I.n_blocks;
+        const int at    = I.block_begin + ( in ? k : 0 );
+        const double ve = __hip_atomic_load( A.part_E + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
+        const double vt = __hip_atomic_load( A.part_T + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
+        pe[u]           = in ? ve : 0.0;
+        pt[u]           = in ? vt : 0.0;
+    }
+    e = pe[0] + pe[1];
+    t = fmax( pt[0], pt[1] );
+    wave_reduce( e, t );
+    if( threadIdx.x == 0 )
+    {
+        __hip_atomic_store( count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
+        image_result( I, img, A.n_images, e, t, A.fold->obs, A.stop, A.fold->img_stop, A.fold->n_stopped,
+                      A.fold->stop_step, A.step_dev ? *A.step_dev + A.step : A.step, A.check_convergence );
+    }
+}
+
 // ---------------------------------------------------------------------------
 // the stage kernel
 // ---------------------------------------------------------------------------
@@ -29,19 +110,20 @@ namespace spirit_hip
 template<int SOLVER, int STAGE, bool STT_G, bool FEW>
 __global__ void __launch_bounds__( LLG_THREADS ) k_llg_stage( StepArgs A )
 {
-    if( *A.stop )
-        return;
+    // The stop flags and the image's record are requested together: on a lattice of a few blocks a
+    // stage is a chain of such loads, of about half a microsecond each.
     const int blk           = xcd_contiguous_block();
-    const int img           = A.blk_img[blk];
-    if( A.img_stop[img] )
-        return;
+    const int img           = A.n_images > 1 ? A.blk_img[blk] : 0;
     const ImageDev * __restrict__ I = A.imgs + img;
     const HamDev & H        = I->ham;
+    const int stopped       = *A.stop | A.img_stop[img];
     const int nos           = H.nos;
     const long long base    = 3 * I->off;
     const int i             = stage_block_order( H, blk - I->block_begin ) * LLG_THREADS + threadIdx.x;
     const bool act          = i < nos;
     constexpr bool LAST     = ( SOLVER == SOLVER_RK4 ) ? ( STAGE == 3 ) : ( STAGE == 1 );
+    if( stopped )
+        return;
 
     // input configuration of this force evaluation
     const double * x;
@@ -261,7 +343,14 @@ __global__ void __launch_bounds__( LLG_THREADS ) k_llg_stage( StepArgs A )
         }
     }
     if( LAST && A.obs )
-        block_reduce_store( e_i, t_i, A.part_E, A.part_T, blk );
+    {
+        // (in the kernels of long pair tables and of the spin derivative the reduction costs 6 to 38
+        // registers, in this one none)
+        if( FEW && A.fold )
+            fold_finalize( A, *I, img, blk, e_i, t_i );
+        else
+            block_reduce_store( e_i, t_i, A.part_E, A.part_T, blk );
+    }
 }
 
 // The method constructor's force evaluation and Hook_Post_Iteration (Method_LLG.cpp:22-63,
@@ -422,9 +511,7 @@ void llg_launch_energy_terms( const StepArgs & A, const double * x, double * out
     hipLaunchKernelGGL( k_energy_terms, dim3( n_blocks ), dim3( LLG_THREADS ), 0, st, A, x, out );
 }
 
-// Per-image reduction of the partials (one block per image, fixed order); convergence of
-// each image (Method_Solver.hpp:232-239) with the index of the step at which it converged.
-// Once every image has stopped, the run-wide flag stops all further stages.
+// Per-image reduction of the partials (one block per image, fixed order) and the image's result.
 constexpr int FIN_THREADS = 1024;
 __global__ void __launch_bounds__( FIN_THREADS )
     k_finalize( const ImageDev * __restrict__ imgs, int n_images, const double * __restrict__ part_E,
@@ -475,16 +562,8 @@ __global__ void __launch_bounds__( FIN_THREADS )
     }
     if( threadIdx.x == 0 )
     {
-        const double torque = sqrt( sT[0] );
-        obs[2 * img]        = sE[0];
-        obs[2 * img + 1]    = torque;
-        if( check_convergence && torque < I.llg.force_convergence )
-        {
-            img_stop[img]  = 1;
-            stop_step[img] = step_dev ? (long long)*step_dev + step_index : step_index;
-            if( atomicAdd( n_stopped, 1 ) + 1 == n_images )
-                *stop = 1;
-        }
+        image_result( I, img, n_images, sE[0], sT[0], obs, stop, img_stop, n_stopped, stop_step,
+                      step_dev ? *step_dev + (uint64_t)step_index : (uint64_t)step_index, check_convergence );
     }
 }
 
