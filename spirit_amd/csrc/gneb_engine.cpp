@@ -106,7 +106,6 @@ void GNEBRunner::setup_minimiser()
     zeroed( b_mgrad, fd );
     zeroed( b_mgpr, fd );
     zeroed( b_msd, fd );
-    zeroed( b_mq, fd );
     for( int k = 0; k < MIN_MEMORY; ++k )
     {
         zeroed( b_mda[k], fd );
@@ -125,10 +124,9 @@ void GNEBRunner::setup_minimiser()
     M.v         = b_mv.as<double>();
     M.prev      = b_mprev.as<double>();
     M.f         = nullptr;
-    M.grad      = b_mgrad.as<double>();
-    M.grad_pr   = b_mgpr.as<double>();
+    M.grad[0]   = b_mgrad.as<double>();
+    M.grad[1]   = b_mgpr.as<double>();
     M.sd        = b_msd.as<double>();
-    M.q         = b_mq.as<double>();
     for( int k = 0; k < MIN_MEMORY; ++k )
     {
         M.da[k] = b_mda[k].as<double>();

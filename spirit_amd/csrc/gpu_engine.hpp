@@ -327,7 +327,7 @@ private:
     long noise_steps = 0, noise_pos = 0;
     // direct-minimisation solvers (VP, VP_OSO, LBFGS_OSO, LBFGS_Atlas): state of the run
     void setup_minimiser();
-    DeviceBuffer b_mv, b_mprev, b_mf, b_mgrad, b_mgpr, b_msd, b_mq, b_ma3, b_mpart, b_msc;
+    DeviceBuffer b_mv, b_mprev, b_mf, b_mgrad, b_mgpr, b_msd, b_ma3, b_mpart, b_msc;
     DeviceBuffer b_mda[MIN_MEMORY], b_mdg[MIN_MEMORY];
     MinArgs min_args{};
 };
@@ -441,7 +441,7 @@ private:
         b_stop, b_iter, b_count, b_isum;
     // VP_OSO, LBFGS_OSO, LBFGS_Atlas on the chain's forces F_total
     void setup_minimiser();
-    DeviceBuffer b_mv, b_mprev, b_mgrad, b_mgpr, b_msd, b_mq, b_ma3, b_mpart, b_msc;
+    DeviceBuffer b_mv, b_mprev, b_mgrad, b_mgpr, b_msd, b_ma3, b_mpart, b_msc;
     DeviceBuffer b_mda[MIN_MEMORY], b_mdg[MIN_MEMORY];
     MinArgs min_args{};
 };

@@ -25,9 +25,6 @@ namespace spirit_hip
 enum MinPhase
 {
     PH_VP = 0,  // VP: ratio = (v . g) / (g . g)
-    PH_RHO,     // L-BFGS: rho of the newest pair, first alpha, scale after the first loop; restarts
-    PH_ALPHA,   // L-BFGS first loop: alpha_c = rho_c (da_c . q)
-    PH_COEF,    // L-BFGS second loop: alpha_c - rho_c (dg_c . sd)
     PH_SCALE,   // L-BFGS: step scaling to the maximum move; iteration counter
     PH_FLIP,    // atlas: did a spin leave its chart
     PH_FLIPRHO, // atlas: rho after the chart change
@@ -61,17 +58,11 @@ __device__ __forceinline__ MinSite min_site( int bpi, int dim, int nos )
     return m;
 }
 
-// first loop of the two-loop recursion, k = M-1 .. 0
-__device__ __forceinline__ int lbfgs_c1( int li, int k )
+// the memory slot of the L-BFGS pair that is `age` iterations old
+__device__ __forceinline__ int lbfgs_slot( int li, int age )
 {
-    return ( k + li % MIN_MEMORY + 1 ) % MIN_MEMORY;
+    return ( li + MIN_MEMORY - age ) % MIN_MEMORY;
 }
-// second loop, k = 0 .. M-1
-__device__ __forceinline__ int lbfgs_c2( int li, int k )
-{
-    return li < MIN_MEMORY ? k : ( k + li % MIN_MEMORY + 1 ) % MIN_MEMORY;
-}
-
 // fixed-order block sums of NS values; thread 0 gets the totals in x
 template<int NS>
 __device__ __forceinline__ void min_block_sums( double ( &x )[NS] )
@@ -181,8 +172,7 @@ __device__ __forceinline__ void atlas_rotate( const double * sp, double a3, cons
 }
 
 // ---------------------------------------------------------------------------
-// force evaluation: energy partials, force, solver gradient, velocity (VP) or the newest
-// L-BFGS pair and its dot products.  Chains take their forces from M.F_ext.
+// force evaluation: energy partials, force, solver gradient, velocity (VP).  Chains take their forces from M.F_ext.
 // ---------------------------------------------------------------------------
 template<int SOLVER, bool FEW>
 __global__ void __launch_bounds__( LLG_THREADS ) k_min_force( StepArgs A, MinArgs M, int nos )
@@ -192,8 +182,7 @@ __global__ void __launch_bounds__( LLG_THREADS ) k_min_force( StepArgs A, MinArg
     constexpr int D = SOLVER == SOLVER_LBFGS_ATLAS ? 2 : 3;
     const MinSite t = min_site( M.bpi, D, nos );
     const int i     = t.i;
-    const int li    = M.sc->local_iter;
-    double x[4]     = { 0, 0, 0, 0 }; // solver sums, then the energy
+    double x[3]     = { 0, 0, 0 }; // velocity sums, then the energy
     if( i < nos )
     {
         double F[3];
@@ -204,7 +193,7 @@ __global__ void __launch_bounds__( LLG_THREADS ) k_min_force( StepArgs A, MinArg
             const HamDev & H = A.imgs->ham;
             double g[3], e;
             local_gradient<FEW>( H, A.s, nos, i, ( A.h && H.has_ddi ) ? A.h : nullptr, g, e );
-            x[3] = e;
+            x[2] = e;
             F[0] = -1 * g[0], F[1] = -1 * g[1], F[2] = -1 * g[2];
             store3( M.f, nos, i, F );
         }
@@ -243,44 +232,28 @@ __global__ void __launch_bounds__( LLG_THREADS ) k_min_force( StepArgs A, MinArg
                 atlas_gradient( s, F, M.a3[t.b1 + i], gr );
 #pragma unroll
             for( int d = 0; d < D; ++d )
-                M.grad[t.bd + d * nos + i] = gr[d];
-            if( li > 0 )
-            {
-                const int m = li % MIN_MEMORY;
-#pragma unroll
-                for( int d = 0; d < D; ++d )
-                {
-                    const long long k = t.bd + d * nos + i;
-                    const double a    = M.sd[k];
-                    const double dgv  = gr[d] - M.grad_pr[k];
-                    M.da[m][k]        = a;
-                    M.dg[m][k]        = dgv;
-                    x[0] += dgv * a;
-                    x[1] += dgv * dgv;
-                    x[2] += a * gr[d];
-                }
-            }
+                M.grad[M.sc->cur][t.bd + d * nos + i] = gr[d];
         }
     }
-    min_block_sums<4>( x );
+    min_block_sums<3>( x );
     if( threadIdx.x == 0 )
     {
-        for( int s = 0; s < 3; ++s )
+        for( int s = 0; s < 2; ++s )
             M.part[s * M.n_blocks + blockIdx.x] = x[s];
         if( !M.F_ext )
-            A.part_E[blockIdx.x] = x[3];
+            A.part_E[blockIdx.x] = x[2];
     }
 }
 
 // ---------------------------------------------------------------------------
 // the scalar step between launches (one block)
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__( SC_THREADS ) k_min_scalar( StepArgs A, MinArgs M, int phase, int round, int nos )
+__global__ void __launch_bounds__( SC_THREADS ) k_min_scalar( StepArgs A, MinArgs M, int phase, int nos )
 {
     if( min_stopped( A, M ) )
         return;
     __shared__ double sh[3][SC_THREADS];
-    const int ns = ( phase == PH_RHO || phase == PH_FLIPRHO ) ? 3 : ( phase == PH_VP ? 2 : 1 );
+    const int ns = phase == PH_FLIPRHO ? 3 : ( phase == PH_VP ? 2 : 1 );
     if( phase == PH_SCALE )
     {
         // rms of the search direction of each image (the whole block sums its partials),
@@ -334,51 +307,11 @@ __global__ void __launch_bounds__( SC_THREADS ) k_min_scalar( StepArgs A, MinArg
             S.ratio   = t0 / sh[1][0];
             S.vp_zero = t0 <= 0 ? 1 : 0;
             break;
-        case PH_RHO:
-        {
-            const int m = li % MIN_MEMORY;
-            int gd      = li == 0 ? 1 : 0;
-            if( !gd )
-            {
-                if( t0 > LBFGS_EPS )
-                {
-                    S.rho[m]            = 1.0 / t0;
-                    S.alpha[m]          = S.rho[m] * sh[2][0]; // first loop, k = M-1: c = m, q = grad
-                    const double rhody2 = sh[1][0] * S.rho[m];
-                    S.inv_rhody2        = rhody2 > LBFGS_EPS ? 1.0 / rhody2 : 1.0 / ( LBFGS_EPS );
-                }
-                else
-                {
-                    gd           = 1; // restart: steepest descent with an empty memory
-                    S.local_iter = 0;
-                }
-            }
-            if( gd )
-                for( int k = 0; k < MIN_MEMORY; ++k )
-                    S.rho[k] = 0.0;
-            S.gd = gd;
-            break;
-        }
-        case PH_ALPHA:
-            if( !S.gd )
-            {
-                const int c = lbfgs_c1( li, round );
-                S.alpha[c]  = S.rho[c] * t0;
-            }
-            break;
-        case PH_COEF:
-            if( !S.gd )
-            {
-                const int c   = lbfgs_c2( li, round );
-                double rhopdg = t0;
-                rhopdg *= S.rho[c];
-                S.coef = S.alpha[c] - rhopdg;
-            }
-            break;
         case PH_SCALE:
             // t0: the largest rms over the images
             S.scaling    = t0 > M.maxmove ? M.maxmove / t0 : 1.0;
             S.local_iter = li + 1;
+            S.cur ^= 1; // the gradient becomes the previous one
             break;
         case PH_FLIP: S.flip = t0 > 0 ? 1 : 0; break;
         case PH_FLIPRHO:
@@ -395,108 +328,152 @@ __global__ void __launch_bounds__( SC_THREADS ) k_min_scalar( StepArgs A, MinArg
 }
 
 // ---------------------------------------------------------------------------
-// the two-loop recursion, one kernel per dependent dot product
+// the two-loop recursion
 // ---------------------------------------------------------------------------
-// first loop, k = M-2 .. 0: q -= alpha_{c(k+1)} dg_{c(k+1)}, then da_{c(k)} . q
-template<int D>
-__global__ void __launch_bounds__( LLG_THREADS ) k_lbfgs_loop1( StepArgs A, MinArgs M, int nos, int k )
+// Its six dot products depend on each other through q and sd, vector after vector.  But q and sd are
+// combinations of the gradient and the six memory vectors, so products of those (LbfgsDots) give all
+// of them: one pass over memory for the products, one for the direction, where a kernel for each
+// dependent product read and wrote q or sd six times and a one-block kernel after each added its
+// partials.  256 x 256 x 16 spins (25 MB a vector), bound by memory: products 47 us (4.8 TB/s), scalars
+// 6, direction 36 (5.6 TB/s); with the force 34 and the update 26 an iteration without its dipolar
+// field takes 155 us instead of 229.
+enum LbfgsDots // by age: 0 the newest pair; s = da, y = dg, g the gradient
 {
-    if( min_stopped( A, M ) || M.sc->gd )
-        return;
-    const int li       = M.sc->local_iter;
-    const int cp       = lbfgs_c1( li, k + 1 ), c = lbfgs_c1( li, k );
-    const double ap    = M.sc->alpha[cp];
-    const double * src = k == MIN_MEMORY - 2 ? M.grad : M.q;
-    const MinSite t    = min_site( M.bpi, D, nos );
-    double x[1]        = { 0 };
-    if( t.i < nos )
-    {
-#pragma unroll
-        for( int d = 0; d < D; ++d )
-        {
-            const long long j = t.bd + d * nos + t.i;
-            double qv         = src[j];
-            qv += -ap * M.dg[cp][j];
-            M.q[j] = qv;
-            x[0] += M.da[c][j] * qv;
-        }
-    }
-    min_block_sums<1>( x );
-    if( threadIdx.x == 0 )
-        M.part[blockIdx.x] = x[0];
-}
+    SG0, SG1, SG2, // s . g
+    YG0, YG1, YG2, // y . g
+    YY00, YY01, YY02, YY11, YY12, YY22,
+    SY00, SY10, SY20, SY21, // s_i . y_j, i at least as old as j
+    N_DOTS
+};
+static_assert( N_DOTS <= MIN_SLOTS && MIN_MEMORY == 3, "" );
 
-// end of the first loop and the scale: sd = (q - alpha_{c(0)} dg_{c(0)}) / (rho dy2); dg_{c'(0)} . sd
-template<int D>
-__global__ void __launch_bounds__( LLG_THREADS ) k_lbfgs_mid( StepArgs A, MinArgs M, int nos )
-{
-    if( min_stopped( A, M ) || M.sc->gd )
-        return;
-    const int li     = M.sc->local_iter;
-    const int cp     = lbfgs_c1( li, 0 ), c = lbfgs_c2( li, 0 );
-    const double ap  = M.sc->alpha[cp];
-    const double inv = M.sc->inv_rhody2;
-    const MinSite t  = min_site( M.bpi, D, nos );
-    double x[1]      = { 0 };
-    if( t.i < nos )
-    {
-#pragma unroll
-        for( int d = 0; d < D; ++d )
-        {
-            const long long j = t.bd + d * nos + t.i;
-            double qv         = M.q[j];
-            qv += -ap * M.dg[cp][j];
-            const double sdv = inv * qv;
-            M.sd[j]          = sdv;
-            x[0] += M.dg[c][j] * sdv;
-        }
-    }
-    min_block_sums<1>( x );
-    if( threadIdx.x == 0 )
-        M.part[blockIdx.x] = x[0];
-}
+// blocks of k_lbfgs_dots: four for each compute unit, few enough for one block to add their partials
+constexpr int DOT_BLOCKS = 1024;
 
-// second loop, k = 1 .. M-1: sd += coef_{k-1} da_{c'(k-1)}, then dg_{c'(k)} . sd
-template<int D>
-__global__ void __launch_bounds__( LLG_THREADS ) k_lbfgs_loop2( StepArgs A, MinArgs M, int nos, int k )
-{
-    if( min_stopped( A, M ) || M.sc->gd )
-        return;
-    const int li      = M.sc->local_iter;
-    const int cp      = lbfgs_c2( li, k - 1 ), c = lbfgs_c2( li, k );
-    const double coef = M.sc->coef;
-    const MinSite t   = min_site( M.bpi, D, nos );
-    double x[1]       = { 0 };
-    if( t.i < nos )
-    {
-#pragma unroll
-        for( int d = 0; d < D; ++d )
-        {
-            const long long j = t.bd + d * nos + t.i;
-            double sdv        = M.sd[j];
-            sdv += coef * M.da[cp][j];
-            M.sd[j] = sdv;
-            x[0] += M.dg[c][j] * sdv;
-        }
-    }
-    min_block_sums<1>( x );
-    if( threadIdx.x == 0 )
-        M.part[blockIdx.x] = x[0];
-}
-
-// end of the recursion: sd = -(sd + coef da_{c'(M-1)}), grad_pr = grad; on the steepest-descent
-// branch sd = -grad and the memory is cleared.  |sd|^2 partials for the step scaling.
-template<int D>
-__global__ void __launch_bounds__( LLG_THREADS ) k_lbfgs_final( StepArgs A, MinArgs M, int nos )
+// the newest pair (da: the step taken, dg: the gradient's change) and the products, over all
+// n = images x D x nos elements; each thread a few elements apart by the grid
+__global__ void __launch_bounds__( LLG_THREADS ) k_lbfgs_dots( StepArgs A, MinArgs M, long long n )
 {
     if( min_stopped( A, M ) )
         return;
-    const bool gd     = M.sc->gd;
-    const int li      = M.sc->local_iter;
-    const int cp      = lbfgs_c2( li, MIN_MEMORY - 1 );
-    const double coef = M.sc->coef;
-    const MinSite t   = min_site( M.bpi, D, nos );
-    double x[1]       = { 0 };
+    const int li = M.sc->local_iter;
+    if( li == 0 )
+        return;
+    const int c0 = lbfgs_slot( li, 0 ), c1 = lbfgs_slot( li, 1 ), c2 = lbfgs_slot( li, 2 );
+    const double scaling              = M.sc->scaling;
+    const double * __restrict__ grad  = M.grad[M.sc->cur];
+    const double * __restrict__ prev  = M.grad[M.sc->cur ^ 1];
+    const double * __restrict__ sd    = M.sd;
+    const double * __restrict__ da1   = M.da[c1];
+    const double * __restrict__ da2   = M.da[c2];
+    const double * __restrict__ dg1   = M.dg[c1];
+    const double * __restrict__ dg2   = M.dg[c2];
+    double * __restrict__ da0         = M.da[c0];
+    double * __restrict__ dg0         = M.dg[c0];
+    double x[N_DOTS]                  = {};
+    for( long long j = blockIdx.x * (long long)LLG_THREADS + threadIdx.x; j < n;
+         j += gridDim.x * (long long)LLG_THREADS )
+    {
+        const double g = grad[j], s1 = da1[j], s2 = da2[j], y1 = dg1[j], y2 = dg2[j];
+        const double s0 = sd[j] * scaling, y0 = g - prev[j];
+        da0[j] = s0;
+        dg0[j] = y0;
+        x[SG0] += s0 * g, x[SG1] += s1 * g, x[SG2] += s2 * g;
+        x[YG0] += y0 * g, x[YG1] += y1 * g, x[YG2] += y2 * g;
+        x[YY00] += y0 * y0, x[YY01] += y0 * y1, x[YY02] += y0 * y2;
+        x[YY11] += y1 * y1, x[YY12] += y1 * y2, x[YY22] += y2 * y2;
+        x[SY00] += s0 * y0, x[SY10] += s1 * y0, x[SY20] += s2 * y0, x[SY21] += s2 * y1;
+    }
+    min_block_sums<N_DOTS>( x );
+    if( threadIdx.x == 0 )
+    {
+#pragma unroll
+        for( int s = 0; s < N_DOTS; ++s )
+            M.part[s * gridDim.x + blockIdx.x] = x[s];
+    }
+}
+
+// the recursion's scalars from the products (one block, a wave per product); restarts
+// (lbfgs_get_searchdir, Solver_Kernels.hpp:51-191)
+__global__ void __launch_bounds__( 64 * N_DOTS ) k_lbfgs_scalars( StepArgs A, MinArgs M, int n_part )
+{
+    if( min_stopped( A, M ) )
+        return;
+    __shared__ double x[N_DOTS];
+    const int w = threadIdx.x / 64, lane = threadIdx.x % 64;
+    double t    = 0;
+    for( int k0 = 0; k0 < n_part; k0 += 8 * 64 )
+    {
+        double v[8];
+#pragma unroll
+        for( int u = 0; u < 8; ++u )
+        {
+            const int k = k0 + u * 64 + lane;
+            v[u]        = k < n_part ? M.part[w * n_part + k] : 0.0;
+        }
+#pragma unroll
+        for( int u = 0; u < 8; ++u )
+            t += v[u];
+    }
+#pragma unroll
+    for( int off = 32; off > 0; off >>= 1 )
+        t += __shfl_down( t, off, 64 );
+    if( lane == 0 )
+        x[w] = t;
+    __syncthreads();
+    if( threadIdx.x != 0 )
+        return;
+    MinScalars & S = *M.sc;
+    const int li   = S.local_iter;
+    const int c0 = lbfgs_slot( li, 0 ), c1 = lbfgs_slot( li, 1 ), c2 = lbfgs_slot( li, 2 );
+    int gd       = li == 0 ? 1 : 0;
+    if( !gd && !( x[SY00] > LBFGS_EPS ) )
+    {
+        gd           = 1; // restart: steepest descent with an empty memory
+        S.local_iter = 0;
+    }
+    S.gd = gd;
+    if( gd )
+    {
+        for( int k = 0; k < MIN_MEMORY; ++k )
+            S.rho[k] = 0.0;
+        return;
+    }
+    S.rho[c0]           = 1.0 / x[SY00];
+    const double rhody2 = x[YY00] * S.rho[c0];
+    const double inv    = rhody2 > LBFGS_EPS ? 1.0 / rhody2 : 1.0 / ( LBFGS_EPS );
+    const double r0 = S.rho[c0], r1 = S.rho[c1], r2 = S.rho[c2];
+    // first loop, newest to oldest: alpha_i = rho_i (s_i . q)
+    const double a0 = r0 * x[SG0];
+    const double a1 = r1 * ( x[SG1] - a0 * x[SY10] );
+    const double a2 = r2 * ( x[SG2] - a0 * x[SY20] - a1 * x[SY21] );
+    // second loop, oldest to newest: coef_i = alpha_i - rho_i (y_i . sd)
+    const double k2 = a2 - r2 * ( inv * ( x[YG2] - a0 * x[YY02] - a1 * x[YY12] - a2 * x[YY22] ) );
+    const double k1
+        = a1 - r1 * ( inv * ( x[YG1] - a0 * x[YY01] - a1 * x[YY11] - a2 * x[YY12] ) + k2 * x[SY21] );
+    const double k0 = a0
+                      - r0
+                            * ( inv * ( x[YG0] - a0 * x[YY00] - a1 * x[YY01] - a2 * x[YY02] ) + k2 * x[SY20]
+                                + k1 * x[SY10] );
+    S.inv_rhody2 = inv;
+    S.alpha[c0] = a0, S.alpha[c1] = a1, S.alpha[c2] = a2;
+    S.coef[c0] = k0, S.coef[c1] = k1, S.coef[c2] = k2;
+}
+
+// the direction sd = -( (g - sum alpha y) / (rho y.y) + sum coef s ); on the steepest-descent branch
+// sd = -g and the memory is cleared.  |sd|^2 partials for the step scaling.
+template<int D>
+__global__ void __launch_bounds__( LLG_THREADS ) k_lbfgs_direction( StepArgs A, MinArgs M, int nos )
+{
+    if( min_stopped( A, M ) )
+        return;
+    const MinScalars & S = *M.sc;
+    const bool gd        = S.gd;
+    const int li         = S.local_iter;
+    const int c0 = lbfgs_slot( li, 0 ), c1 = lbfgs_slot( li, 1 ), c2 = lbfgs_slot( li, 2 );
+    const double * grad = M.grad[S.cur];
+    const MinSite t     = min_site( M.bpi, D, nos );
+    double x[1]         = { 0 };
     if( t.i < nos )
     {
         double sq = 0;
@@ -504,11 +481,9 @@ __global__ void __launch_bounds__( LLG_THREADS ) k_lbfgs_final( StepArgs A, MinA
         for( int d = 0; d < D; ++d )
         {
             const long long j = t.bd + d * nos + t.i;
-            const double g    = M.grad[j];
-            double sdv;
+            double sdv        = grad[j];
             if( gd )
             {
-                sdv = -g;
 #pragma unroll
                 for( int n = 0; n < MIN_MEMORY; ++n )
                 {
@@ -518,12 +493,16 @@ __global__ void __launch_bounds__( LLG_THREADS ) k_lbfgs_final( StepArgs A, MinA
             }
             else
             {
-                sdv = M.sd[j];
-                sdv += coef * M.da[cp][j];
-                sdv = -sdv;
+                sdv += -S.alpha[c0] * M.dg[c0][j];
+                sdv += -S.alpha[c1] * M.dg[c1][j];
+                sdv += -S.alpha[c2] * M.dg[c2][j];
+                sdv *= S.inv_rhody2;
+                sdv += S.coef[c2] * M.da[c2][j];
+                sdv += S.coef[c1] * M.da[c1][j];
+                sdv += S.coef[c0] * M.da[c0][j];
             }
-            M.grad_pr[j] = g;
-            M.sd[j]      = sdv;
+            sdv     = -sdv;
+            M.sd[j] = sdv;
             sq += sdv * sdv;
         }
         x[0] = sq;
@@ -583,7 +562,6 @@ __global__ void __launch_bounds__( LLG_THREADS ) k_min_update( StepArgs A, MinAr
 #pragma unroll
             for( int q = 0; q < 3; ++q )
                 sd[q] *= S->scaling;
-            store3( M.sd + t.bd, nos, i, sd );
             oso_rotate( s, sd, sn );
         }
         else
@@ -591,8 +569,6 @@ __global__ void __launch_bounds__( LLG_THREADS ) k_min_update( StepArgs A, MinAr
             double d[2] = { M.sd[t.bd + i], M.sd[t.bd + nos + i] };
             d[0] *= S->scaling;
             d[1] *= S->scaling;
-            M.sd[t.bd + i]       = d[0];
-            M.sd[t.bd + nos + i] = d[1];
             atlas_rotate( s, M.a3[t.b1 + i], d, sn );
         }
         store3( A.s + t.b3, nos, i, sn );
@@ -693,7 +669,7 @@ __global__ void __launch_bounds__( LLG_THREADS ) k_atlas_flip_apply( StepArgs A,
         {
             const long long j = t.bd + d * nos + t.i;
             M.sd[j] *= factor;
-            M.grad_pr[j] *= factor;
+            M.grad[M.sc->cur ^ 1][j] *= factor; // (the iteration's, since its PH_SCALE)
 #pragma unroll
             for( int n = 0; n < MIN_MEMORY; ++n )
             {
@@ -713,9 +689,9 @@ bool min_is_solver( int solver )
            || solver == SOLVER_LBFGS_ATLAS;
 }
 
-static void launch_scalar( const StepArgs & A, const MinArgs & M, int phase, int round, int nos, hipStream_t st )
+static void launch_scalar( const StepArgs & A, const MinArgs & M, int phase, int nos, hipStream_t st )
 {
-    hipLaunchKernelGGL( k_min_scalar, dim3( 1 ), dim3( SC_THREADS ), 0, st, A, M, phase, round, nos );
+    hipLaunchKernelGGL( k_min_scalar, dim3( 1 ), dim3( SC_THREADS ), 0, st, A, M, phase, nos );
 }
 
 template<int SOLVER>
@@ -724,7 +700,7 @@ static void vp_iteration( const StepArgs & A, const MinArgs & M, int nos, hipStr
     const dim3 g( M.n_blocks ), b( LLG_THREADS );
     const auto force = A.few_pairs ? k_min_force<SOLVER, true> : k_min_force<SOLVER, false>;
     hipLaunchKernelGGL( force, g, b, 0, st, A, M, nos );
-    launch_scalar( A, M, PH_VP, 0, nos, st );
+    launch_scalar( A, M, PH_VP, nos, st );
     hipLaunchKernelGGL( k_min_update<SOLVER>, g, b, 0, st, A, M, nos );
 }
 
@@ -735,28 +711,18 @@ static void lbfgs_iteration( const StepArgs & A, const MinArgs & M, int nos, hip
     const dim3 g( M.n_blocks ), b( LLG_THREADS );
     const auto force = A.few_pairs ? k_min_force<SOLVER, true> : k_min_force<SOLVER, false>;
     hipLaunchKernelGGL( force, g, b, 0, st, A, M, nos );
-    launch_scalar( A, M, PH_RHO, 0, nos, st );
-    for( int k = MIN_MEMORY - 2; k >= 0; --k )
-    {
-        hipLaunchKernelGGL( k_lbfgs_loop1<D>, g, b, 0, st, A, M, nos, k );
-        launch_scalar( A, M, PH_ALPHA, k, nos, st );
-    }
-    hipLaunchKernelGGL( k_lbfgs_mid<D>, g, b, 0, st, A, M, nos );
-    launch_scalar( A, M, PH_COEF, 0, nos, st );
-    for( int k = 1; k < MIN_MEMORY; ++k )
-    {
-        hipLaunchKernelGGL( k_lbfgs_loop2<D>, g, b, 0, st, A, M, nos, k );
-        launch_scalar( A, M, PH_COEF, k, nos, st );
-    }
-    hipLaunchKernelGGL( k_lbfgs_final<D>, g, b, 0, st, A, M, nos );
-    launch_scalar( A, M, PH_SCALE, 0, nos, st );
+    const int n_dot = M.n_blocks < DOT_BLOCKS ? M.n_blocks : DOT_BLOCKS;
+    hipLaunchKernelGGL( k_lbfgs_dots, dim3( n_dot ), b, 0, st, A, M, (long long)M.noi * D * nos );
+    hipLaunchKernelGGL( k_lbfgs_scalars, dim3( 1 ), dim3( 64 * N_DOTS ), 0, st, A, M, n_dot );
+    hipLaunchKernelGGL( k_lbfgs_direction<D>, g, b, 0, st, A, M, nos );
+    launch_scalar( A, M, PH_SCALE, nos, st );
     hipLaunchKernelGGL( k_min_update<SOLVER>, g, b, 0, st, A, M, nos );
     if constexpr( SOLVER == SOLVER_LBFGS_ATLAS )
     {
         hipLaunchKernelGGL( k_atlas_check, g, b, 0, st, A, M, nos );
-        launch_scalar( A, M, PH_FLIP, 0, nos, st );
+        launch_scalar( A, M, PH_FLIP, nos, st );
         hipLaunchKernelGGL( k_atlas_flip_sums, g, b, 0, st, A, M, nos );
-        launch_scalar( A, M, PH_FLIPRHO, 0, nos, st );
+        launch_scalar( A, M, PH_FLIPRHO, nos, st );
         hipLaunchKernelGGL( k_atlas_flip_apply, g, b, 0, st, A, M, nos );
     }
 }

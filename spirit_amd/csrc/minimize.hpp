@@ -17,7 +17,7 @@ namespace spirit_hip
 {
 
 constexpr int MIN_MEMORY = 3; // L-BFGS memory (n_lbfgs_memory, Solver_LBFGS_OSO.hpp:15)
-constexpr int MIN_SLOTS  = 4; // partial sums per block of one reduction
+constexpr int MIN_SLOTS  = 16; // partial sums per block of one reduction
 
 // Scalars of a minimisation run, kept in device memory so that an iteration is a fixed
 // sequence of launches (no host round trip; graph-capturable).
@@ -27,10 +27,11 @@ struct MinScalars
     double alpha[MIN_MEMORY];
     double ratio;      // VP: projection / |g|^2
     double inv_rhody2; // L-BFGS: scale of the direction after the first loop
-    double coef;       // L-BFGS second loop: alpha_c - rho_c (dg_c . sd)
+    double coef[MIN_MEMORY]; // L-BFGS second loop: alpha_c - rho_c (dg_c . sd)
     double scaling;    // L-BFGS: scale of the step to the maximum move
     int vp_zero;       // VP: the projection was <= 0 (velocities reset)
     int local_iter;    // L-BFGS iteration counter
+    int cur;           // L-BFGS: which of MinArgs::grad holds this iteration's gradient
     int gd;            // this iteration takes the steepest-descent branch (first or restart)
     int flip;          // atlas: a spin left its chart (s_z a3 < -0.6)
 };
@@ -42,10 +43,8 @@ struct MinArgs
     double * v;       // VP, VP_OSO: velocities
     double * prev;    // VP: force of the previous iteration; VP_OSO: its gradient
     double * f;       // force F = -g of the current iteration
-    double * grad;    // L-BFGS: OSO gradient or atlas residual
-    double * grad_pr; // L-BFGS: gradient of the previous iteration
-    double * sd;      // search direction
-    double * q;       // L-BFGS two-loop vector
+    double * grad[2]; // L-BFGS: OSO gradients or atlas residuals of this iteration and the previous one
+    double * sd;      // search direction, before its scaling
     double * da[MIN_MEMORY];
     double * dg[MIN_MEMORY];
     double * a3;          // atlas: chart of each spin (+1 / -1)
