@@ -137,6 +137,17 @@ struct LLGDev
     const double * temp_site; // per-site temperature of a temperature gradient (nullable: homogeneous)
 };
 
+// Where an observed step's results go when its last stage reduces the partials (in the image record: only
+// the block that ends an image reads it; as kernel arguments it would cost every block registers).
+struct FoldDev
+{
+    int * count; // blocks of the image that have stored their partials
+    double * obs;
+    int * img_stop;
+    int * n_stopped;
+    long long * stop_step;
+};
+
 // One image of a batched launch: where its fields live and how it is parameterised.
 struct ImageDev
 {
@@ -145,6 +156,7 @@ struct ImageDev
     long long off;      // spin offset of this image inside the batched SoA buffers (fields at 3*off)
     int block_begin;    // first block of this image in the launch
     int n_blocks;       // blocks of this image
+    FoldDev fold;
 };
 
 // Division by d for small numerators (mix_div): the rounded reciprocal.

@@ -920,22 +920,19 @@ LLGRunner::LLGRunner( const std::vector<ImageSpec> & images, int solver_ ) : spe
     b_stop.resize( sizeof( int ) );
     b_stopstep.resize( sizeof( long long ) * specs.size() );
     b_img_stop.resize( sizeof( int ) * specs.size() );
-    b_nstop.resize( sizeof( int ) );
+    b_nstop.resize( sizeof( int ) * FOLD_COUNT_STRIDE * ( 1 + specs.size() ) ); // then the images' counters
     b_step.resize( sizeof( uint64_t ) );
     HIPCHECK( hipMemset( b_img_stop.as<void>(), 0, sizeof( int ) * specs.size() ) );
-    HIPCHECK( hipMemset( b_nstop.as<void>(), 0, sizeof( int ) ) );
+    HIPCHECK( hipMemset( b_nstop.as<void>(), 0, b_nstop.size() ) );
     HIPCHECK( hipMemset( b_stop.as<void>(), 0, sizeof( int ) ) );
     img_stopped.assign( specs.size(), 0 );
     steps_last.assign( specs.size(), 0 );
     b_obs.resize( sizeof( double ) * 2 * specs.size() );
     HIPCHECK( hipMemset( b_obs.as<void>(), 0, sizeof( double ) * 2 * specs.size() ) );
     HIPCHECK( hipMemset( b_eff.as<void>(), 0, f3 ) );
-    b_count.resize( sizeof( int ) * FOLD_COUNT_STRIDE * specs.size() );
-    HIPCHECK( hipMemset( b_count.as<void>(), 0, b_count.size() ) );
-    const FoldDev fold_dev = { b_count.as<int>(), b_obs.as<double>(), b_img_stop.as<int>(), b_nstop.as<int>(),
-                               b_stopstep.as<long long>() };
-    b_fold.resize( sizeof( FoldDev ) );
-    HIPCHECK( hipMemcpy( b_fold.as<void>(), &fold_dev, sizeof( FoldDev ), hipMemcpyHostToDevice ) );
+    for( size_t k = 0; k < specs.size(); ++k )
+        imgs_host[k].fold = { b_nstop.as<int>() + FOLD_COUNT_STRIDE * ( 1 + k ), b_obs.as<double>(),
+                              b_img_stop.as<int>(), b_nstop.as<int>(), b_stopstep.as<long long>() };
     obs_host.assign( 2 * specs.size(), 0.0 );
     b_blk.resize( sizeof( int ) * blk_img_host.size() );
     HIPCHECK( hipMemcpy( b_blk.as<void>(), blk_img_host.data(), sizeof( int ) * blk_img_host.size(),
@@ -1531,7 +1528,7 @@ void LLGRunner::step( bool obs, bool count, bool check, double conv )
         ++noise_pos;
     }
     const bool fold     = obs && folds();
-    A.fold              = fold ? b_fold.as<FoldDev>() : nullptr;
+    A.fold              = fold ? 1 : 0;
     A.check_convergence = check ? 1 : 0;
     launch_step( A );
     if( obs && !fold )
@@ -1568,7 +1565,7 @@ bool LLGRunner::capture_step_graph( int len, int period, bool check, double conv
         A.obs          = obs ? 1 : 0;
         A.step         = (uint64_t)k;
         const bool fold     = obs && folds();
-        A.fold              = fold ? b_fold.as<FoldDev>() : nullptr;
+        A.fold              = fold ? 1 : 0;
         A.check_convergence = check ? 1 : 0;
         launch_step( A );
         if( obs && !fold )

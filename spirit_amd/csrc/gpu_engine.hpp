@@ -283,7 +283,6 @@ private:
     void launch_step( const StepArgs & A );
     // an observed step's reduction: in its last stage (every image at most FOLD_BLOCKS blocks) or after it
     bool folds() const;
-    DeviceBuffer b_fold, b_count;
     // Graph of `len` steps reading the step index from b_step; with period > 0 every
     // period-th step is observed (finalize with check / conv), with period 0 none is.
     bool capture_step_graph( int len, int period, bool check, double conv );

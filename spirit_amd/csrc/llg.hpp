@@ -8,17 +8,6 @@ namespace spirit_hip
 
 constexpr int LLG_THREADS = 256;
 
-// Where an observed step's results go when its last stage reduces the partials (device memory: read only
-// by the blocks that end an image, its pointers would cost every block registers as arguments).
-struct FoldDev
-{
-    int * count; // per image (FOLD_COUNT_STRIDE apart): blocks that have stored their partials
-    double * obs;
-    int * img_stop;
-    int * n_stopped;
-    long long * stop_step;
-};
-
 // Arguments of one stage launch.  Fields are batched SoA buffers; image k's
 // three components start at 3*imgs[k].off.
 struct StepArgs
@@ -48,7 +37,7 @@ struct StepArgs
     int obs;               // compute observables (energy, torque, effective field)
     int n_images;
     int check_convergence; // with fold: images whose torque is below their limit stop
-    const FoldDev * fold;  // observed steps: the last stage also reduces each image's partials (nullable)
+    int fold;              // observed steps: the last stage also reduces each image's partials
     int few_pairs;         // every image's pair tables are few_pairs
     int stt_gradient;      // some image's STT uses the spin derivative along the current (STT_GRADIENT)
 };

@@ -60,7 +60,7 @@ __device__ __forceinline__ void fold_finalize( const StepArgs & A, const ImageDe
     __syncthreads();
     if( threadIdx.x >= 64 )
         return;
-    int * count = A.fold->count + FOLD_COUNT_STRIDE * img;
+    int * count = I.fold.count;
     int arrived = 0;
     if( threadIdx.x == 0 )
     {
@@ -96,8 +96,8 @@ __device__ __forceinline__ void fold_finalize( const StepArgs & A, const ImageDe
     if( threadIdx.x == 0 )
     {
         __hip_atomic_store( count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
-        image_result( I, img, A.n_images, e, t, A.fold->obs, A.stop, A.fold->img_stop, A.fold->n_stopped,
-                      A.fold->stop_step, A.step_dev ? *A.step_dev + A.step : A.step, A.check_convergence );
+        image_result( I, img, A.n_images, e, t, I.fold.obs, A.stop, I.fold.img_stop, I.fold.n_stopped,
+                      I.fold.stop_step, A.step_dev ? *A.step_dev + A.step : A.step, A.check_convergence );
     }
 }
 
