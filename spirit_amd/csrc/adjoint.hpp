@@ -38,6 +38,7 @@ struct AdjArgs
     int solver;        // SOLVER_DEPONDT or SOLVER_HEUN
     uint64_t step;     // index of the step (thermal-noise counter)
     double site_n[3];  // axis of the per-site anisotropy K_i
+    int n_J, n_D;      // exchange and DMI parameters (shells)
     // tape of the step
     const double * s;
     const double * F1;

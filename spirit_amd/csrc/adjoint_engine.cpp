@@ -171,6 +171,8 @@ void AdjointRunner::backward( const double * dL_dsN, double * dL_ds0, double * d
     A.L      = run->image_host( 0 ).llg;
     A.nos    = nos;
     A.solver = solver;
+    A.n_J    = n_exch_shells;
+    A.n_D    = n_dmi_sh;
     for( int c = 0; c < 3; ++c )
         A.site_n[c] = ham->site_n[c];
     A.sp     = b_sp.as<double>();
