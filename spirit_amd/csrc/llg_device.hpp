@@ -230,6 +230,16 @@ __device__ __forceinline__ void store3( double * f, int nos, int i, const double
     f[i] = v[0], f[nos + i] = v[1], f[2 * nos + i] = v[2];
 }
 
+// spin i of a configuration: three components apart, or (AOS) a caller's array of spins
+template<bool AOS>
+__device__ __forceinline__ void load_spin( const double * f, int nos, int i, double * v )
+{
+    if constexpr( AOS )
+        v[0] = f[3LL * i], v[1] = f[3LL * i + 1], v[2] = f[3LL * i + 2];
+    else
+        load3( f, nos, i, v );
+}
+
 // ---------------------------------------------------------------------------
 // neighbour index, Vectormath.hpp:437-528 (defects off)
 // ---------------------------------------------------------------------------
@@ -307,6 +317,7 @@ constexpr int LG_MAX_NB = GATHER_PAIRS;
 // The exchange neighbours of spin i (a table of few_pairs), all loads issued before any is used.
 // A pair that does not start at this basis atom or leaves an open boundary reads the spin itself
 // and yields exactly zero (its loaded values are replaced).
+template<bool AOS = false>
 __device__ __forceinline__ void gather_exchange_neighbours( const HamDev & H, const double * __restrict__ x, int nos,
                                                             int i, int ib, int a, int b, int c,
                                                             double ( &se )[LG_MAX_NB][3] )
@@ -317,7 +328,7 @@ __device__ __forceinline__ void gather_exchange_neighbours( const HamDev & H, co
         {
             const PairDev & p = H.exch_g[k];
             const int j       = p.i != ib ? -1 : pair_neighbour_delta( H, i, a, b, c, p );
-            load3( x, nos, j >= 0 ? j : i, se[k] );
+            load_spin<AOS>( x, nos, j >= 0 ? j : i, se[k] );
             if( j < 0 )
                 se[k][0] = se[k][1] = se[k][2] = 0.0;
         }
@@ -362,7 +373,7 @@ struct SiteOffsets
 
 // f( k, spin, weight ) for the n pairs at p of spin i, weight 0 (and the spin itself) for a pair
 // without a neighbour; the loads of a group of LG_MAX_NB pairs are issued before any is used
-template<typename F>
+template<bool AOS, typename F>
 __device__ __forceinline__ void for_pairs( const HamDev & H, const SiteOffsets & off, const PairDev * __restrict__ p,
                                            int n, const double * __restrict__ x, int nos, int i, int ib, F f )
 {
@@ -377,7 +388,7 @@ __device__ __forceinline__ void for_pairs( const HamDev & H, const SiteOffsets &
             const PairDev & q = p[k0 + k < n ? k0 + k : n - 1];
             const int j       = off.neighbour( q, i, ib );
             is[k]             = j >= 0 && k0 + k < n;
-            load3( x, nos, j >= 0 ? j : i, se[k] );
+            load_spin<AOS>( x, nos, j >= 0 ? j : i, se[k] );
         }
 #pragma unroll
         for( int k = 0; k < LG_MAX_NB; ++k )
@@ -393,6 +404,7 @@ __device__ __forceinline__ void for_pairs( const HamDev & H, const SiteOffsets &
 // role's translation, wrapped along periodic axes); the quadruplet counts only if all four of
 // its spins exist from that anchor.  Returns the sum t; the spin's energy share is -t.s/4
 // (E_Quadruplet, :513-557).
+template<bool AOS = false>
 __device__ __forceinline__ void quadruplet_gradient( const HamDev & H, const double * __restrict__ x, int nos, int ib,
                                                      int a, int b, int c, double * t )
 {
@@ -439,10 +451,10 @@ __device__ __forceinline__ void quadruplet_gradient( const HamDev & H, const dou
             if( sj_ < 0 || sk_ < 0 || sl_ < 0 )
                 continue;
             double vi[3], vj[3], vk[3], vl[3];
-            load3( x, nos, si_, vi );
-            load3( x, nos, sj_, vj );
-            load3( x, nos, sk_, vk );
-            load3( x, nos, sl_, vl );
+            load_spin<AOS>( x, nos, si_, vi );
+            load_spin<AOS>( x, nos, sj_, vj );
+            load_spin<AOS>( x, nos, sk_, vk );
+            load_spin<AOS>( x, nos, sl_, vl );
             if( r < 2 )
             {
                 const double kl = dot3( vk, vl );
@@ -465,7 +477,8 @@ __device__ __forceinline__ void quadruplet_gradient( const HamDev & H, const dou
 // (1/2 g.s over aniso+exchange+DMI+DDI, plus the cubic and Zeeman energies).
 // FEW: every image's exchange table fits one group and holds its DMI pairs (few_pairs), the usual
 // nearest-neighbour model; its kernels need no group loops, which cost ten registers.
-template<bool FEW = false>
+// AOS: x is an array of spins.
+template<bool FEW = false, bool AOS = false>
 __device__ __forceinline__ void local_gradient( const HamDev & H, const double * __restrict__ x, int nos, int i,
                                                 const double * __restrict__ hddi, double * g, double & e )
 {
@@ -475,7 +488,8 @@ __device__ __forceinline__ void local_gradient( const HamDev & H, const double *
     const int a    = cell - rest * H.Na;
     const int c    = fast_div( rest, H.div_Nb );
     const int b    = rest - c * H.Nb;
-    const double s[3] = { x[i], x[nos + i], x[2 * nos + i] };
+    double s[3];
+    load_spin<AOS>( x, nos, i, s );
     // Every load this spin needs is issued before the first use: the per-site K_i, the DDI
     // field and the neighbour spins (up to LG_MAX_NB of them gathered into registers), so
     // the memory latencies overlap instead of adding up pair after pair.
@@ -485,7 +499,7 @@ __device__ __forceinline__ void local_gradient( const HamDev & H, const double *
         load3( hddi, nos, i, hd );
     double se[FEW ? LG_MAX_NB : 1][3];
     if constexpr( FEW )
-        gather_exchange_neighbours( H, x, nos, i, ib, a, b, c, se );
+        gather_exchange_neighbours<AOS>( H, x, nos, i, ib, a, b, c, se );
     g[0] = g[1] = g[2] = 0;
     // anisotropy, :785-800
     for( int k = 0; k < H.n_aniso; ++k )
@@ -535,13 +549,13 @@ __device__ __forceinline__ void local_gradient( const HamDev & H, const double *
         const SiteOffsets off( H, a, b, c );
         const PairDev * __restrict__ ex = H.exch;
         const PairDev * __restrict__ dm = H.dmi;
-        for_pairs( H, off, ex, H.n_exch, x, nos, i, ib, [&]( int k, const double * sj, double w ) {
+        for_pairs<AOS>( H, off, ex, H.n_exch, x, nos, i, ib, [&]( int k, const double * sj, double w ) {
             const double J = w * ex[k].J;
 #pragma unroll
             for( int q = 0; q < 3; ++q )
                 g[q] -= J * sj[q];
         } );
-        for_pairs( H, off, dm, H.n_dmi, x, nos, i, ib, [&]( int k, const double * sj, double w ) {
+        for_pairs<AOS>( H, off, dm, H.n_dmi, x, nos, i, ib, [&]( int k, const double * sj, double w ) {
             const double D = w * dm[k].D;
             double cr[3];
             cross3( sj, dm[k].n, cr );
@@ -561,7 +575,7 @@ __device__ __forceinline__ void local_gradient( const HamDev & H, const double *
             if( j < 0 )
                 continue;
             double sj[3], cr[3];
-            load3( x, nos, j, sj );
+            load_spin<AOS>( x, nos, j, sj );
             cross3( sj, p.n, cr );
 #pragma unroll
             for( int q = 0; q < 3; ++q )
@@ -600,7 +614,7 @@ __device__ __forceinline__ void local_gradient( const HamDev & H, const double *
     if( H.quad_in_step )
     {
         double t[3];
-        quadruplet_gradient( H, x, nos, ib, a, b, c, t );
+        quadruplet_gradient<AOS>( H, x, nos, ib, a, b, c, t );
         g[0] -= t[0];
         g[1] -= t[1];
         g[2] -= t[2];

@@ -7,15 +7,18 @@
 // are the caller's device arrays, and everything else the kernels need lives in `scratch`,
 // a file-scope device array of fixed size that each GPU holds until the process ends.
 //
-// Scratch layout (byte offsets): the image record, the pair and quadruplet tables, the
-// block -> image table, the per-block energy and torque partials, the per-site K_i, and the
-// structure-of-arrays spins and gradient the field kernel reads and writes.  Every call
-// rewrites what it reads: nothing has to start at zero.  Calls on one GPU share the array;
+// A call is one kernel for lattices of up to FOLD_BLOCKS blocks of a nearest-neighbour model, two for
+// larger ones: it reads and writes the caller's arrays as they are, its Hamiltonian is a kernel
+// argument, and only tables that do not fit one are copied.
+//
+// Scratch layout (byte offsets): the counter of the blocks that have stored their energy (zero between
+// calls), the pair and quadruplet tables, the per-block energy partials, the per-site K_i, and the
+// gradient where the caller's arrays overlap.  Calls on one GPU share the array;
 // the entry point holds a per-device lock until its stream has finished, so calls through it
 // never overlap on one GPU, but any other user of the array would race with them.
 #include "api_common.hpp"
 #include "gpu_engine.hpp"
-#include "llg.hpp"
+#include "llg_device.hpp"
 
 #include <mutex>
 
@@ -34,15 +37,12 @@ constexpr size_t align256( size_t x )
 {
     return ( x + 255 ) / 256 * 256;
 }
-constexpr size_t OFF_IMAGE  = 0;
-constexpr size_t OFF_PAIRS  = align256( OFF_IMAGE + sizeof( ImageDev ) );
+constexpr size_t OFF_COUNT  = 0;
+constexpr size_t OFF_PAIRS  = align256( OFF_COUNT + sizeof( int ) );
 constexpr size_t OFF_QUADS  = align256( OFF_PAIRS + sizeof( PairDev ) * NA_MAX_PAIR_ENTRIES );
-constexpr size_t OFF_BLKIMG = align256( OFF_QUADS + sizeof( QuadDev ) * NA_MAX_QUADS );
-constexpr size_t OFF_PART_E = align256( OFF_BLKIMG + sizeof( int ) * NA_MAX_BLOCKS );
-constexpr size_t OFF_PART_T = align256( OFF_PART_E + sizeof( double ) * NA_MAX_BLOCKS );
-constexpr size_t OFF_SITE_K = align256( OFF_PART_T + sizeof( double ) * NA_MAX_BLOCKS );
-constexpr size_t OFF_X      = align256( OFF_SITE_K + sizeof( double ) * NA_MAX_SPINS );
-constexpr size_t OFF_G      = align256( OFF_X + sizeof( double ) * 3 * NA_MAX_SPINS );
+constexpr size_t OFF_PART_E = align256( OFF_QUADS + sizeof( QuadDev ) * NA_MAX_QUADS );
+constexpr size_t OFF_SITE_K = align256( OFF_PART_E + sizeof( double ) * NA_MAX_BLOCKS );
+constexpr size_t OFF_G      = align256( OFF_SITE_K + sizeof( double ) * NA_MAX_SPINS );
 constexpr size_t SCRATCH_BYTES = align256( OFF_G + sizeof( double ) * 3 * NA_MAX_SPINS );
 
 } // namespace
@@ -86,46 +86,95 @@ DeviceScratch & scratch_address( int & device )
     return d;
 }
 
-__global__ void k_na_aos_to_soa( const double * __restrict__ aos, double * __restrict__ soa, int nos )
+// E = sum of the n block partials in block order, the order Spirit_HIP_Gradient_and_Energy adds them on
+// the host, so both entry points return the same bits: the block brings them to LDS, thread 0 adds.
+__device__ __forceinline__ void sum_partials( const double * part, int n, double * out )
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if( i < nos )
+    constexpr int CHUNK = 4 * LLG_THREADS;
+    __shared__ double lds[CHUNK];
+    double E = 0;
+    for( int k0 = 0; k0 < n; k0 += CHUNK )
     {
-        soa[i]           = aos[3 * (long long)i];
-        soa[nos + i]     = aos[3 * (long long)i + 1];
-        soa[2 * nos + i] = aos[3 * (long long)i + 2];
+        const int m = n - k0 < CHUNK ? n - k0 : CHUNK;
+        for( int k = threadIdx.x; k < m; k += LLG_THREADS )
+            lds[k] = __hip_atomic_load( part + k0 + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
+        __syncthreads();
+        if( threadIdx.x == 0 )
+        {
+#pragma unroll 8
+            for( int k = 0; k < m; ++k )
+                E += lds[k];
+        }
+        __syncthreads();
     }
-}
-
-__global__ void k_na_soa_to_aos( const double * __restrict__ soa, double * __restrict__ aos, int nos )
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if( i < nos )
-    {
-        aos[3 * (long long)i]     = soa[i];
-        aos[3 * (long long)i + 1] = soa[nos + i];
-        aos[3 * (long long)i + 2] = soa[2 * nos + i];
-    }
-}
-
-__global__ void k_na_fill_int( int * p, int n, int v )
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if( i < n )
-        p[i] = v;
-}
-
-// E = sum of the block partials in block order, the order Spirit_HIP_Gradient_and_Energy adds
-// them on the host, so both entry points return the same bits.
-__global__ void k_na_sum_partials( const double * __restrict__ part, int n, double * __restrict__ out )
-{
-    if( threadIdx.x == 0 && blockIdx.x == 0 )
-    {
-        double E = 0;
-        for( int k = 0; k < n; ++k )
-            E += part[k];
+    if( threadIdx.x == 0 )
         *out = E;
+}
+
+__global__ void __launch_bounds__( LLG_THREADS ) k_na_sum( const double * part, int n, double * out )
+{
+    sum_partials( part, n, out );
+}
+
+__global__ void __launch_bounds__( LLG_THREADS ) k_na_copy( const double * src, double * dst, long long n )
+{
+    const long long i = blockIdx.x * (long long)LLG_THREADS + threadIdx.x;
+    if( i < n )
+        dst[i] = src[i];
+}
+
+// Gradient of the spins x (an array of spins, like the gradient) and every block's energy; with out, the
+// last block to arrive adds the energies (fold_finalize of the stage kernels has the protocol, its cost
+// and the line FOLD_BLOCKS).  A call was bound by its launches and copies, not by this kernel: five
+// kernels and two copies took 37.6 us for 64 x 64 spins, this one 23.5, of which the kernel is 10.
+template<bool FEW>
+__global__ void __launch_bounds__( LLG_THREADS )
+    k_na_gradient( HamDev H, const double * __restrict__ x, double * __restrict__ grad, double * part, int * count,
+                   double * out )
+{
+    const int blk = xcd_contiguous_block();
+    const int i   = blk * LLG_THREADS + threadIdx.x;
+    double e_i    = 0;
+    if( i < H.nos )
+    {
+        double g[3];
+        local_gradient<FEW, true>( H, x, H.nos, i, nullptr, g, e_i );
+#pragma unroll
+        for( int q = 0; q < 3; ++q )
+            grad[3LL * i + q] = g[q];
     }
+    __shared__ double sE[LLG_THREADS / 64];
+    __shared__ int last;
+    double t = 0;
+    wave_reduce( e_i, t );
+    if( threadIdx.x % 64 == 0 )
+        sE[threadIdx.x / 64] = e_i;
+    __syncthreads();
+    if( threadIdx.x == 0 )
+    {
+        for( int k = 1; k < LLG_THREADS / 64; ++k )
+            e_i += sE[k];
+        __hip_atomic_store( part + blk, e_i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
+        last = 0;
+        if( out )
+        {
+            __builtin_amdgcn_fence( __ATOMIC_RELEASE, "workgroup" );
+            __builtin_amdgcn_s_waitcnt( 0 ); // the store is performed
+            last = __hip_atomic_fetch_add( count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT ) == (int)gridDim.x - 1;
+        }
+    }
+    __syncthreads();
+    if( !last )
+        return;
+    if( threadIdx.x == 0 )
+        __hip_atomic_store( count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
+    sum_partials( part, gridDim.x, out );
+}
+
+// whether n doubles at p and m doubles at q have memory in common
+bool overlap( const double * p, long long n, const double * q, long long m )
+{
+    return (uintptr_t)p < (uintptr_t)( q + m ) && (uintptr_t)q < (uintptr_t)( p + n );
 }
 
 void check( hipError_t e, const char * what )
@@ -174,23 +223,21 @@ try
     char * base           = ds.ptr;
     const hipStream_t st  = static_cast<hipStream_t>( stream );
     const int n_blocks    = ( nos + LLG_THREADS - 1 ) / LLG_THREADS;
-    ImageDev * d_img      = reinterpret_cast<ImageDev *>( base + OFF_IMAGE );
+    int * d_count         = reinterpret_cast<int *>( base + OFF_COUNT );
     PairDev * d_pairs     = reinterpret_cast<PairDev *>( base + OFF_PAIRS );
     QuadDev * d_quads     = reinterpret_cast<QuadDev *>( base + OFF_QUADS );
-    int * d_blk_img       = reinterpret_cast<int *>( base + OFF_BLKIMG );
     double * d_part_E     = reinterpret_cast<double *>( base + OFF_PART_E );
-    double * d_part_T     = reinterpret_cast<double *>( base + OFF_PART_T );
     double * d_site_K     = reinterpret_cast<double *>( base + OFF_SITE_K );
-    double * d_x          = reinterpret_cast<double *>( base + OFF_X );
     double * d_g          = reinterpret_cast<double *>( base + OFF_G );
 
-    // the image record and its tables, built on the host stack and copied into the scratch
+    // the Hamiltonian and its tables, built on the host stack; tables that are no part of it are copied
+    // into the scratch
     PairDev pairs[NA_MAX_PAIR_ENTRIES];
     QuadDev quads[NA_MAX_QUADS];
-    ImageDev I{};
-    const int n_pairs = fill_ham_dev( g, h, I.ham, pairs, NA_MAX_PAIR_ENTRIES );
-    I.ham.exch        = d_pairs;
-    I.ham.dmi         = d_pairs + I.ham.n_exch;
+    HamDev H{};
+    const int n_pairs = fill_ham_dev( g, h, H, pairs, NA_MAX_PAIR_ENTRIES );
+    H.exch        = d_pairs;
+    H.dmi         = d_pairs + H.n_exch;
     const int n_quads = (int)h.quads.size();
     for( int k = 0; k < n_quads; ++k )
     {
@@ -210,38 +257,34 @@ try
     }
     if( n_quads > 0 )
     {
-        I.ham.n_quad       = n_quads;
-        I.ham.quad_in_step = h.quadruplets_in_gradient_and_energy() ? 1 : 0;
-        I.ham.quad         = d_quads;
+        H.n_quad       = n_quads;
+        H.quad_in_step = h.quadruplets_in_gradient_and_energy() ? 1 : 0;
+        H.quad         = d_quads;
     }
-    if( I.ham.has_site_K )
-        I.ham.site_K = d_site_K;
-    I.off         = 0;
-    I.block_begin = 0;
-    I.n_blocks    = n_blocks;
+    if( H.has_site_K )
+        H.site_K = d_site_K;
 
-    check( hipMemcpyAsync( d_img, &I, sizeof( ImageDev ), hipMemcpyHostToDevice, st ), "copy of the image record" );
-    if( n_pairs > 0 )
+    const bool few = few_pairs( H );
+    if( n_pairs > 0 && !few )
         check( hipMemcpyAsync( d_pairs, pairs, sizeof( PairDev ) * n_pairs, hipMemcpyHostToDevice, st ),
                "copy of the pair table" );
     if( n_quads > 0 )
         check( hipMemcpyAsync( d_quads, quads, sizeof( QuadDev ) * n_quads, hipMemcpyHostToDevice, st ),
                "copy of the quadruplets" );
-    if( I.ham.has_site_K )
+    if( H.has_site_K )
         check( hipMemcpyAsync( d_site_K, h.site_K.data(), sizeof( double ) * nos, hipMemcpyHostToDevice, st ),
                "copy of the per-site anisotropy" );
-    hipLaunchKernelGGL( k_na_fill_int, dim3( ( n_blocks + 255 ) / 256 ), dim3( 256 ), 0, st, d_blk_img, n_blocks, 0 );
-    hipLaunchKernelGGL( k_na_aos_to_soa, dim3( n_blocks ), dim3( LLG_THREADS ), 0, st, spins, d_x, nos );
-
-    StepArgs A{};
-    A.imgs      = d_img;
-    A.blk_img   = d_blk_img;
-    A.part_E    = d_part_E;
-    A.part_T    = d_part_T;
-    A.few_pairs = few_pairs( I.ham ) ? 1 : 0;
-    llg_launch_gradient( A, d_x, d_g, n_blocks, st );
-    hipLaunchKernelGGL( k_na_soa_to_aos, dim3( n_blocks ), dim3( LLG_THREADS ), 0, st, d_g, gradient, nos );
-    hipLaunchKernelGGL( k_na_sum_partials, dim3( 1 ), dim3( 64 ), 0, st, d_part_E, n_blocks, energy );
+    // arrays that share memory: the gradient is formed beside them and copied, the energy stored last
+    const bool apart = !overlap( spins, 3LL * nos, gradient, 3LL * nos ) && !overlap( spins, 3LL * nos, energy, 1 )
+                       && !overlap( gradient, 3LL * nos, energy, 1 );
+    const bool fold  = apart && n_blocks <= FOLD_BLOCKS;
+    hipLaunchKernelGGL( few ? k_na_gradient<true> : k_na_gradient<false>, dim3( n_blocks ), dim3( LLG_THREADS ), 0, st,
+                        H, spins, apart ? gradient : d_g, d_part_E, d_count, fold ? energy : nullptr );
+    if( !apart )
+        hipLaunchKernelGGL( k_na_copy, dim3( ( 3 * nos + LLG_THREADS - 1 ) / LLG_THREADS ), dim3( LLG_THREADS ), 0, st,
+                            d_g, gradient, 3LL * nos );
+    if( !fold )
+        hipLaunchKernelGGL( k_na_sum, dim3( 1 ), dim3( LLG_THREADS ), 0, st, d_part_E, n_blocks, energy );
     check( hipGetLastError(), "kernel launch" );
     // the host-side tables above are read by the copies: wait for the stream before they go
     check( hipStreamSynchronize( st ), "stream synchronisation" );
