@@ -920,7 +920,7 @@ LLGRunner::LLGRunner( const std::vector<ImageSpec> & images, int solver_ ) : spe
     b_stop.resize( sizeof( int ) );
     b_stopstep.resize( sizeof( long long ) * specs.size() );
     b_img_stop.resize( sizeof( int ) * specs.size() );
-    b_nstop.resize( sizeof( int ) * FOLD_COUNT_STRIDE * ( 1 + specs.size() ) ); // then the images' counters
+    b_nstop.resize( sizeof( int ) * FOLD_COUNT_STRIDE * ( 1 + FOLD_COUNTERS * specs.size() ) ); // then the images' counters
     b_step.resize( sizeof( uint64_t ) );
     HIPCHECK( hipMemset( b_img_stop.as<void>(), 0, sizeof( int ) * specs.size() ) );
     HIPCHECK( hipMemset( b_nstop.as<void>(), 0, b_nstop.size() ) );
@@ -931,7 +931,7 @@ LLGRunner::LLGRunner( const std::vector<ImageSpec> & images, int solver_ ) : spe
     HIPCHECK( hipMemset( b_obs.as<void>(), 0, sizeof( double ) * 2 * specs.size() ) );
     HIPCHECK( hipMemset( b_eff.as<void>(), 0, f3 ) );
     for( size_t k = 0; k < specs.size(); ++k )
-        imgs_host[k].fold = { b_nstop.as<int>() + FOLD_COUNT_STRIDE * ( 1 + k ), b_obs.as<double>(),
+        imgs_host[k].fold = { b_nstop.as<int>() + FOLD_COUNT_STRIDE * ( 1 + FOLD_COUNTERS * k ), b_obs.as<double>(),
                               b_img_stop.as<int>(), b_nstop.as<int>(), b_stopstep.as<long long>() };
     obs_host.assign( 2 * specs.size(), 0.0 );
     b_blk.resize( sizeof( int ) * blk_img_host.size() );

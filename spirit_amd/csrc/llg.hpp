@@ -59,8 +59,10 @@ void llg_launch_observe( const StepArgs & A, int solver, int n_blocks, hipStream
 void llg_launch_project_field( const double * F, const double * s, double * out, int nos, hipStream_t st );
 // An image's partials are reduced by its last block of the last stage up to FOLD_BLOCKS blocks an image
 // (fold_finalize has both sides' times), by a kernel of their own (llg_launch_finalize) above.
-constexpr int FOLD_BLOCKS       = 128;
+constexpr int FOLD_BLOCKS       = 512;
+constexpr int FOLD_GROUP        = 64; // blocks that share a counter, at a time one of the image's
 constexpr int FOLD_COUNT_STRIDE = 32; // ints: a cache line of its own per counter
+constexpr int FOLD_COUNTERS     = 1 + FOLD_BLOCKS / FOLD_GROUP; // of an image: its own and its groups'
 // Per-image energy / max torque into obs[2*img], [2*img+1]; with check_convergence an image whose
 // torque is below force_convergence stops (img_stop, stop_step[img]); the run-wide stop flag is set
 // when n_stopped reaches n_images.

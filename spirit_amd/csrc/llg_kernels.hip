@@ -43,10 +43,11 @@ __device__ __forceinline__ void image_result( const ImageDev & I, int img, int n
 // image's last block to arrive reduces them in k_finalize's order, so that both give the same bits.
 // Partials are stored and read at device scope and a block counts itself only when its stores are
 // performed (pass_tail of the chain kernels has why no cache is written back or invalidated for it);
-// the counter is rearmed by the block that completed it.  A launch of its own for the reduction costs
-// 4.4 us of a 16.3 us step of 64 x 64 spins; here the step takes 14.9 us, of 181 x 181 spins (128 blocks)
-// 16.1 instead of 16.7.  The arrivals take 8 ns each, one after the other: 256 blocks 18.3 instead of
-// 17.4 us, 1024 blocks 31.8 instead of 23.5, hence FOLD_BLOCKS.
+// counters are rearmed by the blocks that completed them.  A launch of its own for the reduction costs
+// 4.4 us of a 16.1 us step of 64 x 64 spins; here the step takes 14.3 us, of 256 x 256 spins (256 blocks)
+// 16.4 instead of 17.0, of 362 x 362 (512) 18.0 instead of 18.7.  Arrivals at one counter take 8 ns each,
+// one after the other (with a counter for all blocks 256 x 256 spins took 18.3 us), hence groups; and
+// every block waits about a microsecond for its store and arrival, which larger lattices don't win back.
 __device__ __forceinline__ void fold_finalize( const StepArgs & A, const ImageDev & I, int img, int blk, double e,
                                                double t )
 {
@@ -60,8 +61,11 @@ __device__ __forceinline__ void fold_finalize( const StepArgs & A, const ImageDe
     __syncthreads();
     if( threadIdx.x >= 64 )
         return;
-    int * count = I.fold.count;
-    int arrived = 0;
+    // counters: the image's, then its groups'
+    const int group    = ( blk - I.block_begin ) / FOLD_GROUP;
+    const int n_groups = ( I.n_blocks + FOLD_GROUP - 1 ) / FOLD_GROUP;
+    int * count        = I.fold.count + FOLD_COUNT_STRIDE * ( 1 + group );
+    int last           = 0;
     if( threadIdx.x == 0 )
     {
         for( int k = 1; k < LLG_THREADS / 64; ++k )
@@ -73,29 +77,54 @@ __device__ __forceinline__ void fold_finalize( const StepArgs & A, const ImageDe
         __hip_atomic_store( A.part_T + blk, t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
         __builtin_amdgcn_fence( __ATOMIC_RELEASE, "workgroup" );
         __builtin_amdgcn_s_waitcnt( 0 ); // the stores are performed
-        arrived = __hip_atomic_fetch_add( count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
+        const int size = group < n_groups - 1 ? FOLD_GROUP : I.n_blocks - group * FOLD_GROUP;
+        last = __hip_atomic_fetch_add( count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT ) == size - 1;
+        if( last )
+        {
+            __hip_atomic_store( count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
+            last = n_groups == 1
+                   || __hip_atomic_fetch_add( I.fold.count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT )
+                          == n_groups - 1;
+        }
     }
-    if( __builtin_amdgcn_readfirstlane( arrived ) != I.n_blocks - 1 )
+    if( !__builtin_amdgcn_readfirstlane( last ) )
         return;
-    static_assert( FOLD_BLOCKS == 128, "two partials a lane" );
-    double pe[2], pt[2];
-#pragma unroll
-    for( int u = 0; u < 2; ++u )
+    auto partial = [&]( const double * part, int k ) {
+        const double v = __hip_atomic_load( part + I.block_begin + ( k < I.n_blocks ? k : 0 ), __ATOMIC_RELAXED,
+                                            __HIP_MEMORY_SCOPE_AGENT );
+        return k < I.n_blocks ? v : 0.0;
+    };
+    if( n_groups == 1 )
     {
-        const int k     = threadIdx.x + 64 * u;
-        const bool in   = k < I.n_blocks;
-        const int at    = I.block_begin + ( in ? k : 0 );
-        const double ve = __hip_atomic_load( A.part_E + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
-        const double vt = __hip_atomic_load( A.part_T + at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
-        pe[u]           = in ? ve : 0.0;
-        pt[u]           = in ? vt : 0.0;
+        e = partial( A.part_E, threadIdx.x );
+        t = partial( A.part_T, threadIdx.x );
     }
-    e = pe[0] + pe[1];
-    t = fmax( pt[0], pt[1] );
+    else
+    {
+        static_assert( FOLD_BLOCKS == 512 && FOLD_GROUP == 64, "eight partials a lane" );
+        double pe[8], pt[8];
+#pragma unroll
+        for( int u = 0; u < 8; ++u )
+        {
+            pe[u] = partial( A.part_E, threadIdx.x + 64 * u );
+            pt[u] = partial( A.part_T, threadIdx.x + 64 * u );
+        }
+#pragma unroll
+        for( int w = 4; w > 0; w >>= 1 )
+#pragma unroll
+            for( int u = 0; u < w; ++u )
+            {
+                pe[u] += pe[u + w];
+                pt[u] = fmax( pt[u], pt[u + w] );
+            }
+        e = pe[0];
+        t = pt[0];
+    }
     wave_reduce( e, t );
     if( threadIdx.x == 0 )
     {
-        __hip_atomic_store( count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
+        if( n_groups > 1 )
+            __hip_atomic_store( I.fold.count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT );
         image_result( I, img, A.n_images, e, t, I.fold.obs, A.stop, I.fold.img_stop, I.fold.n_stopped,
                       I.fold.stop_step, A.step_dev ? *A.step_dev + A.step : A.step, A.check_convergence );
     }

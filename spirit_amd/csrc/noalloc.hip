@@ -7,7 +7,7 @@
 // are the caller's device arrays, and everything else the kernels need lives in `scratch`,
 // a file-scope device array of fixed size that each GPU holds until the process ends.
 //
-// A call is one kernel for lattices of up to FOLD_BLOCKS blocks of a nearest-neighbour model, two for
+// A call is one kernel for lattices of up to NA_FOLD_BLOCKS blocks of a nearest-neighbour model, two for
 // larger ones: it reads and writes the caller's arrays as they are, its Hamiltonian is a kernel
 // argument, and only tables that do not fit one are copied.
 //
@@ -32,6 +32,7 @@ constexpr long long NA_MAX_SPINS  = SPIRIT_HIP_NOALLOC_MAX_SPINS;
 constexpr int NA_MAX_BLOCKS       = (int)( ( NA_MAX_SPINS + LLG_THREADS - 1 ) / LLG_THREADS );
 constexpr int NA_MAX_PAIR_ENTRIES = 2 * MAX_PAIRS; // exchange + DMI
 constexpr int NA_MAX_QUADS        = 512;
+constexpr int NA_FOLD_BLOCKS      = 128; // blocks whose energies the gradient kernel adds itself
 
 constexpr size_t align256( size_t x )
 {
@@ -124,8 +125,8 @@ __global__ void __launch_bounds__( LLG_THREADS ) k_na_copy( const double * src, 
 }
 
 // Gradient of the spins x (an array of spins, like the gradient) and every block's energy; with out, the
-// last block to arrive adds the energies (fold_finalize of the stage kernels has the protocol, its cost
-// and the line FOLD_BLOCKS).  A call was bound by its launches and copies, not by this kernel: five
+// last block to arrive adds the energies (fold_finalize of the stage kernels has the protocol; with one
+// counter 128 blocks take 1 us to arrive, 256 as long as a launch costs).  A call was bound by its launches and copies, not by this kernel: five
 // kernels and two copies took 37.6 us for 64 x 64 spins, this one 23.5, of which the kernel is 10.
 template<bool FEW>
 __global__ void __launch_bounds__( LLG_THREADS )
@@ -277,7 +278,7 @@ try
     // arrays that share memory: the gradient is formed beside them and copied, the energy stored last
     const bool apart = !overlap( spins, 3LL * nos, gradient, 3LL * nos ) && !overlap( spins, 3LL * nos, energy, 1 )
                        && !overlap( gradient, 3LL * nos, energy, 1 );
-    const bool fold  = apart && n_blocks <= FOLD_BLOCKS;
+    const bool fold  = apart && n_blocks <= NA_FOLD_BLOCKS;
     hipLaunchKernelGGL( few ? k_na_gradient<true> : k_na_gradient<false>, dim3( n_blocks ), dim3( LLG_THREADS ), 0, st,
                         H, spins, apart ? gradient : d_g, d_part_E, d_count, fold ? energy : nullptr );
     if( !apart )

@@ -1,9 +1,10 @@
 """An observed step's energy and torque, reduced by the last block of its last stage (lattices of up to
-128 blocks of 256 spins) or by a kernel of its own (larger ones, and batches that hold one): lattices of
-1, 2, 64, 65, 127, 128 and 129 blocks, full and with one spin in the last, alone and in a batch with a
-larger one.  Both reductions add in the same order: spins, energies and torques are equal, and the
-oracle's to 1e-9 (30 steps); the interface hands out energy and torque in single precision, which adds
-at most 6e-8 of them to 1e-11 of the sum's up to 10 meV a spin and to 1e-9."""
+512 blocks of 256 spins, which arrive in groups of 64) or by a kernel of its own (larger ones, and batches
+that hold one): lattices of 1, 2, 64, 65, 128, 129, 512 and 513 blocks, full and with few spins in the
+last, alone and in batches with and without a larger one.  Both reductions add in the same order:
+spins, energies and torques are equal, and the oracle's to 1e-9 (30 steps); the interface hands out
+energy and torque in single precision, which adds at most 6e-8 of them to 1e-11 of the sum's up to
+10 meV a spin and to 1e-9."""
 import numpy as np
 import pytest
 
@@ -11,7 +12,8 @@ from test_gpu_batch import replica_cfg, spins, states  # noqa: F401  (fixture)
 
 pytestmark = pytest.mark.gpu
 
-CELLS = [[5, 3, 1], [16, 16, 1], [257, 1, 1], [128, 128, 1], [127, 129, 1], [256, 127, 1], [256, 128, 1], [331, 99, 1]]
+CELLS = [[5, 3, 1], [16, 16, 1], [257, 1, 1], [128, 128, 1], [127, 130, 1], [256, 128, 1], [331, 99, 1],
+         [256, 512, 1], [257, 511, 1]]
 
 
 def replica(k, cells, T):
@@ -25,7 +27,7 @@ def test_reductions(states, oracle, solver, T):  # noqa: F811
     print("CASE fold", solver, T, flush=True)
     cfgs = [replica(k, c, T) for k, c in enumerate(CELLS)]
     lone, lone2, bat = states(cfgs), states(cfgs), states(cfgs)
-    small = [p for p, c in zip(lone2, CELLS) if c[0] * c[1] <= 128 * 256]
+    small = [p for p, c in zip(lone2, CELLS) if c[0] * c[1] <= 512 * 256]
     for p in lone:
         simulation.start(p, simulation.METHOD_LLG, solver, n_iterations=30)
     hip.llg_start_batch(bat, solver, n_iterations=30)
