@@ -271,17 +271,20 @@ __global__ void __launch_bounds__( GNEB_THREADS ) k_gneb_pass( GnebArgs A )
         double v[2] = { 0, 0 };
         if( act )
         {
-            const ImageDev & I = A.imgs[img];
+            // the distance's loads go out before the field's: on images of a few thousand spins the pass is a
+            // chain of loads (21 images of 6944 spins: 16.8 instead of 18.1 us; of 16384: within 1%)
+            double a[3], b[3];
+            load3( A.x + base, nos, i, a );
+            if( img > 0 )
+                load3( A.x + base - n3, nos, i, b );
+            const HamDev & __restrict__ H = A.imgs[img].ham;
             double g[3], e;
-            local_gradient<FEW>( I.ham, A.x + base, nos, i, ( A.h && I.ham.has_ddi ) ? A.h + base : nullptr, g, e );
+            local_gradient<FEW>( H, A.x + base, nos, i, ( A.h && H.has_ddi ) ? A.h + base : nullptr, g, e );
             v[0] = e;
             double ef[3] = { -1 * g[0], -1 * g[1], -1 * g[2] };
             store3( A.eff + base, nos, i, ef );
             if( img > 0 )
             {
-                double a[3], b[3];
-                load3( A.x + base, nos, i, a );
-                load3( A.x + base - n3, nos, i, b );
                 const double t = angle3( a, b );
                 v[1]           = t * t;
             }
