@@ -49,8 +49,8 @@ SPIRIT_API int Spirit_HIP_Gradient_and_Energy( State * state, double * gradient,
  * gradient and energy as Spirit_HIP_Gradient_and_Energy, of spins the caller already holds
  * on the current device.  spins and gradient are device arrays of 3*nos doubles (AoS, as
  * System_Get_Spin_Directions), energy a device array of one double; stream is a hipStream_t
- * (NULL: the default stream).  The call allocates nothing: its tables, partial sums and
- * structure-of-arrays copies live in a fixed device array of the library (about 57 MiB per
+ * (NULL: the default stream).  The call allocates nothing: its tables and partial sums (and
+ * the gradient of arrays that share memory) live in a fixed device array of the library (about 32 MiB per
  * GPU, held until the process ends), shared by every call on that GPU.  Limits: at most
  * SPIRIT_HIP_NOALLOC_MAX_SPINS spins, 128 exchange + DMI pairs, 512 quadruplets and no
  * dipolar interactions (ddi_method none); beyond them it logs an error and returns 1 without
