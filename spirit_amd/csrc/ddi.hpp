@@ -10,11 +10,11 @@ namespace spirit_hip
 {
 
 // The mixed-radix plans of the three lengths (host memory; the plans' tables are device memory)
-// and their radices, from which the launches take their tile shapes.
+// and their shapes, from which the launches take their tiles.
 struct DdiMixHost
 {
     MixPlan plan[3]; // a, b, c
-    int radix[3][MAX_MIX_STAGES];
+    MixLen len[3];
 };
 
 struct DdiDev

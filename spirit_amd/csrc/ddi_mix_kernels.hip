@@ -16,11 +16,11 @@
 #include "ddi_device.hpp"
 #include "fft_mix.hpp"
 
-#include <algorithm>
-#include <cmath>
-
 namespace spirit_hip
 {
+
+// Passes A, A^-1, B and B^-1 derive their addresses from the thread's line once: their tiles have a
+// thread for every line (T.nc == T.nl, mix_line_tile).
 
 // Pass A: row pairs (b0 = 2 bp, b0 + 1) of one component and plane, zero-padded.
 template<bool WIDE>
@@ -200,94 +200,41 @@ __global__ void __launch_bounds__( 1024 )
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
-// LDS of a tile of nl lines (row stride lsr) and the twiddles behind it
-static size_t mix_lds( const MixPlan & P, int lsr )
-{
-    return sizeof( double2 ) * ( (size_t)P.n * (size_t)lsr + (size_t)P.n_tw );
-}
-
-// The tile of nl lines and the threads a line gets: at least what the in-place stages' registers
-// need (mix_per), and of the counts up to a quarter of the line the one with the fewest idle lanes
-// over the stages and wavefronts, weighed against the waves a CU then holds (sixteen at the
-// kernels' registers).  All lines at once, or the largest divisor of nl whose threads fit a block.
-static MixTile mix_tile( const DdiDev & d, int axis, int nl, int lsr )
-{
-    const MixPlan & P = d.mix->plan[axis];
-    const int * rad   = d.mix->radix[axis];
-    const int blocks  = std::max( 1, (int)( (size_t)d.lds_max / mix_lds( P, lsr ) ) );
-    int lo            = 1;
-    for( int s = 0; s < P.ns; ++s )
-        lo = std::max( lo, ( P.n / rad[s] + mix_per( rad[s] ) - 1 ) / mix_per( rad[s] ) );
-    MixTile best{ nl, lsr, 1, lo };
-    double best_score = -1;
-    for( int m = lo; m <= std::max( lo, ( P.n + 3 ) / 4 ); ++m )
-    {
-        int nc = nl;
-        while( nc > 1 && ( nc * m > 1024 || nl % nc != 0 ) )
-            --nc;
-        double rounds = 0;
-        for( int s = 0; s < P.ns; ++s )
-            rounds += ( P.n / rad[s] + m - 1 ) / m * rad[s];
-        const int waves    = ( nc * m + 63 ) / 64;
-        const double use   = (double)P.n * P.ns / ( rounds * m ) * ( nc * m ) / ( 64.0 * waves );
-        const double score = use * std::sqrt( std::min( 1.0, blocks * waves / 16.0 ) );
-        if( nc * m <= 1024 && score > best_score + 1e-9 )
-            best_score = score, best.nc = nc, best.m = m;
-    }
-    return best;
-}
-
 static bool mix_wide( const DdiDev & d, int axis )
 {
-    return d.mix->radix[axis][0] > 10; // the largest radix is the first
+    return d.mix->len[axis].radix[0] > 10; // the largest radix is the first
 }
 
-// Lines of a tile (a power of two).  A row piece of a column tile is 16 cw bytes, so tiles of the
-// column passes are 16 wide where two blocks then fit a CU's LDS, else 8, and narrower only where
-// LDS forces it or fewer than 192 blocks would leave CUs idle (not below 4, 64 bytes): 14 us a
-// pass against 18 and 22 at 16, 8, 4 columns of 300 points, 13 against 16 and 22 at 8, 4, 2 of
-// 1000.  Row pairs (pass A) are contiguous whatever cw is: 4, fewer where that fills the chip.
-static int mix_lines( const DdiDev & d, const MixPlan & P, int arrays, long long n_cols, int want, int least )
+static MixTile mix_a_tile( const DdiDev & d )
 {
-    auto lds = [&]( int cw ) { return mix_lds( P, arrays * cw ); };
-    int cw   = want;
-    while( cw > 1
-           && ( lds( cw ) > (size_t)d.lds_max / ( cw > 8 ? 2 : 1 )
-                || ( cw > least && ( n_cols + cw - 1 ) / cw < 192 ) ) )
-        cw /= 2;
-    return cw;
+    return mix_row_tile( d.mix->len[0], 3LL * d.nb * ( ( d.Nb + 1 ) / 2 ) * d.Nc, d.lds_max );
 }
 
-static int mix_a_lines( const DdiDev & d )
+static MixTile mix_b_tile( const DdiDev & d )
 {
-    return mix_lines( d, d.mix->plan[0], 1, 3LL * d.nb * ( ( d.Nb + 1 ) / 2 ) * d.Nc, 4, 1 );
-}
-
-static int mix_b_cols( const DdiDev & d )
-{
-    return mix_lines( d, d.mix->plan[1], 1, (long long)d.Ha * d.Nc * 3 * d.nb, 16, 4 );
+    return mix_column_tile( d.mix->len[1], (long long)d.Ha * d.Nc * 3 * d.nb, d.lds_max );
 }
 
 bool mix_a_ok( const DdiDev & d )
 {
-    return mix_lds( d.mix->plan[0], mix_a_lines( d ) ) <= (size_t)d.lds_max;
+    return mix_a_tile( d ).nl > 0;
 }
 
 bool mix_b_ok( const DdiDev & d )
 {
-    return mix_lds( d.mix->plan[1], mix_b_cols( d ) ) <= (size_t)d.lds_max;
+    return mix_b_tile( d ).nl > 0;
 }
 
 // Columns and LDS row stride of the convolution pass.  Along b a block holds all arrays of its
 // columns and there are only Ha / cw blocks, so its tiles narrow down to one column.
 static int mix_conv_cols( const DdiDev & d, bool along_b, int & lsr )
 {
-    const MixPlan & P = d.mix->plan[along_b ? 1 : 2];
-    const int cw      = along_b ? mix_lines( d, P, 3 * d.nb, d.Ha, 16, 1 )
-                                : mix_lines( d, P, 3 * d.nb, (long long)d.Ha * d.Pb, 16, 4 );
+    const MixLen & L = d.mix->len[along_b ? 1 : 2];
+    const int cw     = along_b ? mix_lines( L, 3 * d.nb, d.Ha, 16, 1, d.lds_max )
+                               : mix_lines( L, 3 * d.nb, (long long)d.Ha * d.Pb, 16, 4, d.lds_max );
     // an odd row stride spreads the spectrum product's column accesses over the banks
     lsr = ( 3 * d.nb * cw ) | 1;
-    if( mix_lds( P, lsr ) > (size_t)d.lds_max )
+    if( mix_lds( L, lsr ) > (size_t)d.lds_max )
         lsr = 3 * d.nb * cw;
     return cw;
 }
@@ -296,41 +243,37 @@ bool mix_conv_ok( const DdiDev & d, bool along_b )
 {
     int lsr;
     (void)mix_conv_cols( d, along_b, lsr );
-    return mix_lds( d.mix->plan[along_b ? 1 : 2], lsr ) <= (size_t)d.lds_max;
+    return mix_lds( d.mix->len[along_b ? 1 : 2], lsr ) <= (size_t)d.lds_max;
 }
 
 void mix_launch_a_fwd( const DdiDev & d, const double * s, int nos, hipStream_t st )
 {
-    const int cw          = mix_a_lines( d );
-    const MixTile T       = mix_tile( d, 0, cw, cw );
+    const MixTile T       = mix_a_tile( d );
     const long long lines = 3LL * d.nb * ( ( d.Nb + 1 ) / 2 ) * d.Nc;
     const auto k          = mix_wide( d, 0 ) ? k_mix_a_fwd<true> : k_mix_a_fwd<false>;
-    hipLaunchKernelGGL( k, dim3( (unsigned)( ( lines + cw - 1 ) / cw ) ), dim3( T.nc * T.m ),
-                        mix_lds( d.mix->plan[0], cw ), st, d, d.mix->plan[0], T, s, nos );
+    hipLaunchKernelGGL( k, dim3( (unsigned)( ( lines + T.nl - 1 ) / T.nl ) ), dim3( T.nc * T.m ),
+                        mix_lds( d.mix->len[0], T.lsr ), st, d, d.mix->plan[0], T, s, nos );
 }
 
 void mix_launch_a_inv( const DdiDev & d, double * h, int nos, hipStream_t st )
 {
-    const int cw          = mix_a_lines( d );
-    const MixTile T       = mix_tile( d, 0, cw, cw );
+    const MixTile T       = mix_a_tile( d );
     const long long lines = 3LL * d.nb * ( ( d.Nb + 1 ) / 2 ) * d.Nc;
     const auto k          = mix_wide( d, 0 ) ? k_mix_a_inv<true> : k_mix_a_inv<false>;
-    hipLaunchKernelGGL( k, dim3( (unsigned)( ( lines + cw - 1 ) / cw ) ), dim3( T.nc * T.m ),
-                        mix_lds( d.mix->plan[0], cw ), st, d, d.mix->plan[0], T, h, nos );
+    hipLaunchKernelGGL( k, dim3( (unsigned)( ( lines + T.nl - 1 ) / T.nl ) ), dim3( T.nc * T.m ),
+                        mix_lds( d.mix->len[0], T.lsr ), st, d, d.mix->plan[0], T, h, nos );
 }
 
 void mix_launch_b( const DdiDev & d, bool inverse, hipStream_t st )
 {
-    const int cw    = mix_b_cols( d );
-    const MixTile T = mix_tile( d, 1, cw, cw );
-    const int tiles = ( d.Ha + cw - 1 ) / cw;
+    const MixTile T = mix_b_tile( d );
+    const int tiles = ( d.Ha + T.nl - 1 ) / T.nl;
     const dim3 g( (unsigned)( (long long)tiles * d.Nc * 3 * d.nb ) ), b( T.nc * T.m );
-    const size_t lds = mix_lds( d.mix->plan[1], cw );
-    const bool w     = mix_wide( d, 1 );
-    const auto k     = inverse ? ( w ? k_mix_b<true, true> : k_mix_b<true, false> )
-                               : ( w ? k_mix_b<false, true> : k_mix_b<false, false> );
-    hipLaunchKernelGGL( k, g, b, lds, st, d, d.mix->plan[1], T, d.X, tiles, inverse ? d.Pb : d.Nb,
-                        inverse ? d.Nb : d.Pb );
+    const bool w = mix_wide( d, 1 );
+    const auto k = inverse ? ( w ? k_mix_b<true, true> : k_mix_b<true, false> )
+                           : ( w ? k_mix_b<false, true> : k_mix_b<false, false> );
+    hipLaunchKernelGGL( k, g, b, mix_lds( d.mix->len[1], T.lsr ), st, d, d.mix->plan[1], T, d.X, tiles,
+                        inverse ? d.Pb : d.Nb, inverse ? d.Nb : d.Pb );
 }
 
 void mix_launch_conv( const DdiDev & d, bool along_b, hipStream_t st )
@@ -339,8 +282,9 @@ void mix_launch_conv( const DdiDev & d, bool along_b, hipStream_t st )
     const int axis    = along_b ? 1 : 2;
     const int cw      = mix_conv_cols( d, along_b, lsr );
     const MixPlan & P = d.mix->plan[axis];
+    const MixLen & L  = d.mix->len[axis];
     const int tiles   = ( d.Ha + cw - 1 ) / cw;
-    const MixTile T   = mix_tile( d, axis, 3 * d.nb * cw, lsr );
+    const MixTile T   = mix_tile( L, 3 * d.nb * cw, lsr, false, d.lds_max );
     const MixDiv by_cw{ 1.0f / (float)cw }, by_n{ 1.0f / (float)P.n };
     const bool w = mix_wide( d, axis ), one = d.nb == 1;
     const auto k = along_b ? ( w     ? k_mix_conv<true, true, false>
@@ -350,7 +294,7 @@ void mix_launch_conv( const DdiDev & d, bool along_b, hipStream_t st )
                                : one ? k_mix_conv<false, false, true>
                                      : k_mix_conv<false, false, false> );
     hipLaunchKernelGGL( k, dim3( (unsigned)( (long long)tiles * ( along_b ? 1 : d.Pb ) ) ), dim3( T.nc * T.m ),
-                        mix_lds( P, lsr ), st, d, P, T, d.X, cw, by_cw, by_n, tiles, !along_b && d.sym_b ? 1 : 0 );
+                        mix_lds( L, lsr ), st, d, P, T, d.X, cw, by_cw, by_n, tiles, !along_b && d.sym_b ? 1 : 0 );
 }
 
 } // namespace spirit_hip

@@ -4,6 +4,8 @@
 // (the reference's index convention, core/src/data/Geometry.cpp:150-157).
 #pragma once
 
+#include "mix_tiles.hpp"
+
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -178,19 +180,6 @@ struct MixPlan
     int n, ns, n_tw;
     const MixStage * st; // ns stages, device memory
     const double2 * tw;  // n_tw stage twiddles, device memory
-};
-constexpr int MAX_MIX_STAGES = 5; // enough for every length to 4096 with prime factors to 13
-
-// most butterflies of radix R a thread holds in an in-place stage
-constexpr int mix_per( int R )
-{
-    return R >= 8 ? 1 : ( 10 + R - 1 ) / R;
-}
-
-// A tile of lines (MixBlock): nl lines in groups of nc, LDS row stride lsr, m threads a line.
-struct MixTile
-{
-    int nl, lsr, nc, m;
 };
 
 // One FFT length: Stockham stage radices and the n-th roots of unity exp(-2 pi i e / n).

@@ -3,7 +3,6 @@
 
 #include <algorithm>
 #include <chrono>
-#include <functional>
 #include <map>
 #include <mutex>
 #include <cmath>
@@ -117,59 +116,16 @@ void FftLenHost::build( int n )
     }
 }
 
-// The radices of the mixed-radix plan of n (at most 10, or 13 with a factor 11 or 13): as few stages
-// as possible, then the smallest largest radix (registers), then the smallest sum; the largest
-// first, where half of a zero-padded line's inputs need no load.
-static std::vector<int> mix_radices( int n )
-{
-    std::vector<int> best, now;
-    auto better = [&]( const std::vector<int> & a ) {
-        if( best.empty() )
-            return true;
-        if( a.size() != best.size() )
-            return a.size() < best.size();
-        if( a[0] != best[0] )
-            return a[0] < best[0];
-        int sa = 0, sb = 0;
-        for( size_t k = 0; k < a.size(); ++k )
-            sa += a[k], sb += best[k];
-        return sa < sb;
-    };
-    // radices in descending order
-    std::function<void( int, int )> search = [&]( int m, int top ) {
-        if( m == 1 )
-        {
-            if( better( now ) )
-                best = now;
-            return;
-        }
-        if( now.size() == MAX_MIX_STAGES )
-            return;
-        for( int r = std::min( top, m ); r >= 2; --r )
-            if( m % r == 0 )
-            {
-                now.push_back( r );
-                search( m / r, r );
-                now.pop_back();
-            }
-    };
-    if( n == 1 )
-        return { 1 };
-    search( n, n % 11 == 0 || n % 13 == 0 ? 13 : 10 );
-    if( best.empty() )
-        throw std::runtime_error( "DDI FFT: no mixed-radix plan for length " + std::to_string( n ) );
-    return best;
-}
-
 void FftLenHost::build_mix( const std::vector<double2> & w )
 {
-    const int n                = dev.n;
-    const std::vector<int> rad = mix_radices( n );
+    const int n = dev.n;
+    mix_len     = mix_length( n );
     std::vector<MixStage> st;
     std::vector<double2> t;
     int Ns = 1;
-    for( int R : rad )
+    for( int s = 0; s < mix_len.ns; ++s )
     {
+        const int R = mix_len.radix[s];
         MixStage S{};
         S.R     = R;
         S.Ns    = Ns;
@@ -180,11 +136,12 @@ void FftLenHost::build_mix( const std::vector<double2> & w )
             for( int r = 1; r < R; ++r )
                 for( int jm = 0; jm < Ns; ++jm )
                     t.push_back( w[( (long long)r * jm * ( n / ( Ns * R ) ) ) % n] );
-        mix_radix[st.size()] = R;
         st.push_back( S );
         Ns *= R;
     }
     mix.n_tw = (int)t.size();
+    if( mix.n_tw != mix_len.n_tw )
+        throw std::runtime_error( "DDI FFT: twiddle table layout" );
     if( t.empty() )
         t.push_back( make_double2( 1.0, 0.0 ) );
     mix_st.resize( sizeof( MixStage ) * st.size() );
@@ -336,7 +293,7 @@ void DdiPlan::build( const Geometry & g, const Hamiltonian & h, hipStream_t st )
     for( int k = 0; k < 3; ++k )
     {
         mix.plan[k] = len[k]->mix;
-        std::copy( len[k]->mix_radix, len[k]->mix_radix + MAX_MIX_STAGES, mix.radix[k] );
+        mix.len[k]  = len[k]->mix_len;
     }
     d.mix = &mix;
     // inter_sublattice_lookup, Hamiltonian_Heisenberg.cpp:1415-1428 and 1545-1554

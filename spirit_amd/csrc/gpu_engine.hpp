@@ -62,7 +62,7 @@ struct FftLenHost
 {
     FftLen dev{};
     MixPlan mix{};
-    int mix_radix[MAX_MIX_STAGES] = {};
+    MixLen mix_len{};
     DeviceBuffer W, TW2, mix_st, mix_tw;
     void build( int n );
 

@@ -1,0 +1,168 @@
+// Shapes of the mixed-radix transforms (fft_mix.hpp): the radices of a length, and the tile of lines
+// a block transforms with the threads a line gets.  Plain C++, for the host.
+#pragma once
+
+#include <algorithm>
+#include <cmath>
+#include <cstddef>
+#include <functional>
+#include <stdexcept>
+#include <string>
+#include <vector>
+
+namespace spirit_hip
+{
+
+constexpr int MAX_MIX_STAGES  = 5;    // enough for every length to 4096 with prime factors to 13
+constexpr int MIX_MAX_THREADS = 1024; // of a block
+
+// most butterflies of radix R a thread holds in an in-place stage
+constexpr int mix_per( int R )
+{
+    return R >= 8 ? 1 : ( 10 + R - 1 ) / R;
+}
+
+// A tile of lines (MixBlock): nl lines in groups of nc, LDS row stride lsr, m threads a line.
+struct MixTile
+{
+    int nl, lsr, nc, m;
+};
+
+// A length: its ns radices, the largest first, and the entries of its stage-twiddle table.
+struct MixLen
+{
+    int n, ns, n_tw;
+    int radix[MAX_MIX_STAGES];
+};
+
+// The radices of n (at most 10, or 13 with a factor 11 or 13): as few stages as possible, then the
+// smallest largest radix (registers), then the smallest sum; the largest first, where half of a
+// zero-padded line's inputs need no load.
+inline MixLen mix_length( int n )
+{
+    std::vector<int> best, now;
+    auto better = [&]( const std::vector<int> & a ) {
+        if( best.empty() )
+            return true;
+        if( a.size() != best.size() )
+            return a.size() < best.size();
+        if( a[0] != best[0] )
+            return a[0] < best[0];
+        int sa = 0, sb = 0;
+        for( size_t k = 0; k < a.size(); ++k )
+            sa += a[k], sb += best[k];
+        return sa < sb;
+    };
+    // radices in descending order
+    std::function<void( int, int )> search = [&]( int m, int top ) {
+        if( m == 1 )
+        {
+            if( better( now ) )
+                best = now;
+            return;
+        }
+        if( (int)now.size() == MAX_MIX_STAGES )
+            return;
+        for( int r = std::min( top, m ); r >= 2; --r )
+            if( m % r == 0 )
+            {
+                now.push_back( r );
+                search( m / r, r );
+                now.pop_back();
+            }
+    };
+    if( n == 1 )
+        best = { 1 };
+    else
+        search( n, n % 11 == 0 || n % 13 == 0 ? 13 : 10 );
+    if( best.empty() )
+        throw std::runtime_error( "DDI FFT: no mixed-radix plan for length " + std::to_string( n ) );
+    MixLen L{ n, (int)best.size(), 0, {} };
+    std::copy( best.begin(), best.end(), L.radix );
+    for( int s = 1, Ns = L.radix[0]; s < L.ns; Ns *= L.radix[s++] )
+        L.n_tw += ( L.radix[s] - 1 ) * Ns;
+    return L;
+}
+
+// bytes of FP64 complex values: a tile of rows of lsr values and the twiddles behind it
+inline size_t mix_lds( const MixLen & L, int lsr )
+{
+    return 16 * ( (size_t)L.n * (size_t)lsr + (size_t)L.n_tw );
+}
+
+// fewest threads a line needs: what the in-place stages' registers hold (mix_per)
+inline int mix_least_threads( const MixLen & L )
+{
+    int lo = 1;
+    for( int s = 0; s < L.ns; ++s )
+        lo = std::max( lo, ( L.n / L.radix[s] + mix_per( L.radix[s] ) - 1 ) / mix_per( L.radix[s] ) );
+    return lo;
+}
+
+// The tile of nl lines and the threads a line gets: at least mix_least_threads, and of the counts up to
+// a quarter of the line the one with the fewest idle lanes over the stages and wavefronts, weighed
+// against the waves a CU then holds (sixteen at the kernels' registers).  All lines at once, or, unless
+// whole, the largest divisor of nl whose threads fit a block.
+inline MixTile mix_tile( const MixLen & L, int nl, int lsr, bool whole, size_t lds_max )
+{
+    const int blocks = std::max( 1, (int)( lds_max / mix_lds( L, lsr ) ) );
+    const int lo     = mix_least_threads( L );
+    MixTile best{ nl, lsr, whole ? nl : 1, lo };
+    double best_score = -1;
+    for( int m = lo; m <= std::max( lo, ( L.n + 3 ) / 4 ); ++m )
+    {
+        int nc = nl;
+        while( !whole && nc > 1 && ( nc * m > MIX_MAX_THREADS || nl % nc != 0 ) )
+            --nc;
+        double rounds = 0;
+        for( int s = 0; s < L.ns; ++s )
+            rounds += ( L.n / L.radix[s] + m - 1 ) / m * L.radix[s];
+        const int waves    = ( nc * m + 63 ) / 64;
+        const double use   = (double)L.n * L.ns / ( rounds * m ) * ( nc * m ) / ( 64.0 * waves );
+        const double score = use * std::sqrt( std::min( 1.0, blocks * waves / 16.0 ) );
+        if( nc * m <= MIX_MAX_THREADS && score > best_score + 1e-9 )
+            best_score = score, best.nc = nc, best.m = m;
+    }
+    return best;
+}
+
+// Lines of a tile (a power of two), of n_lines altogether, `arrays` lines in LDS for each; fewer than
+// `least` only where LDS forces it.
+inline int mix_lines( const MixLen & L, int arrays, long long n_lines, int want, int least, size_t lds_max )
+{
+    int cw = want;
+    while( cw > 1
+           && ( mix_lds( L, arrays * cw ) > lds_max / ( cw > 8 ? 2 : 1 )
+                || ( cw > least && ( n_lines + cw - 1 ) / cw < 192 ) ) )
+        cw /= 2;
+    return cw;
+}
+
+// The tile of a pass whose threads keep one line for the whole transform (A, A^-1, B, B^-1): no more
+// lines than the block has threads for; nl = 0 where none fits.
+inline MixTile mix_line_tile( const MixLen & L, long long n_lines, int want, int least, size_t lds_max )
+{
+    int cw = mix_lines( L, 1, n_lines, want, least, lds_max );
+    while( cw > 1 && cw * mix_least_threads( L ) > MIX_MAX_THREADS )
+        cw /= 2;
+    if( mix_lds( L, cw ) > lds_max || cw * mix_least_threads( L ) > MIX_MAX_THREADS )
+        return MixTile{ 0, 0, 0, 0 };
+    return mix_tile( L, cw, cw, true, lds_max );
+}
+
+// Pass A: row pairs are contiguous whatever their number is: 4, fewer where that fills the chip.
+inline MixTile mix_row_tile( const MixLen & L, long long n_lines, size_t lds_max )
+{
+    return mix_line_tile( L, n_lines, 4, 1, lds_max );
+}
+
+// Pass B: a row piece of a column tile is 16 cw bytes, so tiles are 16 wide where two blocks then fit a
+// CU's LDS, else 8, and narrower only where LDS forces it or fewer than 192 blocks would leave CUs
+// idle (not below 4, 64 bytes): 14 us a pass against 18 and 22 at 16, 8, 4 columns of 300 points, 13
+// against 16 and 22 at 8, 4, 2 of 1000.
+inline MixTile mix_column_tile( const MixLen & L, long long n_lines, size_t lds_max )
+{
+    return mix_line_tile( L, n_lines, 16, 4, lds_max );
+}
+
+} // namespace spirit_hip

@@ -1,7 +1,7 @@
 """The dipolar FFT convolution at transform lengths that are no power of two, against the oracle's
 field: every radix (2 to 13) on every axis, lengths of one point, odd row counts (the last row pair
-has one row), partly filled column tiles, unpadded periodic lengths, two basis atoms and lattices of
-one plane.  Tolerance 1e-12 of the largest gradient: the transforms' rounding, eps log2(n) with the
+has one row), partly filled column tiles, narrow tiles of long lines and wide ones of many columns,
+unpadded periodic lengths, two basis atoms and lattices of one plane.  Tolerance 1e-12 of the largest gradient: the transforms' rounding, eps log2(n) with the
 sums over a lattice, stays below 1e-14."""
 import numpy as np
 import pytest
@@ -32,6 +32,16 @@ CASES = [
     ([22, 26, 1], "110", 0, 2),
     ([1, 7, 1], "000", 1, 1),
     ([7, 1, 1], "000", 1, 1),
+    # tiles that more than a block's threads could serve: few columns or row pairs a tile
+    ([200, 520, 4], "000", 1, 1),  # 1040 along b
+    ([128, 560, 8], "000", 1, 1),  # 1120 along b
+    ([6, 864, 2], "000", 1, 1),    # 1728 along b
+    ([6, 1008, 2], "000", 1, 1),   # 2016 along b
+    ([864, 16, 35], "000", 1, 1),  # 1728 along a, 840 row pairs
+    ([1008, 16, 35], "000", 1, 1), # 2016 along a
+    # the tiles of films: 16 columns of 300 points, 8 of 400, 4 row pairs
+    ([64, 150, 32], "000", 1, 1),
+    ([100, 200, 20], "000", 1, 1),
 ]
 
 
