@@ -79,8 +79,6 @@ struct DhatSymmetry
     double max_abs, max_imag, max_asym_b, max_asym_c;
 };
 
-int fft_lines_per_block( const FftLen & L );
-
 // Pass C kernels that can run this plan, as (c_kind, c_tk) pairs (at least one).
 std::vector<std::pair<int, int>> ddi_pass_c_candidates( const DdiDev & d );
 
@@ -94,6 +92,11 @@ void mix_launch_a_fwd( const DdiDev & d, const double * s, int nos, hipStream_t 
 void mix_launch_a_inv( const DdiDev & d, double * h, int nos, hipStream_t st );
 void mix_launch_b( const DdiDev & d, bool inverse, hipStream_t st );
 void mix_launch_conv( const DdiDev & d, bool along_b, hipStream_t st );
+
+// The kernel spectrum of the real-space tensor D[6 * n_inter][Pc][Pb][Pa], transformed along a, b (in
+// `work`, rows of stride Hs) and c on the same tiles: any number of values, whatever a block's threads hold.
+bool mix_spectrum_ok( const DdiDev & d );
+void mix_launch_spectrum( const DdiDev & d, const double * D, double2 * work, double2 * Dfull, hipStream_t st );
 
 // nullptr if every pass of the plan fits the device's LDS, else the reason it does not.
 const char * ddi_plan_problem( const DdiDev & d );

@@ -3,7 +3,7 @@
 #pragma once
 
 #include "ddi.hpp"
-#include "fft_lds.hpp"
+#include "fft_small.hpp"
 
 namespace spirit_hip
 {

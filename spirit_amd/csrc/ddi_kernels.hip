@@ -24,125 +24,6 @@
 namespace spirit_hip
 {
 
-constexpr int FFT_THREADS = 256;
-constexpr int LDS_CPLX    = 4096; // 64 KiB of FP64 complex for the generic kernels
-
-// ===========================================================================
-// Kernel-spectrum set-up (any padded length with factors 2,3,5,7,11,13)
-// ===========================================================================
-
-// Pass A: real rows of n_arr arrays -> half spectra; output rows of stride hs.
-__global__ void __launch_bounds__( FFT_THREADS )
-    k_pass_a_fwd( DdiDev d, const double * __restrict__ src, int n_arr, int Na_in, int Nb_in, int Nc_in, int hs,
-                  double2 * __restrict__ out, int lines_per_block )
-{
-    extern __shared__ double2 lds[];
-    const int Pa            = d.La.n;
-    const int ls            = Pa + 1;
-    const long long n_lines = (long long)n_arr * Nb_in * Nc_in;
-    const long long line0   = (long long)blockIdx.x * lines_per_block;
-    int nl                  = lines_per_block;
-    if( line0 + nl > n_lines )
-        nl = (int)( n_lines - line0 );
-
-    for( int e = threadIdx.x; e < nl * Pa; e += blockDim.x )
-    {
-        int l          = e / Pa;
-        int a          = e - l * Pa;
-        long long line = line0 + l;
-        double v       = a < Na_in ? src[line * (long long)Na_in + a] : 0.0;
-        lds[l * ls + a] = make_double2( v, 0.0 );
-    }
-    __syncthreads();
-    lds_fft<false>( lds, ls, nl, d.La );
-    const int Ha = d.Ha;
-    for( int e = threadIdx.x; e < nl * Ha; e += blockDim.x )
-    {
-        int l          = e / Ha;
-        int ka         = e - l * Ha;
-        long long line = line0 + l;
-        out[line * hs + ka] = lds[l * ls + ka];
-    }
-}
-
-// Pass B: columns along b for (arr, c, ka-tile), in place; rows of stride hs.
-__global__ void __launch_bounds__( FFT_THREADS )
-    k_pass_b( DdiDev d, double2 * __restrict__ X, int n_arr, int c_ext, int hs, int tk )
-{
-    extern __shared__ double2 lds[];
-    const int Pb      = d.Lb.n;
-    const int Ha      = d.Ha;
-    const int ls      = Pb + 1;
-    const int n_tiles = ( Ha + tk - 1 ) / tk;
-    long long bid     = blockIdx.x;
-    const int tile    = (int)( bid % n_tiles );
-    bid /= n_tiles;
-    const int c    = (int)( bid % c_ext );
-    const int arr  = (int)( bid / c_ext );
-    const int ka0  = tile * tk;
-    int nk         = tk;
-    if( ka0 + nk > Ha )
-        nk = Ha - ka0;
-    double2 * slab = X + ( (long long)arr * c_ext + c ) * (long long)Pb * hs;
-
-    for( int e = threadIdx.x; e < nk * Pb; e += blockDim.x )
-    {
-        int l           = e % nk;
-        int b           = e / nk;
-        lds[l * ls + b] = slab[(long long)b * hs + ka0 + l];
-    }
-    __syncthreads();
-    lds_fft<false>( lds, ls, nk, d.Lb );
-    for( int e = threadIdx.x; e < nk * Pb; e += blockDim.x )
-    {
-        int l                             = e % nk;
-        int b                             = e / nk;
-        slab[(long long)b * hs + ka0 + l] = lds[l * ls + b];
-    }
-}
-
-// Pass C for the kernel spectrum (set-up): forward along c over all Pc planes,
-// stored as Dfull[kb][ka][kc][arr] with arr = 6*b_inter + component.
-__global__ void __launch_bounds__( FFT_THREADS )
-    k_pass_c_kernel( DdiDev d, const double2 * __restrict__ XD, double2 * __restrict__ Dfull, int tk )
-{
-    extern __shared__ double2 lds[];
-    const int Pc          = d.Lc.n;
-    const int Ha          = d.Ha;
-    const int ls          = Pc + 1;
-    const int n_arr       = 6 * d.n_inter;
-    const int n_tiles     = ( Ha + tk - 1 ) / tk;
-    const int tile        = (int)( blockIdx.x % n_tiles );
-    const int rest0       = (int)( blockIdx.x / n_tiles );
-    const int kb          = rest0 % d.Pb;
-    const int arr0        = ( rest0 / d.Pb ) * 6;
-    const int ka0         = tile * tk;
-    int nk                = tk;
-    if( ka0 + nk > Ha )
-        nk = Ha - ka0;
-    const long long plane = (long long)d.Pb * d.Hs;
-
-    for( int e = threadIdx.x; e < 6 * nk * Pc; e += blockDim.x )
-    {
-        int l    = e % nk;
-        int rest = e / nk;
-        int c    = rest % Pc;
-        int a6   = rest / Pc;
-        lds[( a6 * nk + l ) * ls + c]
-            = XD[( (long long)( arr0 + a6 ) * Pc + c ) * plane + (long long)kb * d.Hs + ka0 + l];
-    }
-    __syncthreads();
-    lds_fft<false>( lds, ls, 6 * nk, d.Lc );
-    for( int e = threadIdx.x; e < 6 * nk * Pc; e += blockDim.x )
-    {
-        int a6   = e % 6;
-        int rest = e / 6;
-        int kc   = rest % Pc;
-        int l    = rest / Pc;
-        Dfull[( ( (long long)kb * Ha + ka0 + l ) * Pc + kc ) * n_arr + arr0 + a6] = lds[( a6 * nk + l ) * ls + kc];
-    }
-}
-
 // Real-space dipole tensor on the padded grid, FFT_Dipole_Matrices (Hamiltonian_Heisenberg.cpp:1406-1499).
 // out[(b_inter*6 + comp)][c][b][a]
 __global__ void k_dipole_matrices( DipoleArgs g, double * __restrict__ out )
@@ -824,31 +705,6 @@ __global__ void __launch_bounds__( 1024 ) k_p2_c( DdiDev d, double2 * __restrict
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
-int fft_lines_per_block( const FftLen & L )
-{
-    // nlines * (n+1) <= LDS_CPLX, and every stage's butterflies fit the
-    // (16/R)*R values a thread may hold for radix R
-    const int n = L.n;
-    int vals    = 16;
-    for( int s = 0; s < L.n_stages; ++s )
-    {
-        int r = L.radix[s];
-        int v = ( 16 / r ) * r;
-        if( v < vals )
-            vals = v;
-    }
-    int lines = LDS_CPLX / ( n + 1 );
-    int cap   = ( vals * FFT_THREADS ) / n;
-    if( cap < lines )
-        lines = cap;
-    return lines < 1 ? 1 : lines;
-}
-
-static size_t lds_bytes( int lines, int n )
-{
-    return sizeof( double2 ) * (size_t)lines * (size_t)( n + 1 );
-}
-
 static bool is_p2( const FftLen & L )
 {
     return L.n >= 8 && L.n <= 4096 && ( L.n & ( L.n - 1 ) ) == 0 && L.tw2 != nullptr;
@@ -969,14 +825,13 @@ std::vector<std::pair<int, int>> ddi_pass_c_candidates( const DdiDev & d )
 
 const char * ddi_plan_problem( const DdiDev & d )
 {
-    const size_t lim = (size_t)d.lds_max;
-    if( ( !p2_ab_ok( d, d.La ) && !mix_a_ok( d ) ) || lds_bytes( fft_lines_per_block( d.La ), d.La.n ) > lim )
+    if( !p2_ab_ok( d, d.La ) && !mix_a_ok( d ) )
         return "padded length along a exceeds the LDS of one block";
-    if( ( !p2_b_ok( d ) && !mix_b_ok( d ) ) || lds_bytes( fft_lines_per_block( d.Lb ), d.Lb.n ) > lim )
+    if( !p2_b_ok( d ) && !mix_b_ok( d ) )
         return "padded length along b exceeds the LDS of one block";
     if( !p2_c1_ok( d ) && p2_c_tk( d ) == 0 && !mix_conv_ok( d, false ) )
         return "padded length along c times 3*n_cell_atoms exceeds the LDS of one block";
-    if( lds_bytes( 6 * std::max( 1, fft_lines_per_block( d.Lc ) / 6 ), d.Lc.n ) > lim )
+    if( !mix_spectrum_ok( d ) )
         return "padded length along c exceeds the LDS of the kernel-spectrum set-up";
     return nullptr;
 }
@@ -1129,31 +984,7 @@ void ddi_launch_kernel_spectrum( const DdiDev & d, const DipoleArgs & g, double 
 {
     const long long M = (long long)d.La.n * d.Lb.n * d.Lc.n;
     hipLaunchKernelGGL( k_dipole_matrices, dim3( (unsigned)( ( M + 255 ) / 256 ) ), dim3( 256 ), 0, st, g, work );
-    const int n_arr = 6 * d.n_inter;
-    const int Pa = d.La.n, Pb = d.Lb.n, Pc = d.Lc.n;
-    {
-        const int lpb         = fft_lines_per_block( d.La );
-        const long long lines = (long long)n_arr * Pb * Pc;
-        const int blocks      = (int)( ( lines + lpb - 1 ) / lpb );
-        hipLaunchKernelGGL( k_pass_a_fwd, dim3( blocks ), dim3( FFT_THREADS ), lds_bytes( lpb, Pa ), st, d, work,
-                            n_arr, Pa, Pb, Pc, d.Hs, work2, lpb );
-    }
-    {
-        const int tk     = fft_lines_per_block( d.Lb );
-        const int tiles  = ( d.Ha + tk - 1 ) / tk;
-        const int blocks = tiles * Pc * n_arr;
-        hipLaunchKernelGGL( k_pass_b, dim3( blocks ), dim3( FFT_THREADS ), lds_bytes( tk, Pb ), st, d, work2, n_arr,
-                            Pc, d.Hs, tk );
-    }
-    {
-        int tk = fft_lines_per_block( d.Lc ) / 6;
-        if( tk < 1 )
-            tk = 1;
-        const int tiles  = ( d.Ha + tk - 1 ) / tk;
-        const int blocks = tiles * Pb * d.n_inter;
-        hipLaunchKernelGGL( k_pass_c_kernel, dim3( blocks ), dim3( FFT_THREADS ), lds_bytes( 6 * tk, Pc ), st, d,
-                            work2, Dfull, tk );
-    }
+    mix_launch_spectrum( d, work, work2, Dfull, st );
 }
 
 void ddi_launch_symmetry_check( const DdiDev & d, const double2 * Dfull, DhatSymmetry * out, hipStream_t st )

@@ -28,7 +28,7 @@ __global__ void __launch_bounds__( 1024 )
     k_mix_a_fwd( DdiDev d, MixPlan P, MixTile tile, const double * __restrict__ s, int nos )
 {
     extern __shared__ double2 lds[];
-    const MixBlock T( tile, P, lds );
+    const MixBlock<> T( tile, P, lds );
     const int N         = P.n;
     const int cw        = T.nl;
     const int l         = T.lc; // this thread's line
@@ -77,7 +77,7 @@ __global__ void __launch_bounds__( 1024 )
     k_mix_a_inv( DdiDev d, MixPlan P, MixTile tile, double * __restrict__ h, int nos )
 {
     extern __shared__ double2 lds[];
-    const MixBlock T( tile, P, lds );
+    const MixBlock<> T( tile, P, lds );
     const int N          = P.n;
     const int cw         = T.nl;
     const int l          = T.lc;
@@ -128,7 +128,7 @@ __global__ void __launch_bounds__( 1024 )
     k_mix_b( DdiDev d, MixPlan P, MixTile tile, double2 * __restrict__ X, int n_tiles, int b_in, int b_out )
 {
     extern __shared__ double2 lds[];
-    const MixBlock T( tile, P, lds );
+    const MixBlock<> T( tile, P, lds );
     const int cw   = T.nl;
     const int l    = T.lc;
     const int bid  = ( d.rev & ( INV ? DDI_REV_B_INV : DDI_REV_B_FWD ) ) ? gridDim.x - 1 - blockIdx.x : blockIdx.x;
@@ -157,7 +157,7 @@ __global__ void __launch_bounds__( 1024 )
                 int n_tiles, int order_pairs )
 {
     extern __shared__ double2 lds[];
-    const MixBlock T( mt, P, lds );
+    const MixBlock<> T( mt, P, lds );
     // XCD-contiguous block order: neighbouring column tiles share cache lines of a row
     const int nblk = gridDim.x;
     const int full = ( nblk / 8 ) * 8;
@@ -198,6 +198,55 @@ __global__ void __launch_bounds__( 1024 )
 }
 
 // ---------------------------------------------------------------------------
+// the kernel spectrum (set-up)
+// ---------------------------------------------------------------------------
+// Rows along a: one real row a line, its half spectrum to a row of stride Hs.
+template<bool WIDE>
+__global__ void __launch_bounds__( 1024 )
+    k_mix_rows( MixPlan P, MixTile tile, const double * __restrict__ src, double2 * __restrict__ out, long long n_rows,
+                int Ha, int Hs )
+{
+    extern __shared__ double2 lds[];
+    const MixBlock<> T( tile, P, lds );
+    const long long row = (long long)blockIdx.x * T.nl + T.lc;
+    const bool act      = row < n_rows;
+    const double * in   = src + row * P.n;
+    mix_fft_to_lds<false, WIDE>( P, T, [&]( int, int a ) { return make_double2( act ? in[a] : 0.0, 0.0 ); } );
+    if( act )
+        for( int k = T.j0; k < Ha; k += T.m )
+            out[row * Hs + k] = T.at( k, T.lc );
+}
+
+// Columns along c of the six components of a pair of sublattices, all Pc planes, stored as
+// Dfull[kb][ka][kc][6 * pair + component].
+template<bool WIDE>
+__global__ void __launch_bounds__( 1024 )
+    k_mix_c_spectrum( DdiDev d, MixPlan P, MixTile mt, const double2 * __restrict__ X, double2 * __restrict__ Dfull, int cw,
+                      MixDiv by_cw, int n_tiles )
+{
+    extern __shared__ double2 lds[];
+    const MixBlock<false> T( mt, P, lds );
+    const int rest        = blockIdx.x / n_tiles;
+    const int ka0         = ( blockIdx.x - rest * n_tiles ) * cw;
+    const int pair        = rest / d.Pb;
+    const int kb          = rest - pair * d.Pb;
+    const int nk          = min( cw, d.Ha - ka0 );
+    const long long plane = (long long)d.Pb * d.Hs;
+    const double2 * base  = X + 6LL * pair * P.n * plane + (long long)kb * d.Hs + ka0;
+    mix_fft_to_lds<false, WIDE>( P, T, [&]( int l, int c ) {
+        const int q = mix_div( l, by_cw ), col = l - q * cw;
+        return col < nk ? base[( (long long)q * P.n + c ) * plane + col] : make_double2( 0, 0 );
+    } );
+    double2 * out = Dfull + ( (long long)kb * d.Ha + ka0 ) * P.n * ( 6 * d.n_inter ) + 6 * pair;
+    for( int e = threadIdx.x; e < 6 * nk * P.n; e += blockDim.x )
+    {
+        const int at = e / 6, q = e - 6 * at;
+        const int col = at / P.n, kc = at - col * P.n;
+        out[(long long)at * ( 6 * d.n_inter ) + q] = T.at( kc, q * cw + col );
+    }
+}
+
+// ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
 static bool mix_wide( const DdiDev & d, int axis )
@@ -225,25 +274,15 @@ bool mix_b_ok( const DdiDev & d )
     return mix_b_tile( d ).nl > 0;
 }
 
-// Columns and LDS row stride of the convolution pass.  Along b a block holds all arrays of its
-// columns and there are only Ha / cw blocks, so its tiles narrow down to one column.
-static int mix_conv_cols( const DdiDev & d, bool along_b, int & lsr )
+static MixArraysTile mix_c_tile( const DdiDev & d, bool along_b )
 {
-    const MixLen & L = d.mix->len[along_b ? 1 : 2];
-    const int cw     = along_b ? mix_lines( L, 3 * d.nb, d.Ha, 16, 1, d.lds_max )
-                               : mix_lines( L, 3 * d.nb, (long long)d.Ha * d.Pb, 16, 4, d.lds_max );
-    // an odd row stride spreads the spectrum product's column accesses over the banks
-    lsr = ( 3 * d.nb * cw ) | 1;
-    if( mix_lds( L, lsr ) > (size_t)d.lds_max )
-        lsr = 3 * d.nb * cw;
-    return cw;
+    return along_b ? mix_conv_tile( d.mix->len[1], 3 * d.nb, d.Ha, true, d.lds_max )
+                   : mix_conv_tile( d.mix->len[2], 3 * d.nb, (long long)d.Ha * d.Pb, false, d.lds_max );
 }
 
 bool mix_conv_ok( const DdiDev & d, bool along_b )
 {
-    int lsr;
-    (void)mix_conv_cols( d, along_b, lsr );
-    return mix_lds( d.mix->len[along_b ? 1 : 2], lsr ) <= (size_t)d.lds_max;
+    return mix_c_tile( d, along_b ).t.nl > 0;
 }
 
 void mix_launch_a_fwd( const DdiDev & d, const double * s, int nos, hipStream_t st )
@@ -278,14 +317,11 @@ void mix_launch_b( const DdiDev & d, bool inverse, hipStream_t st )
 
 void mix_launch_conv( const DdiDev & d, bool along_b, hipStream_t st )
 {
-    int lsr           = 0;
-    const int axis    = along_b ? 1 : 2;
-    const int cw      = mix_conv_cols( d, along_b, lsr );
-    const MixPlan & P = d.mix->plan[axis];
-    const MixLen & L  = d.mix->len[axis];
-    const int tiles   = ( d.Ha + cw - 1 ) / cw;
-    const MixTile T   = mix_tile( L, 3 * d.nb * cw, lsr, false, d.lds_max );
-    const MixDiv by_cw{ 1.0f / (float)cw }, by_n{ 1.0f / (float)P.n };
+    const int axis        = along_b ? 1 : 2;
+    const MixPlan & P     = d.mix->plan[axis];
+    const MixArraysTile C = mix_c_tile( d, along_b );
+    const int tiles       = ( d.Ha + C.cw - 1 ) / C.cw;
+    const MixDiv by_cw{ 1.0f / (float)C.cw }, by_n{ 1.0f / (float)P.n };
     const bool w = mix_wide( d, axis ), one = d.nb == 1;
     const auto k = along_b ? ( w     ? k_mix_conv<true, true, false>
                                : one ? k_mix_conv<true, false, true>
@@ -293,8 +329,49 @@ void mix_launch_conv( const DdiDev & d, bool along_b, hipStream_t st )
                            : ( w     ? k_mix_conv<false, true, false>
                                : one ? k_mix_conv<false, false, true>
                                      : k_mix_conv<false, false, false> );
-    hipLaunchKernelGGL( k, dim3( (unsigned)( (long long)tiles * ( along_b ? 1 : d.Pb ) ) ), dim3( T.nc * T.m ),
-                        mix_lds( L, lsr ), st, d, P, T, d.X, cw, by_cw, by_n, tiles, !along_b && d.sym_b ? 1 : 0 );
+    hipLaunchKernelGGL( k, dim3( (unsigned)( (long long)tiles * ( along_b ? 1 : d.Pb ) ) ), dim3( C.t.nc * C.t.m ),
+                        mix_lds( d.mix->len[axis], C.t.lsr ), st, d, P, C.t, d.X, C.cw, by_cw, by_n, tiles,
+                        !along_b && d.sym_b ? 1 : 0 );
+}
+
+static MixArraysTile mix_c_spectrum_tile( const DdiDev & d )
+{
+    return mix_spectrum_tile( d.mix->len[2], (long long)d.Ha * d.Pb * d.n_inter, d.lds_max );
+}
+
+bool mix_spectrum_ok( const DdiDev & d )
+{
+    const long long n_rows = 6LL * d.n_inter * d.Pb * d.Pc, n_cols = 6LL * d.n_inter * d.Ha * d.Pc;
+    return mix_row_tile( d.mix->len[0], n_rows, d.lds_max ).nl > 0
+           && mix_column_tile( d.mix->len[1], n_cols, d.lds_max ).nl > 0 && mix_c_spectrum_tile( d ).t.nl > 0;
+}
+
+void mix_launch_spectrum( const DdiDev & d, const double * D, double2 * work, double2 * Dfull, hipStream_t st )
+{
+    const MixLen * L        = d.mix->len;
+    const long long n_slabs = 6LL * d.n_inter * d.Pc;
+    {
+        const long long n_rows = n_slabs * d.Pb;
+        const MixTile T        = mix_row_tile( L[0], n_rows, d.lds_max );
+        const auto k           = mix_wide( d, 0 ) ? k_mix_rows<true> : k_mix_rows<false>;
+        hipLaunchKernelGGL( k, dim3( (unsigned)( ( n_rows + T.nl - 1 ) / T.nl ) ), dim3( T.nc * T.m ),
+                            mix_lds( L[0], T.lsr ), st, d.mix->plan[0], T, D, work, n_rows, d.Ha, d.Hs );
+    }
+    {
+        const MixTile T = mix_column_tile( L[1], n_slabs * d.Ha, d.lds_max );
+        const int tiles = ( d.Ha + T.nl - 1 ) / T.nl;
+        const auto k    = mix_wide( d, 1 ) ? k_mix_b<false, true> : k_mix_b<false, false>;
+        hipLaunchKernelGGL( k, dim3( (unsigned)( n_slabs * tiles ) ), dim3( T.nc * T.m ), mix_lds( L[1], T.lsr ), st, d,
+                            d.mix->plan[1], T, work, tiles, d.Pb, d.Pb );
+    }
+    {
+        const MixArraysTile C = mix_c_spectrum_tile( d );
+        const int tiles       = ( d.Ha + C.cw - 1 ) / C.cw;
+        const auto k          = mix_wide( d, 2 ) ? k_mix_c_spectrum<true> : k_mix_c_spectrum<false>;
+        hipLaunchKernelGGL( k, dim3( (unsigned)( (long long)tiles * d.Pb * d.n_inter ) ), dim3( C.t.nc * C.t.m ),
+                            mix_lds( L[2], C.t.lsr, false ), st, d, d.mix->plan[2], C.t, work, Dfull, C.cw,
+                            MixDiv{ 1.0f / (float)C.cw }, tiles );
+    }
 }
 
 } // namespace spirit_hip

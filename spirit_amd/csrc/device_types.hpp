@@ -15,7 +15,6 @@ namespace spirit_hip
 
 constexpr int MAX_BASIS      = 8;
 constexpr int MAX_PAIRS      = 64;
-constexpr int MAX_FFT_STAGES = 16;
 constexpr int MAX_REACH      = 3; // cells away that the pair loops' offset table covers (SiteOffsets)
 constexpr int GATHER_PAIRS   = 6; // pair tables up to this size are gathered into registers per spin
 
@@ -182,15 +181,13 @@ struct MixPlan
     const double2 * tw;  // n_tw stage twiddles, device memory
 };
 
-// One FFT length: Stockham stage radices and the n-th roots of unity exp(-2 pi i e / n).
+// One FFT length: the n-th roots of unity exp(-2 pi i e / n).
 // For powers of two >= 8, tw2 holds the twiddles of the register-resident radix-8
 // plan in stage order: stage s (>= 1, radix R, Ns = 8^s) at offset 8^s - 8,
 // entry jm*(R-1) + r-1 = w_n^(r * jm * n/(Ns*R)).
 struct FftLen
 {
     int n;
-    int n_stages;
-    int radix[MAX_FFT_STAGES];
     const double2 * W;
     const double2 * tw2;
 };

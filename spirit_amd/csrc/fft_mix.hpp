@@ -15,10 +15,10 @@
 // outputs after it.
 //
 // Stage twiddles w_n^(r jm n/(Ns R)) come from a table in stage order, [r - 1][jm], which the
-// block copies to LDS behind its tile: the lanes that share jm read one address.
+// block copies to LDS behind its tile (or reads where it is): the lanes that share jm read one address.
 #pragma once
 
-#include "fft_lds.hpp"
+#include "fft_small.hpp"
 
 namespace spirit_hip
 {
@@ -181,7 +181,7 @@ __device__ __forceinline__ void mix_dft( double2 * v )
     if constexpr( R == 1 )
         return;
     else if constexpr( R == 2 || R == 4 || R == 8 )
-        dft_small<R, INV>( v, nullptr, R );
+        dft_small<R, INV>( v );
     else if constexpr( R == 6 )
         dft_coprime<2, 3, INV>( v );
     else if constexpr( R == 9 )
@@ -203,6 +203,8 @@ struct MixPer
 
 // The tile a block transforms: nl lines, LDS row stride lsr, m threads a line; a tile of more
 // lines than the block has threads for is taken in groups of nc lines.
+// TW_LDS: the twiddles are copied behind the tile, else they are read from the plan's table.
+template<bool TW_LDS = true>
 struct MixBlock
 {
     int nl, lsr, nc, m;
@@ -210,14 +212,17 @@ struct MixBlock
     double2 * lds;
     const double2 * tw;
     __device__ __forceinline__ MixBlock( const MixTile & T, const MixPlan & P, double2 * mem )
-            : nl( T.nl ), lsr( T.lsr ), nc( T.nc ), m( T.m ), lds( mem ), tw( mem + P.n * T.lsr )
+            : nl( T.nl ), lsr( T.lsr ), nc( T.nc ), m( T.m ), lds( mem ), tw( TW_LDS ? mem + P.n * T.lsr : P.tw )
     {
         j0 = (int)threadIdx.x / nc;
         lc = (int)threadIdx.x - j0 * nc;
-        // settled by the barrier behind the first stage
-        double2 * t = mem + P.n * T.lsr;
-        for( int e = threadIdx.x; e < P.n_tw; e += blockDim.x )
-            t[e] = P.tw[e];
+        if constexpr( TW_LDS )
+        {
+            // settled by the barrier behind the first stage
+            double2 * t = mem + P.n * T.lsr;
+            for( int e = threadIdx.x; e < P.n_tw; e += blockDim.x )
+                t[e] = P.tw[e];
+        }
     }
     __device__ __forceinline__ double2 & at( int p, int l ) const
     {
@@ -241,7 +246,8 @@ __device__ __forceinline__ MixStage mix_stage( const MixPlan & P, int s )
 
 // A thread's first butterfly, opaque to the optimiser: the index arithmetic of a stage stays inside
 // its radix's branch (hoisted out of the radix switch, the variants' indices spill registers).
-__device__ __forceinline__ int mix_j0( const MixBlock & T )
+template<typename BLK>
+__device__ __forceinline__ int mix_j0( const BLK & T )
 {
     int t = T.j0;
     asm volatile( "" : "+v"( t ) );
@@ -256,8 +262,8 @@ __device__ __forceinline__ int mix_opaque( int x )
 }
 
 // first stage: inputs from ld( l, point ), outputs to st( l, position, value )
-template<int R, bool INV, typename LD, typename ST>
-__device__ __forceinline__ void mix_first( const MixStage & S, const MixBlock & T, LD ld, ST st )
+template<int R, bool INV, typename BLK, typename LD, typename ST>
+__device__ __forceinline__ void mix_first( const MixStage & S, const BLK & T, LD ld, ST st )
 {
     const int nbf = mix_opaque( S.nbf );
 #pragma unroll 1
@@ -276,8 +282,8 @@ __device__ __forceinline__ void mix_first( const MixStage & S, const MixBlock & 
         }
 }
 
-template<int R, bool INV>
-__device__ __forceinline__ void mix_twiddle( const MixBlock & T, const MixStage & S, int jm, double2 * u )
+template<int R, bool INV, typename BLK>
+__device__ __forceinline__ void mix_twiddle( const BLK & T, const MixStage & S, int jm, double2 * u )
 {
     if( S.Ns == 1 )
         return;
@@ -293,8 +299,8 @@ __device__ __forceinline__ void mix_twiddle( const MixBlock & T, const MixStage 
 }
 
 // a stage from LDS to LDS, in place; every thread of the block calls it; LDS is settled on return
-template<int R, bool INV>
-__device__ __forceinline__ void mix_mid( const MixStage & S, const MixBlock & T )
+template<int R, bool INV, typename BLK>
+__device__ __forceinline__ void mix_mid( const MixStage & S, const BLK & T )
 {
     if constexpr( R == 1 )
         return; // a line of one point
@@ -338,8 +344,8 @@ __device__ __forceinline__ void mix_mid( const MixStage & S, const MixBlock & T 
 }
 
 // last stage: inputs from LDS, output of point p of line l to st( l, p, value )
-template<int R, bool INV, typename ST>
-__device__ __forceinline__ void mix_last( const MixStage & S, const MixBlock & T, ST st )
+template<int R, bool INV, typename BLK, typename ST>
+__device__ __forceinline__ void mix_last( const MixStage & S, const BLK & T, ST st )
 {
     const int nbf = mix_opaque( S.nbf );
 #pragma unroll 1
@@ -387,8 +393,8 @@ __device__ __forceinline__ void mix_last( const MixStage & S, const MixBlock & T
             break;                                                                                                     \
     }
 
-template<bool INV, bool WIDE>
-__device__ __forceinline__ void mix_mid_any( const MixPlan & P, const MixBlock & T, int s )
+template<bool INV, bool WIDE, typename BLK>
+__device__ __forceinline__ void mix_mid_any( const MixPlan & P, const BLK & T, int s )
 {
     const MixStage S = mix_stage( P, s );
 #define MIX_CALL( R ) mix_mid<R, INV>( S, T )
@@ -397,8 +403,8 @@ __device__ __forceinline__ void mix_mid_any( const MixPlan & P, const MixBlock &
 }
 
 // The transform of ld's inputs left in LDS in natural order (settled on return).
-template<bool INV, bool WIDE, typename LD>
-__device__ __forceinline__ void mix_fft_to_lds( const MixPlan & P, const MixBlock & T, LD ld )
+template<bool INV, bool WIDE, typename BLK, typename LD>
+__device__ __forceinline__ void mix_fft_to_lds( const MixPlan & P, const BLK & T, LD ld )
 {
     const MixStage S0 = mix_stage( P, 0 );
     auto put          = [&]( int l, int p, double2 v ) { T.at( p, l ) = v; };
@@ -410,8 +416,8 @@ __device__ __forceinline__ void mix_fft_to_lds( const MixPlan & P, const MixBloc
         mix_mid_any<INV, WIDE>( P, T, s );
 }
 
-template<bool INV, bool WIDE, typename ST>
-__device__ __forceinline__ void mix_last_any( const MixPlan & P, const MixBlock & T, ST st )
+template<bool INV, bool WIDE, typename BLK, typename ST>
+__device__ __forceinline__ void mix_last_any( const MixPlan & P, const BLK & T, ST st )
 {
     const MixStage S = mix_stage( P, P.ns - 1 );
 #define MIX_CALL( R ) mix_last<R, INV>( S, T, st )
@@ -420,8 +426,8 @@ __device__ __forceinline__ void mix_last_any( const MixPlan & P, const MixBlock 
 }
 
 // From ld's inputs to st's outputs.
-template<bool INV, bool WIDE, typename LD, typename ST>
-__device__ __forceinline__ void mix_fft( const MixPlan & P, const MixBlock & T, LD ld, ST st )
+template<bool INV, bool WIDE, typename BLK, typename LD, typename ST>
+__device__ __forceinline__ void mix_fft( const MixPlan & P, const BLK & T, LD ld, ST st )
 {
     const MixStage S0 = mix_stage( P, 0 );
     if( P.ns == 1 )
@@ -442,8 +448,8 @@ __device__ __forceinline__ void mix_fft( const MixPlan & P, const MixBlock & T, 
 }
 
 // From LDS (natural order, settled) to st's outputs.
-template<bool INV, bool WIDE, typename ST>
-__device__ __forceinline__ void mix_fft_from_lds( const MixPlan & P, const MixBlock & T, ST st )
+template<bool INV, bool WIDE, typename BLK, typename ST>
+__device__ __forceinline__ void mix_fft_from_lds( const MixPlan & P, const BLK & T, ST st )
 {
     for( int s = 0; s < P.ns - 1; ++s )
         mix_mid_any<INV, WIDE>( P, T, s );

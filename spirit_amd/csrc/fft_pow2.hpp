@@ -9,7 +9,7 @@
 // compile-time constants so all index arithmetic folds to shifts.
 #pragma once
 
-#include "fft_lds.hpp"
+#include "fft_small.hpp"
 
 namespace spirit_hip
 {
@@ -94,7 +94,7 @@ __device__ __forceinline__ void p2_stage( double2 ( &v )[8], double2 * __restric
                 u[r] = cmul( u[r], w );
             }
         }
-        dft_small<R, INV>( u, nullptr, N );
+        dft_small<R, INV>( u );
         if constexpr( LST && KEEP )
         {
             // last stage: Ns = N/R, so idxD + r*Ns = j + r*N/R = t + T*(m + M*r)
@@ -182,7 +182,7 @@ __device__ __forceinline__ void p2_stage_split( double2 ( &v )[8], double * __re
                 u[r] = cmul( u[r], w );
             }
         }
-        dft_small<R, INV>( u, nullptr, N );
+        dft_small<R, INV>( u );
 #pragma unroll
         for( int r = 0; r < R; ++r )
             out[m + M * r] = u[r];
@@ -290,7 +290,7 @@ __device__ __forceinline__ void p4_stage( double2 ( &v )[4], double2 * __restric
                 u[r] = cmul( u[r], w );
             }
         }
-        dft_small<R, INV>( u, nullptr, N );
+        dft_small<R, INV>( u );
         if constexpr( LST )
         {
             // Ns = N/R: output j + r*N/R = t + T*(m + M*r)

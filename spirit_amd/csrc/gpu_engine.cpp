@@ -53,27 +53,14 @@ void FftLenHost::build( int n )
 {
     if( n < 1 || n > 4096 )
         throw std::runtime_error( "DDI FFT: padded length " + std::to_string( n ) + " outside [1, 4096]" );
-    dev.n        = n;
-    dev.n_stages = 0;
-    int m        = n;
-    auto push    = [&]( int r ) {
-        if( dev.n_stages >= MAX_FFT_STAGES )
-            throw std::runtime_error( "DDI FFT: too many stages" );
-        dev.radix[dev.n_stages++] = r;
-        m /= r;
-    };
-    while( m % 8 == 0 )
-        push( 8 );
-    while( m % 4 == 0 )
-        push( 4 );
-    while( m % 2 == 0 )
-        push( 2 );
-    for( int r : { 3, 5, 7, 11, 13 } )
-        while( m % r == 0 )
-            push( r );
+    dev.n = n;
+    int m = n;
+    for( int p : { 2, 3, 5, 7, 11, 13 } )
+        while( m % p == 0 )
+            m /= p;
     if( m != 1 )
         throw std::runtime_error( "DDI FFT: padded length " + std::to_string( n )
-                                  + " has a prime factor above 13 (supported radices 2,3,4,5,7,8,11,13)" );
+                                  + " has a prime factor above 13" );
     std::vector<double2> w( n );
     const long double twopi = 6.283185307179586476925286766559005768L;
     for( int e = 0; e < n; ++e )

@@ -84,10 +84,10 @@ inline MixLen mix_length( int n )
     return L;
 }
 
-// bytes of FP64 complex values: a tile of rows of lsr values and the twiddles behind it
-inline size_t mix_lds( const MixLen & L, int lsr )
+// bytes of FP64 complex values: a tile of rows of lsr values and, with tw_lds, the twiddles behind it
+inline size_t mix_lds( const MixLen & L, int lsr, bool tw_lds = true )
 {
-    return 16 * ( (size_t)L.n * (size_t)lsr + (size_t)L.n_tw );
+    return 16 * ( (size_t)L.n * (size_t)lsr + (size_t)( tw_lds ? L.n_tw : 0 ) );
 }
 
 // fewest threads a line needs: what the in-place stages' registers hold (mix_per)
@@ -103,9 +103,9 @@ inline int mix_least_threads( const MixLen & L )
 // a quarter of the line the one with the fewest idle lanes over the stages and wavefronts, weighed
 // against the waves a CU then holds (sixteen at the kernels' registers).  All lines at once, or, unless
 // whole, the largest divisor of nl whose threads fit a block.
-inline MixTile mix_tile( const MixLen & L, int nl, int lsr, bool whole, size_t lds_max )
+inline MixTile mix_tile( const MixLen & L, int nl, int lsr, bool whole, size_t lds_max, bool tw_lds = true )
 {
-    const int blocks = std::max( 1, (int)( lds_max / mix_lds( L, lsr ) ) );
+    const int blocks = std::max( 1, (int)( lds_max / mix_lds( L, lsr, tw_lds ) ) );
     const int lo     = mix_least_threads( L );
     MixTile best{ nl, lsr, whole ? nl : 1, lo };
     double best_score = -1;
@@ -128,11 +128,12 @@ inline MixTile mix_tile( const MixLen & L, int nl, int lsr, bool whole, size_t l
 
 // Lines of a tile (a power of two), of n_lines altogether, `arrays` lines in LDS for each; fewer than
 // `least` only where LDS forces it.
-inline int mix_lines( const MixLen & L, int arrays, long long n_lines, int want, int least, size_t lds_max )
+inline int mix_lines( const MixLen & L, int arrays, long long n_lines, int want, int least, size_t lds_max,
+                      bool tw_lds = true )
 {
     int cw = want;
     while( cw > 1
-           && ( mix_lds( L, arrays * cw ) > lds_max / ( cw > 8 ? 2 : 1 )
+           && ( mix_lds( L, arrays * cw, tw_lds ) > lds_max / ( cw > 8 ? 2 : 1 )
                 || ( cw > least && ( n_lines + cw - 1 ) / cw < 192 ) ) )
         cw /= 2;
     return cw;
@@ -163,6 +164,40 @@ inline MixTile mix_row_tile( const MixLen & L, long long n_lines, size_t lds_max
 inline MixTile mix_column_tile( const MixLen & L, long long n_lines, size_t lds_max )
 {
     return mix_line_tile( L, n_lines, 16, 4, lds_max );
+}
+
+// The tile of a pass that holds `arrays` lines of each of its cw columns (line = array * cw + column, taken
+// in groups where the threads need it); t.nl = 0 where none fits.
+struct MixArraysTile
+{
+    MixTile t;
+    int cw;
+    bool tw_lds;
+};
+inline MixArraysTile mix_arrays_tile( const MixLen & L, int arrays, long long n_cols, int least, size_t lds_max,
+                                      bool tw_lds )
+{
+    const int cw = mix_lines( L, arrays, n_cols, 16, least, lds_max, tw_lds );
+    // an odd row stride spreads column accesses over the banks
+    int lsr = ( arrays * cw ) | 1;
+    if( mix_lds( L, lsr, tw_lds ) > lds_max )
+        lsr = arrays * cw;
+    if( mix_lds( L, lsr, tw_lds ) > lds_max || mix_least_threads( L ) > MIX_MAX_THREADS )
+        return MixArraysTile{ MixTile{ 0, 0, 0, 0 }, 0, tw_lds };
+    return MixArraysTile{ mix_tile( L, arrays * cw, lsr, false, lds_max, tw_lds ), cw, tw_lds };
+}
+
+// Pass C of n_arrays fields, or the one-plane convolution along b: there a block holds all arrays of its
+// columns and there are only n_cols / cw blocks, so its tiles narrow down to one column.
+inline MixArraysTile mix_conv_tile( const MixLen & L, int n_arrays, long long n_cols, bool along_b, size_t lds_max )
+{
+    return mix_arrays_tile( L, n_arrays, n_cols, along_b ? 1 : 4, lds_max, true );
+}
+
+// The kernel spectrum's pass C: the six components of a pair of sublattices.
+inline MixArraysTile mix_spectrum_tile( const MixLen & L, long long n_cols, size_t lds_max )
+{
+    return mix_arrays_tile( L, 6, n_cols, 1, lds_max, false );
 }
 
 } // namespace spirit_hip

@@ -42,6 +42,15 @@ CASES = [
     # the tiles of films: 16 columns of 300 points, 8 of 400, 4 row pairs
     ([64, 150, 32], "000", 1, 1),
     ([100, 200, 20], "000", 1, 1),
+    # lines of the kernel spectrum's set-up longer than one pass over a block's threads
+    ([4, 3, 264], "000", 1, 1),    # 528 along c
+    ([3, 4, 512], "000", 1, 1),    # 1024 along c
+    ([3, 2, 700], "000", 1, 1),    # 1400 along c
+    ([3, 2, 300], "000", 1, 2),    # 600 along c, two basis atoms
+    ([1500, 4, 2], "000", 1, 1),   # 3000 along a
+    ([3, 1430, 2], "000", 1, 1),   # 2860 along b
+    ([3, 2000, 1], "000", 1, 1),   # 4000 along b, one plane
+    ([2048, 3, 2], "000", 1, 1),   # 4096 along a
 ]
 
 

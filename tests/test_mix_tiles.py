@@ -45,6 +45,15 @@ static void common( const char * pass, const MixLen & L, long long lines, const 
         fail( pass, L, lines, T );
 }
 
+static void arrays( const char * pass, const MixLen & L, long long cols, const MixArraysTile & C, int n )
+{
+    if( C.t.nl == 0 )
+        return; // no tile fits: the plan is refused
+    common( pass, L, cols, C.t );
+    if( C.t.nl != n * C.cw || mix_lds( L, C.t.lsr, C.tw_lds ) > LDS )
+        fail( pass, L, cols, C.t );
+}
+
 int main()
 {
     std::vector<long long> counts;
@@ -79,6 +88,14 @@ int main()
                     fail( "columns: lines without a thread", L, c, T );
                 last_b = cb;
             }
+            if( c > 3000 || c % 7 != 1 )
+                continue;
+            // passes that hold several arrays of a column: the convolution and the kernel spectrum
+            for( int nb = 1; nb <= 8; ++nb )
+                for( int along_b = 0; along_b < 2; ++along_b )
+                    arrays( along_b ? "convolution along b" : "convolution along c", L, c,
+                            mix_conv_tile( L, 3 * nb, c, along_b, LDS ), 3 * nb );
+            arrays( "kernel spectrum", L, c, mix_spectrum_tile( L, c, LDS ), 6 );
         }
     }
     std::printf( "%d tiles, %d bad\n", tiles, bad );
