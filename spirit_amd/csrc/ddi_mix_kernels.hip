@@ -150,14 +150,14 @@ __global__ void __launch_bounds__( 1024 )
 // ALONG_B = false: pass C, the axis is c, one kb plane a block (planes kb and Pb-kb interleaved
 // with order_pairs).  ALONG_B = true: a lattice of one plane has nothing to transform along c, so
 // passes B, C and B^-1 are this one kernel along b.  ONE: one basis atom (the product over pairs of
-// basis atoms indexes a private array, which costs scratch memory).
-template<bool ALONG_B, bool WIDE, bool ONE>
+// basis atoms indexes a private array, which costs scratch memory).  TW_LDS: MixBlock's.
+template<bool ALONG_B, bool WIDE, bool ONE, bool TW_LDS = true>
 __global__ void __launch_bounds__( 1024 )
     k_mix_conv( DdiDev d, MixPlan P, MixTile mt, double2 * __restrict__ X, int cw, MixDiv by_cw, MixDiv by_n,
                 int n_tiles, int order_pairs )
 {
     extern __shared__ double2 lds[];
-    const MixBlock<> T( mt, P, lds );
+    const MixBlock<TW_LDS> T( mt, P, lds );
     // XCD-contiguous block order: neighbouring column tiles share cache lines of a row
     const int nblk = gridDim.x;
     const int full = ( nblk / 8 ) * 8;
@@ -323,14 +323,15 @@ void mix_launch_conv( const DdiDev & d, bool along_b, hipStream_t st )
     const int tiles       = ( d.Ha + C.cw - 1 ) / C.cw;
     const MixDiv by_cw{ 1.0f / (float)C.cw }, by_n{ 1.0f / (float)P.n };
     const bool w = mix_wide( d, axis ), one = d.nb == 1;
-    const auto k = along_b ? ( w     ? k_mix_conv<true, true, false>
-                               : one ? k_mix_conv<true, false, true>
-                                     : k_mix_conv<true, false, false> )
-                           : ( w     ? k_mix_conv<false, true, false>
-                               : one ? k_mix_conv<false, false, true>
-                                     : k_mix_conv<false, false, false> );
+    const auto k = along_b     ? ( w     ? k_mix_conv<true, true, false>
+                                   : one ? k_mix_conv<true, false, true>
+                                         : k_mix_conv<true, false, false> )
+                   : !C.tw_lds ? k_mix_conv<false, true, false, false>
+                               : ( w     ? k_mix_conv<false, true, false>
+                                   : one ? k_mix_conv<false, false, true>
+                                         : k_mix_conv<false, false, false> );
     hipLaunchKernelGGL( k, dim3( (unsigned)( (long long)tiles * ( along_b ? 1 : d.Pb ) ) ), dim3( C.t.nc * C.t.m ),
-                        mix_lds( d.mix->len[axis], C.t.lsr ), st, d, P, C.t, d.X, C.cw, by_cw, by_n, tiles,
+                        mix_lds( d.mix->len[axis], C.t.lsr, C.tw_lds ), st, d, P, C.t, d.X, C.cw, by_cw, by_n, tiles,
                         !along_b && d.sym_b ? 1 : 0 );
 }
 

@@ -188,10 +188,13 @@ inline MixArraysTile mix_arrays_tile( const MixLen & L, int arrays, long long n_
 }
 
 // Pass C of n_arrays fields, or the one-plane convolution along b: there a block holds all arrays of its
-// columns and there are only n_cols / cw blocks, so its tiles narrow down to one column.
+// columns and there are only n_cols / cw blocks, so its tiles narrow down to one column.  Where one
+// column of pass C leaves no room for the twiddles (1463 to 1706 points of two basis atoms, 410 to 426
+// of eight) they stay in global memory; a lattice of one plane has the passes along b instead.
 inline MixArraysTile mix_conv_tile( const MixLen & L, int n_arrays, long long n_cols, bool along_b, size_t lds_max )
 {
-    return mix_arrays_tile( L, n_arrays, n_cols, along_b ? 1 : 4, lds_max, true );
+    const MixArraysTile C = mix_arrays_tile( L, n_arrays, n_cols, along_b ? 1 : 4, lds_max, true );
+    return C.t.nl > 0 || along_b ? C : mix_arrays_tile( L, n_arrays, n_cols, 1, lds_max, false );
 }
 
 // The kernel spectrum's pass C: the six components of a pair of sublattices.

@@ -47,6 +47,8 @@ CASES = [
     ([3, 4, 512], "000", 1, 1),    # 1024 along c
     ([3, 2, 700], "000", 1, 1),    # 1400 along c
     ([3, 2, 300], "000", 1, 2),    # 600 along c, two basis atoms
+    ([2, 3, 735], "000", 1, 2),    # 1470 along c, two atoms: the twiddles do not fit behind the tile
+    ([2, 3, 210], "000", 1, 8),    # 420 along c, eight atoms
     ([1500, 4, 2], "000", 1, 1),   # 3000 along a
     ([3, 1430, 2], "000", 1, 1),   # 2860 along b
     ([3, 2000, 1], "000", 1, 1),   # 4000 along b, one plane
@@ -58,9 +60,10 @@ CASES = [
 def test_ddi_field_of_any_length(engine, oracle, cells, bc, padding, basis):  # noqa: F811
     print("CASE ddi lengths", cells, bc, padding, basis, flush=True)
     cfg = dict(bravais_lattice="sc", n_basis_cells=cells, boundary_conditions=[int(c) for c in bc],
-               mu_s=[2.0, 1.5][:basis], ddi_method="fft", ddi_n_periodic_images=[2, 1, 0], ddi_pb_zero_padding=padding)
-    if basis == 2:
-        cfg["basis"] = [[0, 0, 0], [0.5, 0.4, 0.3]]
+               mu_s=[2.0 - 0.5 * k / max(1, basis - 1) for k in range(basis)], ddi_method="fft", ddi_n_periodic_images=[2, 1, 0], ddi_pb_zero_padding=padding)
+    if basis > 1:
+        cfg["basis"] = [[0, 0, 0], [0.5, 0.4, 0.3], [0.5, 0, 0], [0, 0.5, 0], [0, 0, 0.6], [0.3, 0.7, 0.8], [0.7, 0.2, 0.1],
+                        [0.9, 0.8, 0.4]][:basis]
     e = engine(cfg)
     S = oracle.System(cfg)
     s = oracle.random_spins(S.nos, 77)

@@ -113,6 +113,43 @@ def _compile(tmp_path, source, name):
     return exe
 
 
+# which (basis atoms, points along c) have a pass C: three lines of each atom, one value of padding a
+# line, in a block's LDS, and the same for the kernel spectrum's six lines
+LIMITS = r"""
+#include "mix_tiles.hpp"
+#include <cstdio>
+#include <cstdlib>
+using namespace spirit_hip;
+int main()
+{
+    int n, nb;
+    while( std::scanf( "%d %d", &nb, &n ) == 2 )
+        std::printf( "%d %d %d %d\n", nb, n, mix_conv_tile( mix_length( n ), 3 * nb, 1000, false, 160 * 1024 ).t.nl > 0,
+                     mix_spectrum_tile( mix_length( n ), 1000, 160 * 1024 ).t.nl > 0 );
+}
+"""
+
+
+def test_lengths_along_c_that_fit_without_their_twiddles(tmp_path):
+    smooth = []
+    for n in range(1, 4097):
+        m = n
+        for p in (2, 3, 5, 7, 11, 13):
+            while m % p == 0:
+                m //= p
+        if m == 1:
+            smooth.append(n)
+    exe = _compile(tmp_path, LIMITS, "limits")
+    asked = [(nb, n) for nb in range(1, 9) for n in smooth]
+    out = subprocess.run([exe], input="\n".join("%d %d" % a for a in asked), capture_output=True, text=True, check=True)
+    rows = [tuple(map(int, l.split())) for l in out.stdout.splitlines()]
+    assert len(rows) == len(asked)
+    for nb, n, conv, spectrum in rows:
+        # 10240 complex values fit; the row padding of the lines is given up before the length
+        assert conv == (3 * nb * n <= 10240), (nb, n)
+        assert spectrum == (6 * n <= 10240), (nb, n)
+
+
 def test_every_line_of_every_tile_has_a_thread(tmp_path):
     r = subprocess.run([_compile(tmp_path, SWEEP, "sweep")], capture_output=True, text=True)
     print(r.stdout)
