@@ -272,7 +272,8 @@ __global__ void __launch_bounds__( GNEB_THREADS ) k_gneb_pass( GnebArgs A )
         if( act )
         {
             // the distance's loads go out before the field's: on images of a few thousand spins the pass is a
-            // chain of loads (21 images of 6944 spins: 16.8 instead of 18.1 us; of 16384: within 1%)
+            // chain of loads (21 images of 6944 spins: 16.8 instead of 18.1 us, and 15.8 since the neighbours'
+            // indices need no branches; 32 images of 16384: 29.0 us, and 26.9 since)
             double a[3], b[3];
             load3( A.x + base, nos, i, a );
             if( img > 0 )

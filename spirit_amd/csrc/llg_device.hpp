@@ -12,6 +12,7 @@
 #pragma once
 
 #include "llg.hpp"
+#include "neighbours.hpp"
 
 namespace spirit_hip
 {
@@ -240,98 +241,32 @@ __device__ __forceinline__ void load_spin( const double * f, int nos, int i, dou
         load3( f, nos, i, v );
 }
 
-// ---------------------------------------------------------------------------
-// neighbour index, Vectormath.hpp:437-528 (defects off)
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ int pair_neighbour( const HamDev & H, int a, int b, int c, const PairDev & p )
-{
-    const int Na = H.Na, Nb = H.Nb, Nc = H.Nc;
-    if( abs( p.da ) > Na || abs( p.db ) > Nb || abs( p.dc ) > Nc )
-        return -1;
-    int ja = a + p.da, jb = b + p.db, jc = c + p.dc;
-    if( H.bc[0] || ( 0 <= ja && ja < Na ) )
-    {
-        if( ja < 0 )
-            ja += Na;
-        if( ja >= Na )
-            ja -= Na;
-    }
-    else
-        return -1;
-    if( H.bc[1] || ( 0 <= jb && jb < Nb ) )
-    {
-        if( jb < 0 )
-            jb += Nb;
-        if( jb >= Nb )
-            jb -= Nb;
-    }
-    else
-        return -1;
-    if( H.bc[2] || ( 0 <= jc && jc < Nc ) )
-    {
-        if( jc < 0 )
-            jc += Nc;
-        if( jc >= Nc )
-            jc -= Nc;
-    }
-    else
-        return -1;
-    return p.j + H.nb * ( ja + Na * ( jb + Nb * jc ) );
-}
-
-// The same neighbour (-1: beyond an open boundary) from the pair's fixed index offset: away from the
-// boundaries the neighbour is i + delta, and along an axis with a translation one comparison of the
-// site's coordinate with a uniform number says whether to wrap.  Three vector instructions per axis
-// the pair leaves, against about thirty for the coordinates' general wrap.
-__device__ __forceinline__ int pair_neighbour_delta( const HamDev & H, int i, int a, int b, int c, const PairDev & p )
-{
-    const int N[3] = { H.Na, H.Nb, H.Nc }, x[3] = { a, b, c }, d[3] = { p.da, p.db, p.dc };
-    int j = i + p.delta, unit = H.nb;
-    bool out = false;
-#pragma unroll
-    for( int u = 0; u < 3; ++u )
-    {
-        const int wrap = unit * N[u];
-        if( abs( d[u] ) > N[u] )
-            return -1;
-        if( d[u] > 0 )
-        {
-            const bool w = x[u] >= N[u] - d[u];
-            j -= w ? wrap : 0;
-            out = out || ( w && !H.bc[u] );
-        }
-        else if( d[u] < 0 )
-        {
-            const bool w = x[u] < -d[u];
-            j += w ? wrap : 0;
-            out = out || ( w && !H.bc[u] );
-        }
-        unit = wrap;
-    }
-    return out ? -1 : j;
-}
-
 // neighbours a spin gathers into registers before using them (larger tables in groups)
 constexpr int LG_MAX_NB = GATHER_PAIRS;
 
 // The exchange neighbours of spin i (a table of few_pairs), all loads issued before any is used.
 // A pair that does not start at this basis atom or leaves an open boundary reads the spin itself
-// and yields exactly zero (its loaded values are replaced).
+// and yields exactly zero (its loaded values are replaced, behind all loads: on an open boundary a
+// replacement between them would wait for each pair's in turn).
 template<bool AOS = false>
 __device__ __forceinline__ void gather_exchange_neighbours( const HamDev & H, const double * __restrict__ x, int nos,
                                                             int i, int ib, int a, int b, int c,
                                                             double ( &se )[LG_MAX_NB][3] )
 {
+    bool is[LG_MAX_NB];
 #pragma unroll
     for( int k = 0; k < LG_MAX_NB; ++k )
         if( k < H.n_exch )
         {
             const PairDev & p = H.exch_g[k];
-            const int j       = p.i != ib ? -1 : pair_neighbour_delta( H, i, a, b, c, p );
-            load_spin<AOS>( x, nos, j >= 0 ? j : i, se[k] );
-            if( j < 0 )
-                se[k][0] = se[k][1] = se[k][2] = 0.0;
+            const int n       = pair_neighbour_delta( H, i, a, b, c, p );
+            is[k]             = p.i == ib && n >= 0;
+            load_spin<AOS>( x, nos, is[k] ? n : i, se[k] );
         }
+#pragma unroll
+    for( int k = 0; k < LG_MAX_NB; ++k )
+        if( k < H.n_exch && !is[k] )
+            se[k][0] = se[k][1] = se[k][2] = 0.0;
 }
 
 // Index offsets of the sites up to MAX_REACH cells away along each axis, one column of LDS per
