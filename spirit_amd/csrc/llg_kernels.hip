@@ -385,6 +385,9 @@ __global__ void __launch_bounds__( LLG_THREADS ) k_llg_stage( StepArgs A )
 // The method constructor's force evaluation and Hook_Post_Iteration (Method_LLG.cpp:22-63,
 // 247-301) on the current spins, without a thermal field: energy, max torque of the
 // virtual force projected on s, and the force F (projected when the field is read).
+// FEW: local_gradient's (a nearest-neighbour model of 10^6 spins takes 26.8 us, 33.3 through the long
+// tables' path, 29.2 when one kernel held both).
+template<bool FEW>
 __global__ void __launch_bounds__( LLG_THREADS ) k_observe( StepArgs A, int solver )
 {
     const int blk           = xcd_contiguous_block();
@@ -398,7 +401,7 @@ __global__ void __launch_bounds__( LLG_THREADS ) k_observe( StepArgs A, int solv
     {
         const double * x = A.s + base;
         double g[3], e;
-        local_gradient( H, x, nos, i, ( A.h && H.has_ddi ) ? A.h + base : nullptr, g, e );
+        local_gradient<FEW>( H, x, nos, i, ( A.h && H.has_ddi ) ? A.h + base : nullptr, g, e );
         e_i = e;
         double si[3];
         load3( x, nos, i, si );
@@ -449,7 +452,8 @@ void llg_launch_project_field( const double * F, const double * s, double * out,
 
 void llg_launch_observe( const StepArgs & A, int solver, int n_blocks, hipStream_t st )
 {
-    hipLaunchKernelGGL( k_observe, dim3( n_blocks ), dim3( LLG_THREADS ), 0, st, A, solver );
+    const auto k = A.few_pairs ? k_observe<true> : k_observe<false>;
+    hipLaunchKernelGGL( k, dim3( n_blocks ), dim3( LLG_THREADS ), 0, st, A, solver );
 }
 
 // Gradient (SoA) and energy partials of a configuration, for getters and parity tests.
