@@ -134,7 +134,7 @@ __device__ __forceinline__ void fold_finalize( const StepArgs & A, const ImageDe
 // the stage kernel
 // ---------------------------------------------------------------------------
 // STT_G: some image takes the spin-transfer torque from the spin's derivative along the
-// current (a separate instantiation: its six neighbour loads cost registers the others need);
+// current (separate instantiations: its six neighbour loads cost registers the others need);
 // FEW: local_gradient's
 template<int SOLVER, int STAGE, bool STT_G, bool FEW>
 __global__ void __launch_bounds__( LLG_THREADS ) k_llg_stage( StepArgs A )
@@ -375,7 +375,7 @@ __global__ void __launch_bounds__( LLG_THREADS ) k_llg_stage( StepArgs A )
     {
         // (in the kernels of long pair tables and of the spin derivative the reduction costs 6 to 38
         // registers, in this one none)
-        if( FEW && A.fold )
+        if( FEW && !STT_G && A.fold )
             fold_finalize( A, *I, img, blk, e_i, t_i );
         else
             block_reduce_store( e_i, t_i, A.part_E, A.part_T, blk );
@@ -606,9 +606,10 @@ __global__ void __launch_bounds__( FIN_THREADS )
 template<int SOLVER, int STAGE>
 static void launch_stage( const StepArgs & A, int n_blocks, hipStream_t st )
 {
-    const auto k = A.stt_gradient ? k_llg_stage<SOLVER, STAGE, true, false>
-                   : A.few_pairs  ? k_llg_stage<SOLVER, STAGE, false, true>
-                                  : k_llg_stage<SOLVER, STAGE, false, false>;
+    const auto k = A.stt_gradient ? ( A.few_pairs ? k_llg_stage<SOLVER, STAGE, true, true>
+                                                  : k_llg_stage<SOLVER, STAGE, true, false> )
+                                  : ( A.few_pairs ? k_llg_stage<SOLVER, STAGE, false, true>
+                                                  : k_llg_stage<SOLVER, STAGE, false, false> );
     hipLaunchKernelGGL( k, dim3( n_blocks ), dim3( LLG_THREADS ), 0, st, A );
 }
 

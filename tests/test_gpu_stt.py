@@ -126,6 +126,23 @@ def test_stt_gradient_skewed_two_basis(make_state, oracle):
     assert err <= 1e-9
 
 
+@pytest.mark.parametrize("solver", list(SOLVERS))
+def test_stt_gradient_long_pair_table(make_state, oracle, solver):
+    """The gradient torque with exchange to the third shell (26 neighbours: the stage kernels' path for
+    long pair tables), 100 steps."""
+    cfg = film([12, 9, 4], [1, 0, 1], n_shells_exchange=3, jij=[5.0, 1.0, -0.5], **STT_GRAD)
+    print_case("stt gradient, three shells", solver)
+    p = make_state(cfg)
+    S = oracle.System(cfg)
+    s0 = oracle.random_spins(S.nos, 43)
+    set_spins(p, s0)
+    s, _, _ = run_n_shot(p, SOLVERS[solver], 100)
+    s_ref, _, _, _ = S.llg(s0, SOLVERS[solver], 100, dt=cfg["llg_dt"], damping=cfg["llg_damping"],
+                           beta=STT_GRAD["llg_beta"], stt=(STT_GRAD["llg_stt_magnitude"],
+                                                           STT_GRAD["llg_stt_polarisation_normal"], True))
+    assert float(np.abs(s - s_ref).max()) <= 1e-9
+
+
 def test_stt_gradient_helix_translation(make_state):
     """With beta = alpha the gradient torque turns every spin of a helix about its axis by
     -dt gamma a_j / mu_B * sin(k a) / a per step (the helix moves rigidly along the current):
