@@ -800,11 +800,17 @@ static int p2_c_tk( const DdiDev & d )
 std::vector<std::pair<int, int>> ddi_pass_c_candidates( const DdiDev & d )
 {
     std::vector<std::pair<int, int>> c;
-    // a lattice of one plane: two round trips of the spectrum less than B, C and B^-1 in turn
-    // (500x500x1, padded 1000x1000: 24 us against 15 + 28 + 17), wherever a tile fits
+    // a lattice of one plane: one kernel along b saves two round trips of the spectrum against B, C and
+    // B^-1 in turn.  With one atom it was the faster at every size measured, one-column tiles among them
+    // (a Heun step of 256x256 spins 61 us against 88, 500x500 121 / 198, 64x1024 79 / 119, 600x735
+    // 256 / 351, 1200x1200 560 / 1132).  With several atoms a block holds so many lines that few blocks
+    // may be left: 250x500 cells of two atoms 208 / 254 and 100x100 of six 155 / 289, but 100x256 of four
+    // 228 / 185 and 100x700 of two 228 / 194, so the plan times both.
     if( d.Pc == 1 && mix_conv_ok( d, true ) )
     {
         c.push_back( { DDI_C_MIX_B, 0 } );
+        if( d.nb > 1 && mix_conv_ok( d, false ) )
+            c.push_back( { DDI_C_MIX, 0 } );
         return c;
     }
     if( p2_c1_ok( d ) )

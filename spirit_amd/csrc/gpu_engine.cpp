@@ -381,7 +381,8 @@ struct PassCChoice
 static std::map<std::vector<int>, PassCChoice> pass_c_chosen;
 
 // Times every pass C kernel that can run the plan on a zero configuration (the run time
-// does not depend on the values) and keeps the fastest.  The environment variable
+// does not depend on the values) and keeps the fastest; for lattices of one plane, where one of them
+// takes the place of passes B and B^-1 too, the whole field.  The environment variable
 // SPIRIT_HIP_DDI_PASS_C = generic | lds | reg | reg4 restricts the choice to that kernel where it
 // can run the plan (for tests of each kernel and for tuning).
 void DdiPlan::choose_pass_c( hipStream_t st )
@@ -442,7 +443,14 @@ void DdiPlan::choose_pass_c( hipStream_t st )
         double t = 1e30;
         for( int rep = 0; rep < 3; ++rep )
         {
-            ddi_launch_field( d, s0.as<double>(), h0.as<double>(), (int)nos, st, e0, e1 );
+            if( d.Pc == 1 )
+            {
+                HIPCHECK( hipEventRecord( e0, st ) );
+                ddi_launch_field( d, s0.as<double>(), h0.as<double>(), (int)nos, st );
+                HIPCHECK( hipEventRecord( e1, st ) );
+            }
+            else
+                ddi_launch_field( d, s0.as<double>(), h0.as<double>(), (int)nos, st, e0, e1 );
             HIPCHECK( hipGetLastError() );
             HIPCHECK( hipEventSynchronize( e1 ) );
             float ms = 0;

@@ -72,3 +72,13 @@ def test_ddi_field_of_any_length(engine, oracle, cells, bc, padding, basis):  # 
     g0, E0 = S.gradient_and_energy(s)
     assert np.abs(g - g0).max() <= 1e-12 * np.abs(g0).max()
     assert abs(E - E0) <= 1e-11 * max(abs(E0), np.abs(g0).max())
+
+
+@pytest.mark.parametrize("passes", ["one kernel", "generic"])
+@pytest.mark.parametrize("cells,basis", [([20, 500, 1], 1), ([22, 26, 1], 2), ([10, 128, 1], 4), ([9, 25, 1], 8)])
+def test_ddi_field_of_one_plane_both_ways(engine, oracle, monkeypatch, cells, basis, passes):  # noqa: F811
+    """One kernel along b, and the passes B, C and B^-1 that it takes the place of (plans of several
+    atoms time the two)."""
+    if passes == "generic":
+        monkeypatch.setenv("SPIRIT_HIP_DDI_PASS_C", "generic")
+    test_ddi_field_of_any_length(engine, oracle, cells, "000", 1, basis)
