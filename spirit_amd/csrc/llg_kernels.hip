@@ -44,10 +44,11 @@ __device__ __forceinline__ void image_result( const ImageDev & I, int img, int n
 // Partials are stored and read at device scope and a block counts itself only when its stores are
 // performed (pass_tail of the chain kernels has why no cache is written back or invalidated for it);
 // counters are rearmed by the blocks that completed them.  A launch of its own for the reduction costs
-// 4.4 us of a 16.1 us step of 64 x 64 spins; here the step takes 14.3 us, of 256 x 256 spins (256 blocks)
-// 16.4 instead of 17.0, of 362 x 362 (512) 18.0 instead of 18.7.  Arrivals at one counter take 8 ns each,
-// one after the other (with a counter for all blocks 256 x 256 spins took 18.3 us), hence groups; and
-// every block waits about a microsecond for its store and arrival, which larger lattices don't win back.
+// 4.4 us of a 16.1 us step of 64 x 64 spins; here the step takes 14.3 us (13.1 since the neighbour
+// lookup has no branches), of 256 x 256 spins (256 blocks) 16.4 instead of 17.0, of 362 x 362 (512) 18.0
+// instead of 18.7.  Arrivals at one counter take 8 ns each, one after the other (with a counter for all
+// blocks 256 x 256 spins took 18.3 us), hence groups; and every block waits about a microsecond for its
+// store and arrival, which larger lattices don't win back.
 __device__ __forceinline__ void fold_finalize( const StepArgs & A, const ImageDev & I, int img, int blk, double e,
                                                double t )
 {

@@ -127,7 +127,7 @@ __global__ void __launch_bounds__( LLG_THREADS ) k_na_copy( const double * src, 
 // Gradient of the spins x (an array of spins, like the gradient) and every block's energy; with out, the
 // last block to arrive adds the energies (fold_finalize of the stage kernels has the protocol; with one
 // counter 128 blocks take 1 us to arrive, 256 as long as a launch costs).  A call was bound by its launches and copies, not by this kernel: five
-// kernels and two copies took 37.6 us for 64 x 64 spins, this one 23.5, of which the kernel is 10.
+// kernels and two copies took 37.6 us for 64 x 64 spins, this one 22.8, of which the kernel is 10.
 template<bool FEW>
 __global__ void __launch_bounds__( LLG_THREADS )
     k_na_gradient( HamDev H, const double * __restrict__ x, double * __restrict__ grad, double * part, int * count,
