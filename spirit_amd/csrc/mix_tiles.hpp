@@ -187,13 +187,16 @@ inline MixArraysTile mix_arrays_tile( const MixLen & L, int arrays, long long n_
     return MixArraysTile{ mix_tile( L, arrays * cw, lsr, false, lds_max, tw_lds ), cw, tw_lds };
 }
 
-// Pass C of n_arrays fields, or the one-plane convolution along b: there a block holds all arrays of its
-// columns and there are only n_cols / cw blocks, so its tiles narrow down to one column.  Where one
+// Pass C of n_arrays fields, or the one-plane convolution along b.  A block holds all arrays of its columns,
+// which is much work for one, so the tiles narrow further than pass B's where blocks are few: pass C's to
+// two columns (a Heun step of 12x12x50 cells of eight atoms takes 247 us instead of 527 with four, of four
+// atoms 123 / 187, of one 65 / 65, 7x9x250 of one 78 / 84; one column is within 5% of two), along b, with
+// only n_cols / cw blocks, to one.  Where one
 // column of pass C leaves no room for the twiddles (1463 to 1706 points of two basis atoms, 410 to 426
 // of eight) they stay in global memory; a lattice of one plane has the passes along b instead.
 inline MixArraysTile mix_conv_tile( const MixLen & L, int n_arrays, long long n_cols, bool along_b, size_t lds_max )
 {
-    const MixArraysTile C = mix_arrays_tile( L, n_arrays, n_cols, along_b ? 1 : 4, lds_max, true );
+    const MixArraysTile C = mix_arrays_tile( L, n_arrays, n_cols, along_b ? 1 : 2, lds_max, true );
     return C.t.nl > 0 || along_b ? C : mix_arrays_tile( L, n_arrays, n_cols, 1, lds_max, false );
 }
 
