@@ -38,7 +38,7 @@ struct DdiDev
     int sig_b[6], sig_c[6];
     int lds_max; // dynamic LDS bytes a block may use on this device (host-side launch choice)
     int c_kind;  // pass C kernel (DdiPassC), chosen by timing when the plan is built
-    int c_tk;    // column tile of DDI_C_P2_LDS
+    int c_tk;    // column tile of DDI_C_P2_LDS; widest of DDI_C_MIX, 0 as the sizes say
     int rev;     // DDI_REV_* bits: passes that visit their blocks in reverse order
     const DdiMixHost * mix; // host memory (read by the launchers only)
 };
@@ -87,11 +87,13 @@ std::vector<std::pair<int, int>> ddi_pass_c_candidates( const DdiDev & d );
 // and B^-1 for lattices of one plane.
 bool mix_a_ok( const DdiDev & d );
 bool mix_b_ok( const DdiDev & d );
+constexpr int MIX_WIDEST = 16; // columns of a tile
 bool mix_conv_ok( const DdiDev & d, bool along_b );
+int mix_conv_width( const DdiDev & d ); // columns of pass C's tile
 void mix_launch_a_fwd( const DdiDev & d, const double * s, int nos, hipStream_t st );
 void mix_launch_a_inv( const DdiDev & d, double * h, int nos, hipStream_t st );
 void mix_launch_b( const DdiDev & d, bool inverse, hipStream_t st );
-void mix_launch_conv( const DdiDev & d, bool along_b, hipStream_t st );
+void mix_launch_conv( const DdiDev & d, bool along_b, int want, hipStream_t st ); // tiles at most want wide
 
 // The kernel spectrum of the real-space tensor D[6 * n_inter][Pc][Pb][Pa], transformed along a, b (in
 // `work`, rows of stride Hs) and c on the same tiles: any number of values, whatever a block's threads hold.

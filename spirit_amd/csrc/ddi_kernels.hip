@@ -824,8 +824,16 @@ std::vector<std::pair<int, int>> ddi_pass_c_candidates( const DdiDev & d )
         if( tk / 2 > 0 )
             c.push_back( { DDI_C_P2_LDS, tk / 2 } );
     }
+    // the mixed-radix tile's width: with one atom as the sizes say; with several a column is up to a block's
+    // LDS and neither rule held: 6x150x150 cells of three atoms 1154 / 1014 us a Heun step at 2 / 1 columns,
+    // 2x100x100 of six 997 / 638, 30x30x30 of eight 675 / 778 / 677 at 4 / 2 / 1 (the same bits)
     if( c.empty() )
+    {
         c.push_back( { DDI_C_MIX, 0 } );
+        if( d.nb > 1 && mix_conv_ok( d, false ) )
+            for( int w = mix_conv_width( d ) / 2; w >= 1; w /= 2 )
+                c.push_back( { DDI_C_MIX, w } );
+    }
     return c;
 }
 
@@ -962,7 +970,7 @@ void ddi_launch_field( const DdiDev & d, const double * spins, double * h, int n
 #undef CALL_C
     }
     else
-        mix_launch_conv( d, one_plane, st );
+        mix_launch_conv( d, one_plane, d.c_kind == DDI_C_MIX && d.c_tk > 0 ? d.c_tk : MIX_WIDEST, st );
     if( evc1 )
         (void)hipEventRecord( evc1, st );
     // pass B^-1

@@ -261,7 +261,7 @@ static MixTile mix_a_tile( const DdiDev & d )
 
 static MixTile mix_b_tile( const DdiDev & d )
 {
-    return mix_column_tile( d.mix->len[1], (long long)d.Ha * d.Nc * 3 * d.nb, d.lds_max );
+    return mix_column_tile( d.mix->len[1], 3LL * d.nb * d.Nc, d.Ha, d.lds_max );
 }
 
 bool mix_a_ok( const DdiDev & d )
@@ -274,15 +274,20 @@ bool mix_b_ok( const DdiDev & d )
     return mix_b_tile( d ).nl > 0;
 }
 
-static MixArraysTile mix_c_tile( const DdiDev & d, bool along_b )
+static MixArraysTile mix_c_tile( const DdiDev & d, bool along_b, int want )
 {
-    return along_b ? mix_conv_tile( d.mix->len[1], 3 * d.nb, d.Ha, true, d.lds_max )
-                   : mix_conv_tile( d.mix->len[2], 3 * d.nb, (long long)d.Ha * d.Pb, false, d.lds_max );
+    return along_b ? mix_conv_tile( d.mix->len[1], 3 * d.nb, 1, d.Ha, true, want, d.lds_max )
+                   : mix_conv_tile( d.mix->len[2], 3 * d.nb, d.Pb, d.Ha, false, want, d.lds_max );
 }
 
 bool mix_conv_ok( const DdiDev & d, bool along_b )
 {
-    return mix_c_tile( d, along_b ).t.nl > 0;
+    return mix_c_tile( d, along_b, MIX_WIDEST ).t.nl > 0;
+}
+
+int mix_conv_width( const DdiDev & d )
+{
+    return mix_c_tile( d, false, MIX_WIDEST ).cw;
 }
 
 void mix_launch_a_fwd( const DdiDev & d, const double * s, int nos, hipStream_t st )
@@ -315,11 +320,11 @@ void mix_launch_b( const DdiDev & d, bool inverse, hipStream_t st )
                         inverse ? d.Pb : d.Nb, inverse ? d.Nb : d.Pb );
 }
 
-void mix_launch_conv( const DdiDev & d, bool along_b, hipStream_t st )
+void mix_launch_conv( const DdiDev & d, bool along_b, int want, hipStream_t st )
 {
     const int axis        = along_b ? 1 : 2;
     const MixPlan & P     = d.mix->plan[axis];
-    const MixArraysTile C = mix_c_tile( d, along_b );
+    const MixArraysTile C = mix_c_tile( d, along_b, want );
     const int tiles       = ( d.Ha + C.cw - 1 ) / C.cw;
     const MixDiv by_cw{ 1.0f / (float)C.cw }, by_n{ 1.0f / (float)P.n };
     const bool w = mix_wide( d, axis ), one = d.nb == 1;
@@ -337,14 +342,14 @@ void mix_launch_conv( const DdiDev & d, bool along_b, hipStream_t st )
 
 static MixArraysTile mix_c_spectrum_tile( const DdiDev & d )
 {
-    return mix_spectrum_tile( d.mix->len[2], (long long)d.Ha * d.Pb * d.n_inter, d.lds_max );
+    return mix_spectrum_tile( d.mix->len[2], (long long)d.Pb * d.n_inter, d.Ha, d.lds_max );
 }
 
 bool mix_spectrum_ok( const DdiDev & d )
 {
-    const long long n_rows = 6LL * d.n_inter * d.Pb * d.Pc, n_cols = 6LL * d.n_inter * d.Ha * d.Pc;
-    return mix_row_tile( d.mix->len[0], n_rows, d.lds_max ).nl > 0
-           && mix_column_tile( d.mix->len[1], n_cols, d.lds_max ).nl > 0 && mix_c_spectrum_tile( d ).t.nl > 0;
+    const long long n_slabs = 6LL * d.n_inter * d.Pc;
+    return mix_row_tile( d.mix->len[0], n_slabs * d.Pb, d.lds_max ).nl > 0
+           && mix_column_tile( d.mix->len[1], n_slabs, d.Ha, d.lds_max ).nl > 0 && mix_c_spectrum_tile( d ).t.nl > 0;
 }
 
 void mix_launch_spectrum( const DdiDev & d, const double * D, double2 * work, double2 * Dfull, hipStream_t st )
@@ -359,7 +364,7 @@ void mix_launch_spectrum( const DdiDev & d, const double * D, double2 * work, do
                             mix_lds( L[0], T.lsr ), st, d.mix->plan[0], T, D, work, n_rows, d.Ha, d.Hs );
     }
     {
-        const MixTile T = mix_column_tile( L[1], n_slabs * d.Ha, d.lds_max );
+        const MixTile T = mix_column_tile( L[1], n_slabs, d.Ha, d.lds_max );
         const int tiles = ( d.Ha + T.nl - 1 ) / T.nl;
         const auto k    = mix_wide( d, 1 ) ? k_mix_b<false, true> : k_mix_b<false, false>;
         hipLaunchKernelGGL( k, dim3( (unsigned)( n_slabs * tiles ) ), dim3( T.nc * T.m ), mix_lds( L[1], T.lsr ), st, d,

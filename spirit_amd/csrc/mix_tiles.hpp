@@ -151,19 +151,29 @@ inline MixTile mix_line_tile( const MixLen & L, long long n_lines, int want, int
     return mix_tile( L, cw, cw, true, lds_max );
 }
 
-// Pass A: row pairs are contiguous whatever their number is: 4, fewer where that fills the chip.
+// Pass A: row pairs are contiguous whatever their number is: 4, fewer where that fills the chip, and 16
+// of rows so short that 4 of them leave most of a wavefront idle (a Heun step of 1x512x512 spins takes
+// 418 us instead of 517, of 5x100x60 90 / 103, of 13x100x60 140 / 150; from 28 points on within 2%).
 inline MixTile mix_row_tile( const MixLen & L, long long n_lines, size_t lds_max )
 {
-    return mix_line_tile( L, n_lines, 4, 1, lds_max );
+    return mix_line_tile( L, n_lines, L.n <= 26 ? 16 : 4, 1, lds_max );
+}
+
+// Column tiles no wider than a row of the spectrum needs.
+inline int mix_width( int want, int row )
+{
+    while( want / 2 >= row )
+        want /= 2;
+    return want;
 }
 
 // Pass B: a row piece of a column tile is 16 cw bytes, so tiles are 16 wide where two blocks then fit a
 // CU's LDS, else 8, and narrower only where LDS forces it or fewer than 192 blocks would leave CUs
 // idle (not below 4, 64 bytes): 14 us a pass against 18 and 22 at 16, 8, 4 columns of 300 points, 13
 // against 16 and 22 at 8, 4, 2 of 1000.
-inline MixTile mix_column_tile( const MixLen & L, long long n_lines, size_t lds_max )
+inline MixTile mix_column_tile( const MixLen & L, long long n_rows, int row, size_t lds_max )
 {
-    return mix_line_tile( L, n_lines, 16, 4, lds_max );
+    return mix_line_tile( L, n_rows * row, mix_width( 16, row ), 4, lds_max );
 }
 
 // The tile of a pass that holds `arrays` lines of each of its cw columns (line = array * cw + column, taken
@@ -174,10 +184,10 @@ struct MixArraysTile
     int cw;
     bool tw_lds;
 };
-inline MixArraysTile mix_arrays_tile( const MixLen & L, int arrays, long long n_cols, int least, size_t lds_max,
-                                      bool tw_lds )
+inline MixArraysTile mix_arrays_tile( const MixLen & L, int arrays, long long n_cols, int want, int least,
+                                      size_t lds_max, bool tw_lds )
 {
-    const int cw = mix_lines( L, arrays, n_cols, 16, least, lds_max, tw_lds );
+    const int cw = mix_lines( L, arrays, n_cols, want, least, lds_max, tw_lds );
     // an odd row stride spreads column accesses over the banks
     int lsr = ( arrays * cw ) | 1;
     if( mix_lds( L, lsr, tw_lds ) > lds_max )
@@ -187,23 +197,25 @@ inline MixArraysTile mix_arrays_tile( const MixLen & L, int arrays, long long n_
     return MixArraysTile{ mix_tile( L, arrays * cw, lsr, false, lds_max, tw_lds ), cw, tw_lds };
 }
 
-// Pass C of n_arrays fields, or the one-plane convolution along b.  A block holds all arrays of its columns,
-// which is much work for one, so the tiles narrow further than pass B's where blocks are few: pass C's to
-// two columns (a Heun step of 12x12x50 cells of eight atoms takes 247 us instead of 527 with four, of four
-// atoms 123 / 187, of one 65 / 65, 7x9x250 of one 78 / 84; one column is within 5% of two), along b, with
-// only n_cols / cw blocks, to one.  Where one
-// column of pass C leaves no room for the twiddles (1463 to 1706 points of two basis atoms, 410 to 426
-// of eight) they stay in global memory; a lattice of one plane has the passes along b instead.
-inline MixArraysTile mix_conv_tile( const MixLen & L, int n_arrays, long long n_cols, bool along_b, size_t lds_max )
+// Pass C of n_arrays fields on n_rows rows of `row` columns, or the one-plane convolution along b (one
+// row); want: the widest tile.  A block holds all arrays of its columns, which is much work for one, so
+// the tiles narrow further than pass B's where blocks are few: pass C's to two columns (a Heun step of
+// 12x12x50 cells of eight atoms takes 247 us instead of 527 with four, of four atoms 123 / 187, of one
+// 65 / 65, 7x9x250 of one 78 / 84; one column is within 5% of two), the one along b to one.
+// Where one column of pass C leaves no room for the twiddles (1463 to 1706 points of two basis atoms, 410
+// to 426 of eight) they stay in global memory; a lattice of one plane has the passes along b instead.
+inline MixArraysTile mix_conv_tile( const MixLen & L, int n_arrays, long long n_rows, int row, bool along_b, int want,
+                                    size_t lds_max )
 {
-    const MixArraysTile C = mix_arrays_tile( L, n_arrays, n_cols, along_b ? 1 : 2, lds_max, true );
-    return C.t.nl > 0 || along_b ? C : mix_arrays_tile( L, n_arrays, n_cols, 1, lds_max, false );
+    const int w           = mix_width( want, row );
+    const MixArraysTile C = mix_arrays_tile( L, n_arrays, n_rows * row, w, along_b ? 1 : 2, lds_max, true );
+    return C.t.nl > 0 || along_b ? C : mix_arrays_tile( L, n_arrays, n_rows * row, 1, 1, lds_max, false );
 }
 
 // The kernel spectrum's pass C: the six components of a pair of sublattices.
-inline MixArraysTile mix_spectrum_tile( const MixLen & L, long long n_cols, size_t lds_max )
+inline MixArraysTile mix_spectrum_tile( const MixLen & L, long long n_rows, int row, size_t lds_max )
 {
-    return mix_arrays_tile( L, 6, n_cols, 1, lds_max, false );
+    return mix_arrays_tile( L, 6, n_rows * row, mix_width( 16, row ), 1, lds_max, false );
 }
 
 } // namespace spirit_hip

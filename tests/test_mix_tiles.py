@@ -69,7 +69,8 @@ int main()
         int last_a = -1, last_b = -1;
         for( long long c : counts )
         {
-            const int ca = mix_lines( L, 1, c, 4, 1, LDS ), cb = mix_lines( L, 1, c, 16, 4, LDS );
+            const int ca = mix_lines( L, 1, c, 16, 1, LDS ) + 100 * mix_lines( L, 1, c, 4, 1, LDS );
+            const int cb = mix_lines( L, 1, c, 16, 4, LDS );
             if( ca != last_a )
             {
                 // passes A and A^-1: a thread keeps the line (row pair) threadIdx mod nc
@@ -82,10 +83,13 @@ int main()
             if( cb != last_b )
             {
                 // passes B and B^-1: the same for the columns
-                const MixTile T = mix_column_tile( L, c, LDS );
-                common( "columns", L, c, T );
-                if( T.nc != T.nl || mix_lds( L, T.lsr ) > LDS )
-                    fail( "columns: lines without a thread", L, c, T );
+                for( int row : { 1, 2, 3, 5, 9, 201 } )
+                {
+                    const MixTile T = mix_column_tile( L, ( c + row - 1 ) / row, row, LDS );
+                    common( "columns", L, c, T );
+                    if( T.nc != T.nl || mix_lds( L, T.lsr ) > LDS || T.nl >= 2 * row )
+                        fail( "columns: lines without a thread", L, c, T );
+                }
                 last_b = cb;
             }
             if( c > 3000 || c % 7 != 1 )
@@ -93,9 +97,11 @@ int main()
             // passes that hold several arrays of a column: the convolution and the kernel spectrum
             for( int nb = 1; nb <= 8; ++nb )
                 for( int along_b = 0; along_b < 2; ++along_b )
-                    arrays( along_b ? "convolution along b" : "convolution along c", L, c,
-                            mix_conv_tile( L, 3 * nb, c, along_b, LDS ), 3 * nb );
-            arrays( "kernel spectrum", L, c, mix_spectrum_tile( L, c, LDS ), 6 );
+                    for( int want = 16; want >= 1; want /= 2 )
+                        arrays( along_b ? "convolution along b" : "convolution along c", L, c,
+                                mix_conv_tile( L, 3 * nb, along_b ? 1 : ( c + 200 ) / 201, along_b ? (int)c : 201,
+                                               along_b, want, LDS ), 3 * nb );
+            arrays( "kernel spectrum", L, c, mix_spectrum_tile( L, ( c + 2 ) / 3, 3, LDS ), 6 );
         }
     }
     std::printf( "%d tiles, %d bad\n", tiles, bad );
@@ -124,8 +130,8 @@ int main()
 {
     int n, nb;
     while( std::scanf( "%d %d", &nb, &n ) == 2 )
-        std::printf( "%d %d %d %d\n", nb, n, mix_conv_tile( mix_length( n ), 3 * nb, 1000, false, 160 * 1024 ).t.nl > 0,
-                     mix_spectrum_tile( mix_length( n ), 1000, 160 * 1024 ).t.nl > 0 );
+        std::printf( "%d %d %d %d\n", nb, n, mix_conv_tile( mix_length( n ), 3 * nb, 5, 201, false, 16, 160 * 1024 ).t.nl > 0,
+                     mix_spectrum_tile( mix_length( n ), 5, 201, 160 * 1024 ).t.nl > 0 );
 }
 """
 
